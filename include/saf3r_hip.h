@@ -405,18 +405,17 @@ int64_t saf3r_gather_attn_workspace_bytes(int n, int topk);
  *   idx: int32 [n_q][frames*min(topk, per_frame)] global key rows, frame-major, score descending,
  *   ties to the lower index. topk >= 1 and min(topk, per_frame) <= 128 (the reference's limit);
  *   above 16 per_frame <= 4096.
- *   workspace / workspace_bytes: caller-owned device memory for the scores of a chunk of queries,
- *   used when min(topk, per_frame) > 16 (NULL / 0 otherwise). saf3r_token_topk_workspace_bytes
- *   gives the size that runs every query in one chunk (at most about 1 GiB); any size of at least
- *   the scores of 128 queries (frames * roundup(per_frame, 64) * 4 * 128 bytes) works, in more
- *   chunks. Calls that share a workspace must be ordered (one stream).
+ *   workspace / workspace_bytes: caller-owned device memory, required when
+ *   min(topk, per_frame) > 16 (NULL / 0 otherwise): at least a share for 128 queries
+ *   (frames * roundup(per_frame, 64) * 4 * 128 bytes). The selection keeps its scores in LDS and does
+ *   not read or write it; the requirement stays for callers of this ABI version.
  * Replaces: saf3r/triton/fused_qk_topk.py:120-217 (compute_qk_topk_indices_fused).
  */
 int saf3r_token_topk(const saf3r_rows* q, const saf3r_rows* k, int n_q, int frames, int per_frame, int topk,
                      int32_t* idx, void* workspace, int64_t workspace_bytes, void* stream);
 
-/* Workspace bytes saf3r_token_topk takes for these sizes in one chunk: 0 when
- * min(topk, per_frame) <= 16, -1 for sizes saf3r_token_topk rejects. No counterpart in the
+/* Workspace bytes for every query of a call (at most about 1 GiB; see above for the least that
+ * saf3r_token_topk accepts): 0 when min(topk, per_frame) <= 16, -1 for sizes saf3r_token_topk rejects. No counterpart in the
  * reference (its Triton kernel keeps each query's list in registers). */
 int64_t saf3r_token_topk_workspace_bytes(int n_q, int frames, int per_frame, int topk);
 

@@ -25,11 +25,6 @@ struct TopkParams {
   int kmode;  // key row of (frame f, token j): 1 = frame f row j (rows_per_frame == P), 0 = flat row f*P + j, 2 = general
   int64_t k_fst;  // kmode 0 and 1: rows from frame f to frame f + 1 (P or frame_row_stride)
   int32_t* idx;
-  // score dump (k > 16): queries q_begin .. nq - 1, score of (query qi, frame f, key j) at
-  // ws[(qi - q_begin) * F * ppad + f * ppad + j], ppad = frame length rounded up to 64
-  float* ws;
-  int64_t q_begin;
-  int ppad;
   int fgroups;  // frame groups of the selection launch (grid.y)
 };
 
@@ -87,7 +82,7 @@ __device__ inline void fmax_insert(float (&t)[K], float x) {
 // Step t reads its K fragments, selects over the scores of step t - 1 while those reads are in
 // flight, then issues its MFMAs into the same registers; the two waves of a SIMD alternate their
 // VALU and MFMA phases.
-template <int K, bool FLAT, bool DUMP>
+template <int K, bool FLAT>
 __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkParams p) {
   // groups per lane (2G >= K maxima per query): more groups give a tighter tau for larger K, so that
   // the candidates of a lane fit its buffer
@@ -97,7 +92,7 @@ __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkPar
   __shared__ uint64_t cbuf[(kCand + 1) * 256];
   const int tid = tid_x(), lane = tid & 63, half = lane >> 5, col = lane & 31;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t q0 = p.q_begin + (int64_t)bid_x() * 128;
+  const int64_t q0 = (int64_t)bid_x() * 128;
   const int64_t qi = q0 + 32 * w + col;
   const bool qvalid = qi < p.nq;
 
@@ -111,11 +106,10 @@ __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkPar
 
   const int tiles_pf = (p.P + 63) / 64;
   // frame f: pass 1 over its tiles, then pass 2, for the frames [f_lo, f_hi) of this work-group's
-  // frame group (bid_y of p.fgroups: the split only evens out the tail of the launch); DUMP: one
-  // pass over frame bid_y that stores the scores (a work-group per 128 queries and frame)
-  const int f_lo = __builtin_amdgcn_readfirstlane(DUMP ? bid_y() : p.F * bid_y() / p.fgroups);
-  const int f_hi = __builtin_amdgcn_readfirstlane(DUMP ? f_lo + 1 : p.F * (bid_y() + 1) / p.fgroups);
-  const int total = (f_hi - f_lo) * (DUMP ? 1 : 2) * tiles_pf;
+  // frame group (bid_y of p.fgroups: the split only evens out the tail of the launch)
+  const int f_lo = __builtin_amdgcn_readfirstlane(p.F * bid_y() / p.fgroups);
+  const int f_hi = __builtin_amdgcn_readfirstlane(p.F * (bid_y() + 1) / p.fgroups);
+  const int total = (f_hi - f_lo) * 2 * tiles_pf;
   // LDS chunk position P = 256 j + 64 w + lane of a tile (instruction j of wave w) holds key row
   // P / 8, global 16-byte chunk (P % 8) ^ swz8(row): the swizzle that makes the MFMA fragment
   // reads conflict-free is applied on the load side
@@ -167,10 +161,9 @@ __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkPar
       itb += tbytes;
       if (++iu == tiles_pf) {
         iu = 0;
-        const int adv = DUMP ? 1 : ips;
-        ifr += adv;
+        ifr += ips;
         itb -= tiles_pf * tbytes;
-        if (adv) itb += fbytes;
+        if (ips) itb += fbytes;
         ips ^= 1;
       }
     }
@@ -233,21 +226,7 @@ __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkPar
     const int pbase = 64 * u + 4 * half;
     const int lim = p.P - pbase;  // candidate e is a key of the frame when kpos(e) < lim
     auto sc = [&](int e) { return e < 16 ? s0[e] : s1[e - 16]; };
-    if constexpr (DUMP) {
-      // keys pbase + kpos(4 i) .. + 3 are consecutive: one 16-byte store each (the rows past the
-      // frame's end land in the row's padding)
-      if (qvalid) {
-        float* o = p.ws + (qi - p.q_begin) * ((int64_t)p.F * p.ppad) + (int64_t)f * p.ppad + pbase;
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          *reinterpret_cast<f32x4*>(o + kpos(4 * i)) = f32x4{sc(4 * i), sc(4 * i + 1), sc(4 * i + 2), sc(4 * i + 3)};
-      }
-      if (++u == tiles_pf) {
-        u = 0;
-        ++f;
-      }
-      return;
-    } else if (ps == 0) {
+    if (ps == 0) {
 #pragma unroll
       for (int e = 0; e < 32; ++e)
         gmax[e % G] = fmaxf(gmax[e % G], (!PADDED || kpos(e) < lim) ? sc(e) : -__builtin_inff());
@@ -360,139 +339,364 @@ __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkPar
   wait_vm<0>();  // the trailing loads into unread stages land before the work-group's LDS is released
 }
 
-template <int K>
-static int launch_topk(TopkParams p, hipStream_t st) {
-  // Frame groups: every work-group walks all frames of its queries in 2 passes, so with few, long
-  // work-groups the launch ends with a partly idle last round. The frames split into g groups (one
-  // work-group per 128 queries and group): the largest g of at most 16, with at least 8 frames a
-  // group, whose rounds of resident work-groups (K <= 8: 3 per CU, else 2) are within 2% of the
-  // fullest (at 128 frames x 1369 tokens: g = 16, 10.5 ms against 10.9 with g = 5 and 13.2 with
-  // one group).
-  const int64_t nb = (p.nq + 127) / 128;
+// Frame groups: every work-group walks all frames of its queries, so with few, long work-groups the
+// launch ends with a partly idle last round. The frames split into g groups (one work-group per
+// query block and group): the largest g of at most 16, with at least `least` frames a group, whose
+// rounds of resident work-groups (`per_cu` per CU) are within 2% of the fullest (at 128 frames x
+// 1369 tokens, top-4: g = 16, 10.5 ms against 10.9 with g = 5 and 13.2 with one group).
+static int frame_groups(int64_t nb, int frames, int per_cu, int least) {
   int cus = 0, dev = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
     cus = 256;
-  const int64_t slots = (int64_t)cus * (K <= 8 ? 3 : 2);
-  const int gmax = std::max(1, std::min(16, p.F / 8));
+  const int64_t slots = (int64_t)cus * per_cu;
+  const int gmax = std::max(1, std::min(16, frames / least));
   auto eff = [&](int g) {
     const int64_t wgs = nb * g, rounds = (wgs + slots - 1) / slots;
     return (double)wgs / (double)(rounds * slots);
   };
   double best_eff = 0.0;
   for (int g = 1; g <= gmax; ++g) best_eff = std::max(best_eff, eff(g));
-  int best = 1;
   for (int g = gmax; g >= 1; --g)
-    if (eff(g) >= best_eff - 0.02) {
-      best = g;
-      break;
-    }
-  p.fgroups = best;
-  const dim3 grid((unsigned)nb, (unsigned)best);
-  if (p.kmode == 2) hipLaunchKernelGGL((token_topk_kernel<K, false, false>), grid, dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((token_topk_kernel<K, true, false>), grid, dim3(256), 0, st, p);
+    if (eff(g) >= best_eff - 0.02) return g;
+  return 1;
+}
+
+template <int K>
+static int launch_topk(TopkParams p, hipStream_t st) {
+  const int64_t nb = (p.nq + 127) / 128;
+  p.fgroups = frame_groups(nb, p.F, K <= 8 ? 3 : 2, 8);
+  const dim3 grid((unsigned)nb, (unsigned)p.fgroups);
+  if (p.kmode == 2) hipLaunchKernelGGL((token_topk_kernel<K, false>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((token_topk_kernel<K, true>), grid, dim3(256), 0, st, p);
   return check_launch("saf3r_token_topk");
 }
 
-// ---- per-frame top-k for 16 < k <= 128 (the reference's range): scores, then a selection ----
-constexpr int kLargeMaxP = 4096;  // frame length of that path (values of a segment held by one wave)
+// ---- per-frame top-k for 16 < k <= 128 (the reference's range): score rows in LDS ----
+constexpr int kLargeMaxP = 4096;  // frame length of that path (values of a row held by one wave)
+constexpr int kRowWaves = 16;
 
-// One wave per (query row, frame) segment of P <= 64 NV stored scores. The ke-th largest composite
-// key (sortable float key << 32 | reversed index, the order of the reference's fused top-k) is
-// found by a radix select over the float keys, eight 4-bit digits from the top: every lane counts
-// its own keys into its own 16 LDS bins (bin b of lane l at word 64 b + l: no two lanes share a
-// bank or a word, so the adds never contend), then the wave sums each bin and picks the digit.
-// Keys above the threshold value all count, keys equal to it count from the lowest index on. Each
-// selected key's position is the number of selected keys above it.
-template <int NV>
-__global__ __launch_bounds__(256) void topk_large_kernel(const float* __restrict__ ws, int64_t q_begin, int64_t q_end,
-                                                          int F, int P, int ppad, int ke, int32_t* __restrict__ idx) {
-  __shared__ uint32_t hist[4][16 * 64];
-  __shared__ uint64_t sel[4][128];
-  const int lane = tid_x() & 63, w = tid_x() >> 6;
-  const int64_t seg = (int64_t)bid_x() * 4 + w;
-  if (seg >= (q_end - q_begin) * F) return;  // a whole wave leaves; no work-group barrier follows
-  const int64_t r = seg / F;
-  const int f = (int)(seg - r * F);
-  const float* src = ws + r * ((int64_t)F * ppad) + (int64_t)f * ppad;
-  uint32_t key[NV];
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int j = lane + 64 * i;
-    key[i] = j < P ? fkey(src[j]) : 0;
+// x of lane (lane ^ D)
+template <int CTL>
+__device__ __forceinline__ uint32_t dpp32(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTL, 0xF, 0xF, true);
+}
+template <int D>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t x, int lane) {
+  if constexpr (D == 1) return dpp32<0xB1>(x);
+  else if constexpr (D == 2) return dpp32<0x4E>(x);
+  else if constexpr (D == 4) return dpp32<0x1B>(dpp32<0x141>(x));  // the mirror of 8 lanes (^ 7), then of 4 (^ 3)
+  else if constexpr (D == 8) return dpp32<0x128>(x);
+  else if constexpr (D == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return (lane & 16) ? (uint32_t)r[0] : (uint32_t)r[1];
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return (lane & 32) ? (uint32_t)r[0] : (uint32_t)r[1];
   }
-  uint32_t* hw = hist[w];
-  uint32_t prefix = 0, mask = 0;
-  int need = ke;  // keys still to take at or below the current prefix
-  const int b = lane & 15, g = lane >> 4;  // the bin this lane sums, and its quarter of the lanes
-#pragma unroll 1
-  for (int sh = 28; sh >= 0; sh -= 4) {
-#pragma unroll
-    for (int t = 0; t < 16; ++t) hw[64 * t + lane] = 0;
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-      if (lane + 64 * i < P && (key[i] & mask) == prefix) atomicAdd(&hw[64 * ((key[i] >> sh) & 15) + lane], 1u);
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this lane's counts are in
-    __builtin_amdgcn_wave_barrier();
-    // total of bin b: lanes 16 g .. 16 g + 15 here, the other quarters through two exchanges
-    const u32x4* hb = reinterpret_cast<const u32x4*>(hw + 64 * b + 16 * g);
-    uint32_t tot = 0;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const u32x4 x = hb[t];
-      tot += x[0] + x[1] + x[2] + x[3];
-    }
-    tot += __shfl_xor(tot, 16);
-    tot += __shfl_xor(tot, 32);
-    // keys in bins above b (lanes b + 1 .. 15 of the first quarter hold them)
-    uint32_t incl = tot;
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) {
-      const uint32_t y = __shfl_down(incl, o, 16);
-      if (b + o < 16) incl += y;
-    }
-    const uint32_t above = incl - tot;
-    const bool hit = lane < 16 && above < (uint32_t)need && (uint32_t)need <= incl;
-    const uint64_t m = __ballot(hit);
-    const int src_lane = (int)__builtin_ctzll(m);
-    const int digit = __shfl(b, src_lane);
-    need -= (int)__shfl(above, src_lane);
-    prefix |= (uint32_t)digit << sh;
-    mask |= 0xFu << sh;
-    __builtin_amdgcn_wave_barrier();
-  }
-  // selected: keys above the threshold value, and the first `need` keys equal to it, by index
-  int cnt = 0, eqseen = 0;
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int j = lane + 64 * i;
-    const bool valid = j < P;
-    const bool gt = valid && key[i] > prefix, eq = valid && key[i] == prefix;
-    const uint64_t meq = __ballot(eq);
-    const int req = eqseen + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(meq >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)meq, 0));
-    const bool take = gt || (eq && req < need);
-    const uint64_t mt = __ballot(take);
-    const int pos = cnt + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mt >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mt, 0));
-    if (take) sel[w][pos] = ((uint64_t)key[i] << 32) | (uint64_t)(0xFFFFFFFEu - (uint32_t)j);
-    cnt += __popcll(mt);
-    eqseen += __popcll(meq);
-  }
-  __builtin_amdgcn_s_waitcnt(0xc07f);
-  __builtin_amdgcn_wave_barrier();
-  int32_t* o = idx + (q_begin + r) * ((int64_t)F * ke) + (int64_t)f * ke;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int e = lane + 64 * h;
-    if (e < ke) {
-      const uint64_t x = sel[w][e];
-      int rank = 0;
-      for (int t = 0; t < ke; ++t) rank += sel[w][t] > x;
-      o[rank] = f * P + (int)ckey_index(x);
-    }
+}
+template <int D>
+__device__ __forceinline__ uint64_t lane_xor(uint64_t x, int lane) {
+  return ((uint64_t)lane_xor<D>((uint32_t)(x >> 32), lane) << 32) | lane_xor<D>((uint32_t)x, lane);
+}
+
+template <typename Op>
+__device__ __forceinline__ float wave_reduce32(float x, Op op) {
+  auto at = [](uint32_t y) { return __builtin_bit_cast(float, y); };
+  auto bits = [](float y) { return __builtin_bit_cast(uint32_t, y); };
+  x = op(x, at(dpp32<0xB1>(bits(x))));
+  x = op(x, at(dpp32<0x4E>(bits(x))));
+  x = op(x, at(dpp32<0x141>(bits(x))));
+  x = op(x, at(dpp32<0x128>(bits(x))));
+  const auto a = __builtin_amdgcn_permlane16_swap(bits(x), bits(x), false, false);
+  x = op(at((uint32_t)a[0]), at((uint32_t)a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(bits(x), bits(x), false, false);
+  x = op(at((uint32_t)b[0]), at((uint32_t)b[1]));
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane((int)bits(x)));
+}
+
+// One compare-exchange of a bitonic network over the wave: runs of M lanes, distance D
+// (the lanes that keep the larger value as a literal mask: compares per lane would be hoisted out of
+// the caller's loops, 42 scalar registers)
+constexpr uint64_t keep_max(int M, int D, bool desc) {
+  uint64_t m = 0;
+  for (int l = 0; l < 64; ++l)
+    if ((((l & M) == 0) == ((l & D) == 0)) == desc) m |= 1ull << l;
+  return m;
+}
+template <int M, int D, bool DESC, typename T>
+__device__ __forceinline__ void lane_cas(T& x, int lane) {
+  constexpr uint64_t keep = keep_max(M, D, DESC);
+  const T y = lane_xor<D>(x, lane);
+  x = __builtin_amdgcn_inverse_ballot_w64(~(__builtin_amdgcn_ballot_w64(x > y) ^ keep)) ? x : y;
+}
+// runs of M lanes, each bitonic, to sorted runs (M = 64: the whole wave, descending for DESC)
+template <int M, int D, bool DESC, typename T>
+__device__ __forceinline__ void lane_merge(T& x, int lane) {
+  lane_cas<M, D, DESC>(x, lane);
+  if constexpr (D > 1) lane_merge<M, D / 2, DESC>(x, lane);
+}
+template <bool DESC, int M = 2, typename T>
+__device__ __forceinline__ void lane_sort(T& x, int lane) {
+  lane_merge<M, M / 2, DESC>(x, lane);
+  if constexpr (M < 64) lane_sort<DESC, 2 * M>(x, lane);
+}
+// x, y (empty entries 0) of a wave's n entries, the 64 best descending in x; the rest in y for `both`
+template <typename T>
+__device__ __forceinline__ void lane_sort128(T& x, T& y, int n, bool both, int lane) {
+  lane_sort<true>(x, lane);
+  if (n > 64) {  // wave-uniform
+    lane_sort<false>(y, lane);
+    const T big = x > y ? x : y;
+    y = x > y ? y : x;
+    x = big;
+    lane_merge<64, 32, true>(x, lane);
+    if (both) lane_merge<64, 32, true>(y, lane);
   }
 }
 
-// Bytes of one query's stored scores (frames x frame length rounded up to 64, fp32).
+// base + the set lanes of m below this one
+__device__ __forceinline__ int lanes_before(uint64_t m, int base) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)base));
+}
+// the float bits of a sortable key
+__device__ __forceinline__ uint32_t fkey_bits(uint32_t k) { return k ^ (~(uint32_t)((int32_t)k >> 31) | 0x80000000u); }
+
+// A work-group owns QR queries (16, or 8 of the 16 matrix columns for long frames) and walks the
+// frames of its group. Per frame: the waves share out the frame's 16-key tiles, score them on the
+// matrix core (v_mfma_f32_16x16x32_bf16, S^T = K . Q^T) and put the fp32 scores into LDS rows,
+// one row per query (a tile's loads read whole 128-byte rows and reach the A fragments through a
+// swizzled LDS stage: fragments read straight from global memory touch 16 rows per 16 lanes, which
+// the address unit takes four times as long for); then every wave selects whole rows, a lane holding NV scores of its row:
+//   - a threshold with k .. CAP scores at or above it (or unordered: a NaN never drops out): a first
+//     guess from the lane maxima (one compare and ballot per bisection step), then wave-wide counts
+//     of all scores until the count falls into the window, which mostly takes one or two;
+//   - those candidates, as composite keys, into the row's own LDS space, then a bitonic sort over
+//     the wave (DPP exchanges) and the k best written out in order.
+// A row whose counts jump over the window (more than CAP - k equal scores, or infinities) takes the
+// exact threshold by 32 counts on the sortable keys, equal keys from the lowest index on.
+// CAP is 64 for k <= 32 (one sorted register per lane), else 128 (two, merged).
+// The next frame's fragments load while the rows of this one are selected (NV <= 24; longer frames
+// have no registers for it).
+// Bound by the VALU of the selection and the loads' latency: a work-group of 16 waves fills a CU
+// (its LDS rows take 74 KB at 1036 keys and 90 KB at 1369), scoring takes 220 us of 497 at
+// 16 x 1036 tokens, top-64, and the 128-entry sort 80 us. It replaced a dump of every score to a
+// workspace in HBM and a radix select of eight digit passes over LDS bins per row: 1630 -> 497 us
+// there, 21.9 -> 6.8 ms at 48 x 1369 tokens. A 64-bit sort of (score, index)
+// took 220 VALU instructions against 82, fragments loaded without the LDS stage 50 us more.
+template <int NV, bool FLAT>
+__global__ __launch_bounds__(64 * kRowWaves) void topk_rows_kernel(TopkParams p) {
+  constexpr int QR = NV <= 24 ? 16 : 8;
+  constexpr int kTiles = NV / 4 + (NV % 4 != 0);  // 16-key tiles of a wave
+  const int cap = p.ke <= 32 ? 64 : 128;
+  // m scores at or above a threshold, spread at random, reach 64 (1 - e^(-m / 64)) of the lane
+  // maxima: aim at the middle of the window
+  const int lanes = (int)(64.f * (1.f - __expf(-sqrtf((float)p.ke * cap) / 64.f)));
+  constexpr bool kPrefetch = NV <= 24;
+  // row stride = 4 (mod 64) words: the 16-byte score stores of the 16 query columns take distinct banks
+  // (NV = 64 has no LDS left for it)
+  __shared__ __align__(16) float rows[QR][NV * 64 + (NV < 64 ? 4 : 0)];
+  // a wave's tile on its way from coalesced loads to A fragments: 16 rows of 8 chunks, swizzled
+  __shared__ __align__(16) char stage[kRowWaves][2048];
+  static_assert(sizeof(rows) / QR >= 128 * 8, "a row's candidates fit its LDS space");
+  const int tid = tid_x(), lane = tid & 63, col = lane & 15, kq = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t q0 = (int64_t)bid_x() * QR;
+  bf16x8 qf[2];
+  {
+    const int64_t qi = q0 + col;
+    const bool ok = col < QR && qi < p.nq;
+    const u32x4* qs = reinterpret_cast<const u32x4*>(rows_at(p.qptr, p.q_rs, p.q_base, p.q_rpf, p.q_frs, ok ? qi : 0));
+#pragma unroll
+    for (int s = 0; s < 2; ++s) qf[s] = __builtin_bit_cast(bf16x8, ok ? qs[4 * s + kq] : u32x4{0, 0, 0, 0});
+  }
+  const int f_lo = __builtin_amdgcn_readfirstlane((int)((int64_t)p.F * bid_y() / p.fgroups));
+  const int f_hi = __builtin_amdgcn_readfirstlane((int)((int64_t)p.F * (bid_y() + 1) / p.fgroups));
+  const char* kb0 = reinterpret_cast<const char*>(p.kptr + p.k_base * p.k_rs);
+  const int64_t fbytes = p.k_fst * p.k_rs * 2;
+  const int krow = (int)p.k_rs * 2;  // FLAT: a frame's rows stay below 2^31 bytes
+  // tile w + 16 i of frame f: lane l holds chunk l % 8 of rows l / 8 and 8 + l / 8, so that a load
+  // reads whole rows (rows past the frame's end read its last row)
+  const int lrow = lane >> 3, lchk = lane & 7;
+  auto load_tile = [&](int f, int i, u32x4 (&kt)[2]) __attribute__((always_inline)) {
+    int lrow = lane >> 3;
+    asm volatile("" : "+v"(lrow));  // offsets computed anew, not held across the frame loop
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int j = min(16 * (w + kRowWaves * i) + 8 * h + lrow, p.P - 1);
+      if constexpr (FLAT) {
+        const char* fb = kb0 + f * fbytes;  // wave-uniform, plus a 32-bit lane offset
+        kt[h] = *reinterpret_cast<const u32x4*>(fb + (uint32_t)(j * krow + 16 * lchk));
+      } else {
+        const __bf16* row = rows_at(p.kptr, p.k_rs, p.k_base, p.k_rpf, p.k_frs, (int64_t)f * p.P + j);
+        kt[h] = reinterpret_cast<const u32x4*>(row)[lchk];
+      }
+    }
+  };
+  auto score_tile = [&](int i, const u32x4 (&kt)[2]) __attribute__((always_inline)) {
+    char* st = stage[w];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int r = 8 * h + lrow;
+      *reinterpret_cast<u32x4*>(st + r * 128 + ((lchk ^ swz8(r)) << 4)) = kt[h];
+    }
+    f32x4 d = {};
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const bf16x8 kf = *reinterpret_cast<const bf16x8*>(st + col * 128 + (((4 * s + kq) ^ swz8(col)) << 4));
+      d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[s], d, 0, 0, 0);
+    }
+    const int tile = w + kRowWaves * i;
+    if (16 * tile + 16 > p.P) {  // positions past the frame's end never reach a threshold
+      int left = p.P - 16 * tile - 4 * kq;
+      asm volatile("" : "+v"(left));
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (r >= left) d[r] = -__builtin_inff();
+    }
+    if (tile < 4 * NV && col < QR) *reinterpret_cast<f32x4*>(&rows[col][16 * tile + 4 * kq]) = d;
+  };
+  u32x4 kt[kPrefetch ? kTiles : 1][2];
+  auto prefetch = [&](int f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i) load_tile(f, i, kt[i]);
+  };
+  if constexpr (kPrefetch) prefetch(f_lo);
+
+  for (int f = f_lo; f < f_hi; ++f) {
+    if constexpr (kPrefetch) {
+#pragma unroll
+      for (int i = 0; i < kTiles; ++i) score_tile(i, kt[i]);
+    } else {
+#pragma unroll 2
+      for (int i = 0; i < kTiles; ++i) {
+        load_tile(f, i, kt[0]);
+        score_tile(i, kt[0]);
+      }
+    }
+    __syncthreads();
+    if constexpr (kPrefetch)
+      if (f + 1 < f_hi) prefetch(f + 1);
+    for (int r = w; r < QR; r += kRowWaves) {
+      if (q0 + r >= p.nq) break;
+      float* row = rows[r];
+      // opaque per row: keeps the compiler from holding NV key indices and compares in registers
+      // across the frame loop
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      u32x2* buf = reinterpret_cast<u32x2*>(row);  // candidates: score bits, key index
+      float v[NV];  // score of key lane + 64 i
+#pragma unroll
+      for (int i = 0; i < NV; ++i) v[i] = row[ln + 64 * i];
+      auto count = [&](float t) {  // scores at or above t, wave-wide
+        int c = 0;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) c += __popcll(__builtin_amdgcn_ballot_w64(!(v[i] < t)));
+        return c;
+      };
+      float t = -0x1.fffffep127f;  // P <= cap: every finite score is a candidate
+      bool found = false;
+      if (p.P <= cap) {
+        const int c = count(t);
+        found = c >= p.ke && c <= cap;
+      } else {
+        float lmax = v[0];
+#pragma unroll
+        for (int i = 1; i < NV; ++i) lmax = fmaxf(lmax, v[i]);
+        float hi = wave_reduce32(lmax, [](float a, float b) { return fmaxf(a, b); });
+        float lo = wave_reduce32(lmax, [](float a, float b) { return fminf(a, b); });
+        if (p.ke > 64) lo -= 2.f * (hi - lo);  // 64 scores reach the least lane maximum: look below it
+        // first guess: the value that about `lanes` of the 64 lane maxima reach
+        float a = lo, b = hi;
+        t = 0.5f * a + 0.5f * b;
+        for (int step = 0; step < 10; ++step) {
+          const int c = __popcll(__builtin_amdgcn_ballot_w64(!(lmax < t)));
+          if (c > lanes + 2) a = t;
+          else if (c < lanes - 2) b = t;
+          else break;
+          t = 0.5f * a + 0.5f * b;
+        }
+        for (int step = 0; step < 32; ++step) {
+          if (!(t > lo && t < hi)) break;
+          const int c = count(t);
+          if (c < p.ke) hi = t;
+          else if (c > cap) lo = t;
+          else {
+            found = true;
+            break;
+          }
+          t = 0.5f * lo + 0.5f * hi;
+        }
+      }
+      int n = 0;  // candidates, in increasing key index
+      if (found) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+          const bool take = !(v[i] < t);
+          const uint64_t m = __builtin_amdgcn_ballot_w64(take);
+          const int at = lanes_before(m, n);
+          if (take) buf[at] = u32x2{__builtin_bit_cast(uint32_t, v[i]), (uint32_t)(ln + 64 * i)};
+          n += __popcll(m);
+        }
+      } else {
+        asm volatile("" : "+v"(ln));
+        uint32_t u[NV];  // sortable keys, 0 past the frame's end
+#pragma unroll
+        for (int i = 0; i < NV; ++i) u[i] = ln + 64 * i < p.P ? fkey(v[i]) : 0;
+        uint32_t thr = 0;  // the largest key with at least ke keys at or above it
+#pragma unroll 1
+        for (int b = 31; b >= 0; --b) {
+          const uint32_t cand = thr | (1u << b);
+          int c = 0;
+#pragma unroll
+          for (int i = 0; i < NV; ++i) c += __popcll(__builtin_amdgcn_ballot_w64(u[i] >= cand));
+          if (c >= p.ke) thr = cand;
+        }
+        int need = p.ke;  // keys equal to thr to take
+#pragma unroll
+        for (int i = 0; i < NV; ++i) need -= __popcll(__builtin_amdgcn_ballot_w64(u[i] > thr));
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+          const bool eq = u[i] == thr && ln + 64 * i < p.P;
+          const uint64_t meq = __builtin_amdgcn_ballot_w64(eq);
+          const bool take = u[i] > thr || (eq && lanes_before(meq, 0) < need);
+          const uint64_t m = __builtin_amdgcn_ballot_w64(take);
+          const int at = lanes_before(m, n);
+          if (take) buf[at] = u32x2{fkey_bits(u[i]), (uint32_t)(ln + 64 * i)};
+          n += __popcll(m);
+          need -= min(need, (int)__popcll(meq));
+        }
+        t = __builtin_bit_cast(float, fkey_bits(thr));
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      int32_t* o = p.idx + (q0 + r) * ((int64_t)p.F * p.ke) + (int64_t)f * p.ke;
+      const u32x2 c0 = buf[lane], c1 = buf[64 + lane];  // (entries from n on are not used)
+      const uint32_t k0 = fkey(__builtin_bit_cast(float, c0[0])), k1 = fkey(__builtin_bit_cast(float, c1[0]));
+      const uint32_t kt0 = fkey(t);
+      const bool in0 = lane < n, in1 = 64 + lane < n;
+      if (!__builtin_amdgcn_ballot_w64((in0 && (k0 - kt0) >> 25) || (in1 && (k1 - kt0) >> 25))) {
+        // every candidate within 2^25 float steps of the threshold: one 32-bit word orders them by
+        // score, then by slot (slots are in key order), with the slot in its low 7 bits
+        uint32_t x = in0 ? ((k0 - kt0) << 7) | (uint32_t)(127 - lane) : 0u;
+        uint32_t y = in1 ? ((k1 - kt0) << 7) | (uint32_t)(63 - lane) : 0u;
+        lane_sort128(x, y, n, p.ke > 64, lane);
+        if (lane < p.ke) o[lane] = f * p.P + (int)buf[127 - (x & 127)][1];
+        if (64 + lane < p.ke) o[64 + lane] = f * p.P + (int)buf[127 - (y & 127)][1];
+      } else {
+        uint64_t x = in0 ? ((uint64_t)k0 << 32) | (0xFFFFFFFEu - c0[1]) : 0;
+        uint64_t y = in1 ? ((uint64_t)k1 << 32) | (0xFFFFFFFEu - c1[1]) : 0;
+        lane_sort128(x, y, n, p.ke > 64, lane);
+        if (lane < p.ke) o[lane] = f * p.P + (int)ckey_index(x);
+        if (64 + lane < p.ke) o[64 + lane] = f * p.P + (int)ckey_index(y);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Bytes of one query's workspace share (frames x frame length rounded up to 64, fp32).
 static int64_t large_row_bytes(int frames, int per_frame) { return (int64_t)frames * (64 * ((per_frame + 63) / 64)) * 4; }
 
 // Queries per chunk: a workspace of at most 1 GiB in whole work-groups of 128 queries (at least one).
@@ -503,44 +707,44 @@ static int64_t large_chunk_rows(int n_q, int frames, int per_frame) {
   return nqc < nq128 ? nqc : nq128;
 }
 
-// The caller's workspace holds the scores of `nqc` queries at a time (whole work-groups of 128);
-// chunks run one after another on the stream, so one workspace serves every chunk.
-static int token_topk_large(TopkParams p, int n_q, void* workspace, int64_t workspace_bytes, hipStream_t st) {
-  const int tiles = (p.P + 63) / 64;
-  p.ppad = 64 * tiles;
+template <int NV, bool FLAT = true>
+static void launch_rows(const TopkParams& p, dim3 grid, hipStream_t st) {
+  hipLaunchKernelGGL((topk_rows_kernel<NV, FLAT>), grid, dim3(64 * kRowWaves), 0, st, p);
+}
+
+// Top-k of LDS score rows. The caller's workspace is checked as the ABI states and not used.
+static int token_topk_large(TopkParams p, const void* workspace, int64_t workspace_bytes, hipStream_t st) {
   const int64_t row_bytes = large_row_bytes(p.F, p.P);
-  int64_t nqc = workspace_bytes / row_bytes / 128 * 128;
-  if (!workspace || nqc < 128)
+  if (!workspace || workspace_bytes / row_bytes / 128 * 128 < 128)
     return fail(SAF3R_ERR_INVALID,
                 "saf3r_token_topk: min(topk, per_frame) > 16 needs a workspace of at least %lld bytes "
                 "(saf3r_token_topk_workspace_bytes), got %lld",
                 (long long)(128 * row_bytes), (long long)(workspace ? workspace_bytes : 0));
-  if (nqc > n_q) nqc = n_q;
-  p.ws = static_cast<float*>(workspace);
-  const int nv = tiles <= 4 ? 4 : tiles <= 8 ? 8 : tiles <= 12 ? 12 : tiles <= 16 ? 16 : tiles <= 24 ? 24
-                 : tiles <= 32 ? 32 : tiles <= 48 ? 48 : 64;
-  for (int64_t q0 = 0; q0 < n_q; q0 += nqc) {
-    const int64_t q1 = q0 + nqc < n_q ? q0 + nqc : n_q;
-    p.q_begin = q0;
-    p.nq = (int)q1;
-    const dim3 g1((unsigned)((q1 - q0 + 127) / 128), (unsigned)p.F);
-    if (p.kmode == 2) hipLaunchKernelGGL((token_topk_kernel<1, false, true>), g1, dim3(256), 0, st, p);
-    else hipLaunchKernelGGL((token_topk_kernel<1, true, true>), g1, dim3(256), 0, st, p);
-    if (int rc = check_launch("saf3r_token_topk")) return rc;
-    const dim3 g2((unsigned)(((q1 - q0) * p.F + 3) / 4));
-    switch (nv) {
-      case 4: hipLaunchKernelGGL(topk_large_kernel<4>, g2, dim3(256), 0, st, p.ws, q0, q1, p.F, p.P, p.ppad, p.ke, p.idx); break;
-      case 8: hipLaunchKernelGGL(topk_large_kernel<8>, g2, dim3(256), 0, st, p.ws, q0, q1, p.F, p.P, p.ppad, p.ke, p.idx); break;
-      case 12: hipLaunchKernelGGL(topk_large_kernel<12>, g2, dim3(256), 0, st, p.ws, q0, q1, p.F, p.P, p.ppad, p.ke, p.idx); break;
-      case 16: hipLaunchKernelGGL(topk_large_kernel<16>, g2, dim3(256), 0, st, p.ws, q0, q1, p.F, p.P, p.ppad, p.ke, p.idx); break;
-      case 24: hipLaunchKernelGGL(topk_large_kernel<24>, g2, dim3(256), 0, st, p.ws, q0, q1, p.F, p.P, p.ppad, p.ke, p.idx); break;
-      case 32: hipLaunchKernelGGL(topk_large_kernel<32>, g2, dim3(256), 0, st, p.ws, q0, q1, p.F, p.P, p.ppad, p.ke, p.idx); break;
-      case 48: hipLaunchKernelGGL(topk_large_kernel<48>, g2, dim3(256), 0, st, p.ws, q0, q1, p.F, p.P, p.ppad, p.ke, p.idx); break;
-      default: hipLaunchKernelGGL(topk_large_kernel<64>, g2, dim3(256), 0, st, p.ws, q0, q1, p.F, p.P, p.ppad, p.ke, p.idx); break;
-    }
-    if (int rc = check_launch("saf3r_token_topk")) return rc;
-  }
-  return SAF3R_OK;
+  const int nv = (p.P + 63) / 64;
+  const int qr = nv <= 24 ? 16 : 8;
+  const int64_t nb = ((int64_t)p.nq + qr - 1) / qr;
+  p.fgroups = frame_groups(nb, p.F, 1, 2);
+  const dim3 grid((unsigned)nb, (unsigned)p.fgroups);
+  if (p.kmode == 2) {  // the general row map: four lengths
+    if (nv <= 8) launch_rows<8, false>(p, grid, st);
+    else if (nv <= 24) launch_rows<24, false>(p, grid, st);
+    else if (nv <= 32) launch_rows<32, false>(p, grid, st);
+    else launch_rows<64, false>(p, grid, st);
+  } else if (nv <= 4) launch_rows<4>(p, grid, st);
+  else if (nv <= 6) launch_rows<6>(p, grid, st);
+  else if (nv <= 8) launch_rows<8>(p, grid, st);
+  else if (nv <= 10) launch_rows<10>(p, grid, st);
+  else if (nv <= 12) launch_rows<12>(p, grid, st);
+  else if (nv <= 14) launch_rows<14>(p, grid, st);
+  else if (nv <= 16) launch_rows<16>(p, grid, st);
+  else if (nv <= 18) launch_rows<18>(p, grid, st);
+  else if (nv <= 20) launch_rows<20>(p, grid, st);
+  else if (nv <= 22) launch_rows<22>(p, grid, st);
+  else if (nv <= 24) launch_rows<24>(p, grid, st);
+  else if (nv <= 32) launch_rows<32>(p, grid, st);
+  else if (nv <= 48) launch_rows<48>(p, grid, st);
+  else launch_rows<64>(p, grid, st);
+  return check_launch("saf3r_token_topk");
 }
 
 }  // namespace saf3r
@@ -596,12 +800,9 @@ extern "C" int saf3r_token_topk(const saf3r_rows* q, const saf3r_rows* k, int n_
   p.P = per_frame;
   p.ke = ke;
   p.idx = idx;
-  p.ws = nullptr;
-  p.q_begin = 0;
-  p.ppad = 0;
   p.fgroups = 1;
   hipStream_t st = (hipStream_t)stream;
-  if (ke > 16) return token_topk_large(p, n_q, workspace, workspace_bytes, st);
+  if (ke > 16) return token_topk_large(p, workspace, workspace_bytes, st);
   if (p.ke <= 1) return launch_topk<1>(p, st);
   if (p.ke <= 2) return launch_topk<2>(p, st);
   if (p.ke <= 4) return launch_topk<4>(p, st);

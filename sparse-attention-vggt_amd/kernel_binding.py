@@ -11,7 +11,7 @@ the reference's names, arguments and output shapes and dtypes:
   (``saf3r/triton/fused_qk_topk.py:120-217``): q [B, Nq, D], k [B, Nk, D] -> int32
   [B, Nq, (Nk / num_toks_per_img) * min(topk, num_toks_per_img)], per-frame top-k of bf16 q.k, frame-major,
   score descending, ties to the lower key. Every batch element is computed (one C call each, on the
-  current stream, sharing one score workspace).
+  current stream, sharing one workspace).
 
 This build supports D = Dv = 64 (VGGT's head_dim); other sizes raise ``ValueError`` (the reference
 autotunes BLOCK_D for any D). The reference's assertions are ``ValueError``s here; a C-ABI failure
@@ -119,6 +119,8 @@ def compute_qk_topk_indices_fused(q: torch.Tensor, k: torch.Tensor, topk: int,
     nbytes = lib.saf3r_token_topk_workspace_bytes(Nq, frames, num_toks_per_img, topk)
     if nbytes < 0:
         raise RuntimeError(lib.saf3r_last_error().decode(errors="replace"))
+    if nbytes:  # the entry accepts a share for 128 queries
+        nbytes = min(nbytes, lib.saf3r_token_topk_workspace_bytes(1, frames, num_toks_per_img, topk))
     ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8) if nbytes else None
     for b in range(B):
         _check(lib.saf3r_token_topk(ctypes.byref(_rows(q_bf[b])), ctypes.byref(_rows(k_bf[b])), Nq, frames,

@@ -507,6 +507,16 @@ def token_topk_workspace_bytes(n_q: int, frames: int, per_frame: int, topk: int)
     return int(nbytes)
 
 
+def _token_topk_workspace(n_q: int, frames: int, per_frame: int, topk: int, device) -> torch.Tensor | None:
+    """The smallest workspace ``saf3r_token_topk`` accepts for these sizes (a share for 128 queries; none
+    for top-k <= 16)."""
+    nbytes = token_topk_workspace_bytes(n_q, frames, per_frame, topk)
+    if not nbytes:
+        return None
+    return torch.empty(min(nbytes, token_topk_workspace_bytes(1, frames, per_frame, topk)), dtype=torch.uint8,
+                       device=device)
+
+
 def token_topk(q: torch.Tensor, k: torch.Tensor, frames: int, per_frame: int, topk: int,
                qrows: _lib.Rows | None = None, krows: _lib.Rows | None = None, n_q: int | None = None,
                workspace: torch.Tensor | None = None):
@@ -514,16 +524,15 @@ def token_topk(q: torch.Tensor, k: torch.Tensor, frames: int, per_frame: int, to
     q [Nq, 64], k [frames*per_frame, 64] -> int32 [Nq, frames*min(topk, per_frame)], or with a batch
     dimension q [B, Nq, 64], k [B, frames*per_frame, 64] -> [B, Nq, frames*min(topk, per_frame)]
     (one call per batch element, as the reference's grid dimension 1 runs them; ``:187``). q and k
-    are rounded to bf16, as the reference's kernel multiplies bf16 tiles. Above top-16 the score
-    workspace is a torch allocation of ``token_topk_workspace_bytes`` (or ``workspace``)."""
+    are rounded to bf16, as the reference's kernel multiplies bf16 tiles. Above top-16 the entry
+    takes a workspace (the smallest one it accepts, or ``workspace``)."""
     _need_cuda(q, k) if qrows is None or krows is None else _need_cuda(q)
     if qrows is None and krows is None and q.dim() == 3:
         if k is None or k.dim() != 3 or k.shape[0] != q.shape[0]:
             raise ValueError("batched q needs k of the same batch size")
         ws = workspace
         if ws is None:
-            nbytes = token_topk_workspace_bytes(q.shape[1], frames, per_frame, topk)
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+            ws = _token_topk_workspace(q.shape[1], frames, per_frame, topk, q.device)
         return torch.stack([token_topk(q[b], k[b], frames, per_frame, topk, workspace=ws)
                             for b in range(q.shape[0])])
     lib = _lib.load()
@@ -543,8 +552,7 @@ def token_topk(q: torch.Tensor, k: torch.Tensor, frames: int, per_frame: int, to
     ke = min(topk, per_frame)
     idx = torch.empty(n_q, frames * ke, dtype=torch.int32, device=q.device)
     if workspace is None:
-        nbytes = token_topk_workspace_bytes(n_q, frames, per_frame, topk)
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+        workspace = _token_topk_workspace(n_q, frames, per_frame, topk, q.device)
     _mark("token_topk", "start")
     _lib.check(lib.saf3r_token_topk(ctypes.byref(qrows), ctypes.byref(krows), n_q, frames, per_frame, topk,
                                     _ptr(idx), _ptr(workspace), 0 if workspace is None else workspace.numel(),
