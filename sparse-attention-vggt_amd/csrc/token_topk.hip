@@ -45,13 +45,18 @@ __device__ inline uint64_t partner_u64(uint64_t x) {
   return ((uint64_t)phi << 32) | plo;
 }
 
+// the float bits of a sortable key
+__device__ __forceinline__ uint32_t fkey_bits(uint32_t k) { return k ^ (~(uint32_t)((int32_t)k >> 31) | 0x80000000u); }
+
 // Candidate buffer of pass 2: per lane up to kCand candidates (float bits << 32 | key index), entry i
 // of thread tid at cbuf[i * 256 + tid] (a lane's entries all sit in its own bank pair: no conflicts
 // whatever the fill levels), emptied into the lane's running top-K at the end of each frame. A lane
-// with more candidates than that in one frame (ties on a large scale) loses the rest and has its
-// frame recomputed directly at the frame's end (see token_topk_kernel).
+// with more candidates than that in one frame (ties, or neighbouring keys that share a group) loses
+// the rest and has its frame scanned again at the frame's end (see token_topk_kernel).
 template <int K>
 constexpr int cand_cap() { return K <= 8 ? 12 : 24; }
+constexpr int kGroup = 8;  // candidates whose wave masks are formed together
+constexpr int kStep = 2;   // candidates that share a wave-uniform branch
 constexpr int kStages = 3;  // K tiles in flight: the tile of step t + 2 loads while step t computes
 
 // K-th largest of the running float list t (descending, -inf = empty) after inserting x.
@@ -71,10 +76,17 @@ __device__ inline void fmax_insert(float (&t)[K], float x) {
 //           group maxima of a query (its two lane halves) is a lower bound tau of the query's K-th
 //           best score in the frame (they are 2G >= K distinct candidates);
 //   pass 2: only candidates with score >= tau (or unordered: a NaN never drops out) are appended to
-//           the lane's LDS buffer; a candidate costs one compare and a wave-uniform branch unless
-//           some lane of the wave keeps it. A lane whose buffer overflowed in the frame is served
-//           at the frame's end by a direct pass of its wave over the frame's key rows in global
-//           memory (same MFMAs, so the same scores) that inserts every candidate >= tau.
+//           the lane's LDS buffer; a candidate costs one compare, and two share a wave-uniform branch
+//           unless some lane of the wave keeps one (one branch each: 2 - 5% slower, one for four: the
+//           same). A lane whose buffer overflowed is served at the frame's end by a scan of its wave
+//           over the frame's key rows in global memory (same MFMAs, so the same scores) with the K-th
+//           best of its buffered candidates as the bound, which rises as better ones are found.
+// The second 32 keys of a tile go to the groups in a rotated order (G <= 16): with the same order in
+// both halves, the keys of one image column shared a group on grids 32 patches wide and neighbouring
+// ones on grids of 33, tau fell and frames overflowed (24 frames of 19 x 33, top-8: 153 us against 226).
+// Queries past the last one keep nothing: as ties at 0 they overflowed on every frame, which cost
+// the last work-group of each frame group twice its time (48 x 1369 tokens, top-4, with single-frame
+// groups allowed: 1727 us against 1415).
 // A few candidates per query and frame pass (about 3 of 1369 for top-4 of N(0,1) scores), so the
 // composite-key insertion that dominates a one-pass selection runs a few times per frame instead
 // of for every candidate. Key tiles stream through a 3-stage LDS ring filled by LDS-DMA loads
@@ -82,11 +94,9 @@ __device__ inline void fmax_insert(float (&t)[K], float x) {
 // Step t reads its K fragments, selects over the scores of step t - 1 while those reads are in
 // flight, then issues its MFMAs into the same registers; the two waves of a SIMD alternate their
 // VALU and MFMA phases.
-template <int K, bool FLAT>
+template <int K, int G, bool FLAT>
 __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkParams p) {
-  // groups per lane (2G >= K maxima per query): more groups give a tighter tau for larger K, so that
-  // the candidates of a lane fit its buffer
-  constexpr int G = K <= 4 ? 8 : 2 * K;
+  // G groups per lane: 2G >= K maxima per query
   __shared__ __align__(16) char ring[kStages][8192];
   constexpr int kCand = cand_cap<K>();
   __shared__ uint64_t cbuf[(kCand + 1) * 256];
@@ -192,31 +202,45 @@ __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkPar
   // candidate e of this lane: key 32*(e>>4) + 8*((e&15)>>2) + 4*half + (e&3) of the tile
   auto kpos = [](int e) { return 32 * (e >> 4) + 8 * ((e & 15) >> 2) + (e & 3); };
   int f = f_lo, ps = 0, u = 0;  // frame, pass and tile of the step being selected
-  // Frame f again, for the lanes flagged `over`: every candidate >= tau goes straight into a[]. K
-  // fragments come from global memory (this lane's rows col and 32 + col of each tile, chunks
-  // 4 half .. 4 half + 3), the MFMAs run as in the main loop on the whole wave.
+  // Frame f again, for the lanes flagged `over` (their a[] holds the best K of the buffered ones). K
+  // fragments come from global memory (this lane's rows col of each half tile, chunks 4 half ..
+  // 4 half + 3), the next ones loading while these are scored; the MFMAs run as in the main loop.
+  // Keys come in increasing order, so once a[] is full only a higher score than its last can enter.
   auto direct = [&](bool over) __attribute__((always_inline)) {
+    int cl = col, hf = half;
+    asm volatile("" : "+v"(cl), "+v"(hf));  // addresses formed here, not held through the main loop
+    float bound = over ? fmaxf(tau, __builtin_bit_cast(float, fkey_bits((uint32_t)(a[K - 1] >> 32)))) : __builtin_inff();
     if (over) {
 #pragma unroll
       for (int e = 0; e < K; ++e) a[e] = 0;
     }
-    for (int h2 = 0; h2 < 2 * tiles_pf; ++h2) {  // 32 keys at a time: rows 32 h2 + col
-      const int r = min(32 * h2 + col, p.P - 1);
+    auto fetch = [&](int h2, u32x4 (&t)[4]) __attribute__((always_inline)) {  // rows 32 h2 + col
+      const int r = min(32 * h2 + cl, p.P - 1);
       const __bf16* row;
       if constexpr (FLAT) row = reinterpret_cast<const __bf16*>(kb0 + f * fbytes) + (int64_t)r * p.k_rs;
       else row = rows_at(p.kptr, p.k_rs, p.k_base, p.k_rpf, p.k_frs, (int64_t)f * p.P + r);
-      const u32x4* src = reinterpret_cast<const u32x4*>(row + 32 * half);
-      bf16x8 fa[4];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) fa[s] = __builtin_bit_cast(bf16x8, src[s]);
+      for (int s = 0; s < 4; ++s) t[s] = reinterpret_cast<const u32x4*>(row + 32 * hf)[s];
+    };
+    u32x4 t[4];
+    fetch(0, t);
+#pragma unroll 1
+    for (int h2 = 0; h2 < 2 * tiles_pf; ++h2) {
       f32x16 d = {};
 #pragma unroll
-      for (int s = 0; s < 4; ++s) d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s], qfrag[s], d, 0, 0, 0);
-      const int pb = 32 * h2 + 4 * half;
+      for (int s = 0; s < 4; ++s)
+        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, t[s]), qfrag[s], d, 0, 0, 0);
+      fetch(h2 + 1, t);  // (past the end: the last row again)
+      const int pb = 32 * h2 + 4 * hf;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int pp = pb + kpos(e);
-        if (over && !(d[e] < tau) && pp < p.P) topk_insert<K>(a, ckey(d[e], (uint32_t)pp));
+        const bool keep = over && !(d[e] < bound) && pp < p.P;
+        if (__builtin_amdgcn_ballot_w64(keep)) {
+          topk_insert<K>(a, keep ? ckey(d[e], (uint32_t)pp) : 0);
+          // (a NaN bound keeps every candidate; the insertion decides)
+          if (a[K - 1]) bound = __builtin_bit_cast(float, fkey_bits((uint32_t)(a[K - 1] >> 32) + 1));
+        }
       }
     }
   };
@@ -228,77 +252,85 @@ __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkPar
     auto sc = [&](int e) { return e < 16 ? s0[e] : s1[e - 16]; };
     if (ps == 0) {
 #pragma unroll
-      for (int e = 0; e < 32; ++e)
-        gmax[e % G] = fmaxf(gmax[e % G], (!PADDED || kpos(e) < lim) ? sc(e) : -__builtin_inff());
-      if (u == tiles_pf - 1) {
-        // K-th largest of this query's 2G group maxima (this lane's and its partner half's)
-        float top[K];
-#pragma unroll
-        for (int i = 0; i < K; ++i) top[i] = -__builtin_inff();
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          uint32_t b = __builtin_bit_cast(uint32_t, gmax[g]);
-          auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-          const float other = __builtin_bit_cast(float, (uint32_t)(half ? r[0] : r[1]));
-          fmax_insert<K>(top, gmax[g]);
-          fmax_insert<K>(top, other);
-          gmax[g] = -__builtin_inff();
-        }
-        tau = top[K - 1];
+      for (int e = 0; e < 32; ++e) {
+        const int g = G <= 16 && e >= 16 ? (e + 9) % G : e % G;
+        gmax[g] = fmaxf(gmax[g], (!PADDED || kpos(e) < lim) ? sc(e) : -__builtin_inff());
       }
     } else {
 #pragma unroll
-      for (int e0 = 0; e0 < 32; e0 += 8) {
-        // the wave masks of 8 candidates first, then one uniform branch each: the compares' latency
-        // is paid once per 8
-        uint64_t bm[8];
+      for (int e0 = 0; e0 < 32; e0 += kGroup) {
+        // the wave masks of a group of candidates first, then one uniform branch each: the compares' latency
+        // is paid once per group
+        uint64_t bm[kGroup];
 #pragma unroll
-        for (int i = 0; i < 8; ++i)  // >= tau, or unordered
+        for (int i = 0; i < kGroup; ++i)  // >= tau, or unordered
           bm[i] = __builtin_amdgcn_ballot_w64(!(sc(e0 + i) < tau) && (!PADDED || kpos(e0 + i) < lim));
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          if (bm[i]) {
-            // every lane writes its next entry; only the lanes that keep the candidate advance (a
-            // full buffer stays on the spare row)
-            const int e = e0 + i;
-            const bool keep = !(sc(e) < tau) && (!PADDED || kpos(e) < lim);
-            const uint32_t at = min(wa, wspare);
-            wa += keep ? 2048u : 0u;
-            auto* ew = reinterpret_cast<__attribute__((address_space(3))) uint32_t*>(at);
-            ew[0] = (uint32_t)(pbase + kpos(e));
-            ew[1] = __builtin_bit_cast(uint32_t, sc(e));
+        for (int i0 = 0; i0 < kGroup; i0 += kStep) {
+          uint64_t any = bm[i0];
+#pragma unroll
+          for (int i = i0 + 1; i < i0 + kStep; ++i) any |= bm[i];
+          if (any) {
+            // every lane writes its next entry; only the lanes that keep the candidate advance
+#pragma unroll
+            for (int i = i0; i < i0 + kStep; ++i) {
+              const int e = e0 + i;
+              const bool keep = !(sc(e) < tau) && (!PADDED || kpos(e) < lim);
+              const uint32_t at = min(wa, wspare);
+              wa += keep ? 2048u : 0u;
+              auto* ew = reinterpret_cast<__attribute__((address_space(3))) uint32_t*>(at);
+              ew[0] = (uint32_t)(pbase + kpos(e));
+              ew[1] = __builtin_bit_cast(uint32_t, sc(e));
+            }
           }
         }
       }
-      if (u == tiles_pf - 1) {
-        // empty the buffer (or recompute an overflowed lane), merge the partner half's list, then
-        // write this frame's indices
-        const bool over = count() > kCand;
-        if (__builtin_amdgcn_ballot_w64(over)) direct(over);
-        if (over) wa = wa0;
-        flush();
-        uint64_t b[K];
+    }
+  };
+  // the end of a pass over frame f
+  auto pass_end = [&]() __attribute__((always_inline)) {
+    if (ps == 0) {
+      // K-th largest of this query's 2G group maxima (this lane's and its partner half's)
+      float top[K];
 #pragma unroll
-        for (int e = 0; e < K; ++e) b[e] = partner_u64(a[e]);
+      for (int i = 0; i < K; ++i) top[i] = -__builtin_inff();
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        uint32_t b = __builtin_bit_cast(uint32_t, gmax[g]);
+        auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+        const float other = __builtin_bit_cast(float, (uint32_t)(half ? r[0] : r[1]));
+        fmax_insert<K>(top, gmax[g]);
+        fmax_insert<K>(top, other);
+        gmax[g] = -__builtin_inff();
+      }
+      // lanes past the last query score 0 everywhere: they keep nothing (as ties they would fill
+      // their buffers over and over)
+      tau = qvalid ? top[K - 1] : __builtin_inff();
+    } else {
+      // empty the buffer (and scan the frame again for overflowed lanes), merge the partner half's
+      // list, then write this frame's indices
+      const bool over = count() > kCand;
+      flush();
+      if (__builtin_amdgcn_ballot_w64(over)) direct(over);
+      uint64_t b[K];
+#pragma unroll
+      for (int e = 0; e < K; ++e) b[e] = partner_u64(a[e]);
+#pragma unroll
+      for (int e = 0; e < K; ++e)
+        if (b[e] > a[K - 1]) topk_insert<K>(a, b[e]);
+      if (qvalid && half == 0) {
+        int32_t* o = p.idx + qi * ((int64_t)p.F * p.ke) + (int64_t)f * p.ke;
 #pragma unroll
         for (int e = 0; e < K; ++e)
-          if (b[e] > a[K - 1]) topk_insert<K>(a, b[e]);
-        if (qvalid && half == 0) {
-          int32_t* o = p.idx + qi * ((int64_t)p.F * p.ke) + (int64_t)f * p.ke;
-#pragma unroll
-          for (int e = 0; e < K; ++e)
-            if (e < p.ke) o[e] = a[e] ? (int32_t)(f * p.P + ckey_index(a[e])) : -1;
-        }
-#pragma unroll
-        for (int e = 0; e < K; ++e) a[e] = 0;
-        tau = -__builtin_inff();
+          if (e < p.ke) o[e] = a[e] ? (int32_t)(f * p.P + ckey_index(a[e])) : -1;
       }
+#pragma unroll
+      for (int e = 0; e < K; ++e) a[e] = 0;
+      tau = -__builtin_inff();
+      ++f;
     }
-    if (++u == tiles_pf) {
-      u = 0;
-      if (ps) ++f;
-      ps ^= 1;
-    }
+    u = 0;
+    ps ^= 1;
   };
 
   wait_vm<0>();  // q fragments landed; from here vmcnt counts ring loads only
@@ -307,12 +339,8 @@ __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkPar
   int rst = 0;  // stage of step t
   for (int t = 0; t <= total; ++t) {
     bf16x8 ka[4], kbf[4];
-    if (t < total) {
-      wait_vm<2 * (kStages - 2)>();  // tile t landed: only the loads of step t + 1 are pending
-      barrier_only();                // every wave's share of tile t is in LDS; every wave is done with tile t-1
-      issue(t + kStages - 1);
-      const char* kb = ring[rst];
-      rst = rst == kStages - 1 ? 0 : rst + 1;
+    const char* kb = ring[0];
+    auto read_k = [&]() __attribute__((always_inline)) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int chn = 4 * half + s;
@@ -320,10 +348,22 @@ __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkPar
         ka[s] = *reinterpret_cast<const bf16x8*>(&kb[r0 * 128 + ((chn ^ swz8(r0)) << 4)]);
         kbf[s] = *reinterpret_cast<const bf16x8*>(&kb[r1 * 128 + ((chn ^ swz8(r1)) << 4)]);
       }
+    };
+    if (t < total) {
+      wait_vm<2 * (kStages - 2)>();  // tile t landed: only the loads of step t + 1 are pending
+      barrier_only();                // every wave's share of tile t is in LDS; every wave is done with tile t-1
+      issue(t + kStages - 1);
+      kb = ring[rst];
+      rst = rst == kStages - 1 ? 0 : rst + 1;
+      read_k();
     }
     if (t > 0) {
       if (64 * u + 64 > p.P) select(std::true_type{}, s0, s1);
       else select(std::false_type{}, s0, s1);
+      if (++u == tiles_pf) {
+        pass_end();
+        if (t < total) read_k();  // read again rather than held in 32 registers meanwhile
+      }
     }
     if (t < total) {
       // S^T = K . Q^T over the staged tile: keys 0..31 in s0, 32..63 in s1
@@ -339,18 +379,23 @@ __global__ __launch_bounds__(256, K <= 8 ? 3 : 2) void token_topk_kernel(TopkPar
   wait_vm<0>();  // the trailing loads into unread stages land before the work-group's LDS is released
 }
 
-// Frame groups: every work-group walks all frames of its queries, so with few, long work-groups the
-// launch ends with a partly idle last round. The frames split into g groups (one work-group per
-// query block and group): the largest g of at most 16, with at least `least` frames a group, whose
-// rounds of resident work-groups (`per_cu` per CU) are within 2% of the fullest (at 128 frames x
-// 1369 tokens, top-4: g = 16, 10.5 ms against 10.9 with g = 5 and 13.2 with one group).
-static int frame_groups(int64_t nb, int frames, int per_cu, int least) {
+static int gpu_cus() {
   int cus = 0, dev = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
     cus = 256;
-  const int64_t slots = (int64_t)cus * per_cu;
-  const int gmax = std::max(1, std::min(16, frames / least));
+  return cus;
+}
+
+// Frame groups: every work-group walks all frames of its queries, so with few, long work-groups the
+// launch ends with a partly idle last round. The frames split into g groups (one work-group per
+// query block and group): the largest g of at most 16 whose rounds of resident work-groups (`per_cu`
+// per CU) are within 2% of the fullest (at 128 frames x 1369 tokens, top-4: g = 16, 10.5 ms against
+// 10.9 with g = 5 and 13.2 with one group). Groups of single frames are allowed: with at least 8
+// frames a group, 16 x 1036 tokens took 735 us against 257, 4 x 1036 413 against 107.
+static int frame_groups(int64_t nb, int frames, int per_cu) {
+  const int64_t slots = (int64_t)gpu_cus() * per_cu;
+  const int gmax = std::max(1, std::min(16, frames));
   auto eff = [&](int g) {
     const int64_t wgs = nb * g, rounds = (wgs + slots - 1) / slots;
     return (double)wgs / (double)(rounds * slots);
@@ -362,13 +407,13 @@ static int frame_groups(int64_t nb, int frames, int per_cu, int least) {
   return 1;
 }
 
-template <int K>
+template <int K, int G>
 static int launch_topk(TopkParams p, hipStream_t st) {
   const int64_t nb = (p.nq + 127) / 128;
-  p.fgroups = frame_groups(nb, p.F, K <= 8 ? 3 : 2, 8);
+  p.fgroups = frame_groups(nb, p.F, K <= 8 ? 3 : 2);
   const dim3 grid((unsigned)nb, (unsigned)p.fgroups);
-  if (p.kmode == 2) hipLaunchKernelGGL((token_topk_kernel<K, false>), grid, dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((token_topk_kernel<K, true>), grid, dim3(256), 0, st, p);
+  if (p.kmode == 2) hipLaunchKernelGGL((token_topk_kernel<K, G, false>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((token_topk_kernel<K, G, true>), grid, dim3(256), 0, st, p);
   return check_launch("saf3r_token_topk");
 }
 
@@ -459,9 +504,6 @@ __device__ __forceinline__ void lane_sort128(T& x, T& y, int n, bool both, int l
 __device__ __forceinline__ int lanes_before(uint64_t m, int base) {
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)base));
 }
-// the float bits of a sortable key
-__device__ __forceinline__ uint32_t fkey_bits(uint32_t k) { return k ^ (~(uint32_t)((int32_t)k >> 31) | 0x80000000u); }
-
 // A work-group owns QR queries (16, or 8 of the 16 matrix columns for long frames) and walks the
 // frames of its group. Per frame: the waves share out the frame's 16-key tiles, score them on the
 // matrix core (v_mfma_f32_16x16x32_bf16, S^T = K . Q^T) and put the fp32 scores into LDS rows,
@@ -712,18 +754,12 @@ static void launch_rows(const TopkParams& p, dim3 grid, hipStream_t st) {
   hipLaunchKernelGGL((topk_rows_kernel<NV, FLAT>), grid, dim3(64 * kRowWaves), 0, st, p);
 }
 
-// Top-k of LDS score rows. The caller's workspace is checked as the ABI states and not used.
-static int token_topk_large(TopkParams p, const void* workspace, int64_t workspace_bytes, hipStream_t st) {
-  const int64_t row_bytes = large_row_bytes(p.F, p.P);
-  if (!workspace || workspace_bytes / row_bytes / 128 * 128 < 128)
-    return fail(SAF3R_ERR_INVALID,
-                "saf3r_token_topk: min(topk, per_frame) > 16 needs a workspace of at least %lld bytes "
-                "(saf3r_token_topk_workspace_bytes), got %lld",
-                (long long)(128 * row_bytes), (long long)(workspace ? workspace_bytes : 0));
+// Top-k of LDS score rows.
+static int launch_topk_rows(TopkParams p, hipStream_t st) {
   const int nv = (p.P + 63) / 64;
   const int qr = nv <= 24 ? 16 : 8;
   const int64_t nb = ((int64_t)p.nq + qr - 1) / qr;
-  p.fgroups = frame_groups(nb, p.F, 1, 2);
+  p.fgroups = frame_groups(nb, p.F, 1);
   const dim3 grid((unsigned)nb, (unsigned)p.fgroups);
   if (p.kmode == 2) {  // the general row map: four lengths
     if (nv <= 8) launch_rows<8, false>(p, grid, st);
@@ -745,6 +781,20 @@ static int token_topk_large(TopkParams p, const void* workspace, int64_t workspa
   else if (nv <= 48) launch_rows<48>(p, grid, st);
   else launch_rows<64>(p, grid, st);
   return check_launch("saf3r_token_topk");
+}
+
+// Whether a top-k of at most 16 takes the LDS rows. They start a work-group per 16 queries and frame
+// group and need no second pass, so small launches end sooner; the two-pass kernel does less work
+// per key and wins once it fills the chip. Measured in rounds of 16 queries x 1 frame per CU (us,
+// rows / two passes): top-4 2 x 1036 tokens (1 round) 15 / 29, 3 x 1036 (2.3) 21 / 29, 4 x 1036 (4)
+// 40 / 29, 3 x 1369 (3) 47 / 36; top-8 3 x 1036 21 / 35, 4 x 1036 41 / 35; top-16 5 x 1036 (6.3)
+// 54 / 57, 5 x 1369 (8.4) 81 / 73, 16 x 1036 418 / 274. Short frames leave the two-pass bound of a
+// top-16 weak (64 groups of P / 64 keys): 16 x 256 42 / 79, 64 x 256 553 / 1050.
+static bool topk_takes_rows(const TopkParams& p) {
+  if (p.kmode == 2 || p.P > 1536) return false;
+  if (p.ke > 8 && p.P <= 512) return true;
+  const int64_t tasks = ((int64_t)p.nq + 15) / 16 * p.F;
+  return tasks <= (int64_t)gpu_cus() * (p.ke <= 4 ? 2 : p.ke <= 8 ? 3 : 6);
 }
 
 }  // namespace saf3r
@@ -802,10 +852,21 @@ extern "C" int saf3r_token_topk(const saf3r_rows* q, const saf3r_rows* k, int n_
   p.idx = idx;
   p.fgroups = 1;
   hipStream_t st = (hipStream_t)stream;
-  if (ke > 16) return token_topk_large(p, workspace, workspace_bytes, st);
-  if (p.ke <= 1) return launch_topk<1>(p, st);
-  if (p.ke <= 2) return launch_topk<2>(p, st);
-  if (p.ke <= 4) return launch_topk<4>(p, st);
-  if (p.ke <= 8) return launch_topk<8>(p, st);
-  return launch_topk<16>(p, st);
+  if (ke > 16) {  // the workspace is checked as the ABI states and not used
+    const int64_t row_bytes = large_row_bytes(p.F, p.P);
+    if (!workspace || workspace_bytes / row_bytes < 128)
+      return fail(SAF3R_ERR_INVALID,
+                  "saf3r_token_topk: min(topk, per_frame) > 16 needs a workspace of at least %lld bytes "
+                  "(saf3r_token_topk_workspace_bytes), got %lld",
+                  (long long)(128 * row_bytes), (long long)(workspace ? workspace_bytes : 0));
+    return launch_topk_rows(p, st);
+  }
+  if (topk_takes_rows(p)) return launch_topk_rows(p, st);
+  if (p.ke <= 1) return launch_topk<1, 8>(p, st);
+  if (p.ke <= 2) return launch_topk<2, 8>(p, st);
+  // short frames: 16 groups of a lane (64 x 256 tokens, top-4: 149 us against 245 with 8), whose
+  // registers cost long ones 5% (128 x 1369: 9.68 ms against 9.21)
+  if (p.ke <= 4) return p.P <= 512 ? launch_topk<4, 16>(p, st) : launch_topk<4, 8>(p, st);
+  if (p.ke <= 8) return launch_topk<8, 16>(p, st);
+  return launch_topk<16, 32>(p, st);
 }

@@ -84,3 +84,28 @@ def test_rows_general_row_map(ops):
         kr = ops.rows(store.view(-1, 64), base_row=pad, rows_per_frame=2 * P, frame_row_stride=pad + 2 * P)
         got = ops.token_topk(q.to(DEV), None, frames, P, topk, krows=kr).cpu().numpy()
         assert np.array_equal(got, OS.frame_topk((q.double() @ k.double().T).float().numpy(), frames, topk))
+
+
+@pytest.mark.parametrize("P", [40, 64, 100, 256, 627])
+@pytest.mark.parametrize("topk", [1, 2, 4, 8, 16])
+def test_two_pass_exact(ops, P, topk):
+    """k <= 16 with enough queries and frames for the two-pass kernel (and, for k > 8 on short frames, the
+    rows), the last work-group partly filled; integer scores with many ties: the buffers of its second pass
+    overflow and frames are scanned again."""
+    g = torch.Generator().manual_seed(7 * P + topk)
+    frames, nq = 14, 2005
+    q = torch.randint(-2, 3, (nq, 64), generator=g).float()
+    k = torch.randint(-2, 3, (frames * P, 64), generator=g).float()
+    _check(ops, q, k, frames, P, topk)
+    k[:, 8:] = 0.0  # a few dozen distinct scores
+    _check(ops, q, k, frames, P, topk)
+
+
+@pytest.mark.parametrize("topk", [3, 7, 16])
+def test_small_launches_take_rows(ops, topk):
+    """k <= 16 below the line between the two kernels, and just above it with the same inputs."""
+    g = torch.Generator().manual_seed(topk)
+    for frames, nq, P in ((1, 1, 20), (2, 500, 1036), (7, 1200, 130), (14, 1200, 130)):
+        q = torch.randint(-4, 5, (nq, 64), generator=g).float()
+        k = torch.randint(-4, 5, (frames * P, 64), generator=g).float()
+        _check(ops, q, k, frames, P, topk)
