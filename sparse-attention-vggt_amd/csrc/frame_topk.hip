@@ -7,16 +7,21 @@
 // Scores are bf16 bit patterns; a key is ranked by the score, ties go to the lower key index. The
 // 16-bit order key of a score is its sortable transform (larger score -> larger key, -0 < +0).
 //   frame stage: one wave per (row, frame) holds the frame's scores in registers, finds the k-th
-//                largest order key by bisection with wave-wide counts, and writes the k keys in
-//                increasing key order;
+//                largest order key with wave-wide counts, and writes the k keys in increasing key order;
 //   cap stage:   one work-group per row takes the best `cap` of a candidate list (the frame stage's
 //                output, or every key of the row when selection is not per frame) the same way,
 //                in list order, which is increasing key order.
+#include <cmath>
+#include <type_traits>
+
 #include "common.h"
 
 namespace saf3r {
 
-constexpr int kMaxPerFrame = 4096;  // frame stage: at most 9 chunks of 8 keys per lane
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kMaxPerFrame = 4096;  // frame stage: at most 33 words of two keys per lane
 
 struct FrameTopkParams {
   const uint16_t* scores;
@@ -26,6 +31,7 @@ struct FrameTopkParams {
   int32_t* out;       // frame stage output (idx or candidate list)
   int64_t ors;        // its row stride
   int ocol;           // first column written
+  int lanes;          // lane maxima the first threshold guess aims at
   uint16_t* okey;     // candidate order keys (cap stage input), row stride ors, or null
 };
 
@@ -86,226 +92,214 @@ __device__ inline int radix_bin(uint32_t* counts, int need, int* above, int lane
   return b;
 }
 
-// Wave-wide exclusive prefix of a small per-lane count (0..15) and the wave total, from four
-// ballots of its bits.
-__device__ inline int wave_prefix4(int cnt, int* total) {
-  int pre = 0, tot = 0;
-#pragma unroll
-  for (int bit = 0; bit < 4; ++bit) {
-    const uint64_t m = __ballot((cnt >> bit) & 1);
-    pre += (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0)) << bit;
-    tot += __popcll(m) << bit;
-  }
-  *total = tot;
-  return pre;
+// base + the set lanes of m below this one
+__device__ __forceinline__ int lanes_before(uint64_t m, int base) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)base));
+}
+
+// x over the wave by DPP within rows of 16 lanes and the row / half swaps, as a wave-uniform value
+template <typename Op>
+__device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t x, Op op) {
+  auto mov = [](uint32_t y, auto ctl) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)y, decltype(ctl)::value, 0xF, 0xF, true);
+  };
+  x = op(x, mov(x, std::integral_constant<int, 0xB1>{}));   // quad_perm [1, 0, 3, 2]
+  x = op(x, mov(x, std::integral_constant<int, 0x4E>{}));   // quad_perm [2, 3, 0, 1]
+  x = op(x, mov(x, std::integral_constant<int, 0x141>{}));  // mirror of 8
+  x = op(x, mov(x, std::integral_constant<int, 0x128>{}));  // rotation by 8 of 16
+  const auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  x = op((uint32_t)a[0], (uint32_t)a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)op((uint32_t)b[0], (uint32_t)b[1]));
 }
 
 // ---- frame stage: four waves, one (row, frame) each ----
-// A lane holds RC 16-byte chunks (8 scores each) of its frame: chunk c = lane + 64 r of the frame's
-// aligned span, so element order (r, lane, e) is increasing key order. The threshold t (the k-th
-// largest order key) is found by bisection over the 16-bit key range with wave-wide counts.
-template <int RC>
+// A lane holds NR words of two scores: word lane + 64 r of the frame's span, so element order (r,
+// lane, half) is increasing key order. Words up to NF are whole (the caller picks NR by the frame's
+// length); positions outside the frame hold order key 0, which no threshold of the search counts
+// (its thresholds are >= 1; a real key 0, the lowest, only matters at threshold 0).
+//   1. A threshold with k .. kCands keys at or above it: a first guess from the lanes' largest keys
+//      (one compare and ballot per bisection step), then counts of all keys until one falls into
+//      the window, mostly one or two. A count is one compare per key (the upper half of a word
+//      compares as the word) and scalar adds.
+//   2. Those candidates, (order key, position) in one word, into LDS in key order, two per lane.
+//   3. The exact k-th key by bisection over the candidates, and the k kept ones written out in key
+//      order, equal keys lowest first.
+// A row whose counts jump over the window (many equal scores), or k > kCands, bisects over all its
+// keys instead. Bound by VALU issue (the loads alone would take half the time): about 260 instructions per row
+// and frame of 1036 keys at k = 64. It replaced one bisection over unpacked keys (24 registers for
+// 1036 keys, 9 rounds of two instructions per key) for k > 8, and per-lane sorted lists with a
+// butterfly merge for k <= 8: 4096 rows x 32 frames x 1036 keys,
+// top-64 279 -> 97 us, top-4 111 -> 90 us; 128 x 1369 keys 1070 -> 392 and 475 -> 364 us (3.9 TB/s).
+constexpr int kCands = 128;
+template <int NR, int NF>
 __global__ __launch_bounds__(256) void frame_select_kernel(FrameTopkParams p) {
-  const int lane = tid_x() & 63, w = tid_x() >> 6;
+  __shared__ uint32_t cands[4][kCands];
+  const int lane = tid_x() & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid_x() >> 6);
   const int row = bid_y();
   const int nfr = p.F - p.f0;
   const int fs = bid_x() * 4 + w;  // selected-frame index
-  if (fs >= nfr) return;              // whole wave: no barrier below
-  const int f = p.f0 + fs;
-  const int64_t s0 = (int64_t)f * p.P;        // first key of the frame in the row
-  const int64_t a0 = s0 & ~(int64_t)7;        // aligned span start
-  const uint16_t* rowp = p.scores + (int64_t)row * p.srs;
-  // order keys of the frame's scores; slots outside the frame hold 0, which no threshold of the
-  // search counts (its thresholds are >= 1; a real key 0, the lowest, only matters at t = 0)
-  uint32_t key[RC][8];
-  const int lo_e = (int)(s0 - a0);  // valid slot positions: lo_e <= 8 (lane + 64 r) + e < lo_e + P
-  auto valid = [&](int r, int e) {
-    const uint32_t pos = (uint32_t)(8 * (lane + 64 * r) + e - lo_e);
-    return pos < (uint32_t)p.P;
-  };
-  int nv = 0;
+  if (fs >= nfr) return;              // whole wave: no work-group barrier below
+  const int64_t s0 = (int64_t)(p.f0 + fs) * p.P;  // first key of the frame in the row
+  const int off = (int)(s0 & 1);                  // the span starts at the word of key s0
+  const uint32_t* words = reinterpret_cast<const uint32_t*>(p.scores + (int64_t)row * p.srs + (s0 - off));
+  const int last = (off + p.P - 1) >> 1;          // last word with a key of the frame
+  const int k = p.k;
+  uint32_t key[NR];  // order keys: larger score -> larger key
 #pragma unroll
-  for (int r = 0; r < RC; ++r) {
-    const int64_t e0 = a0 + 8 * (int64_t)(lane + 64 * r);
-    u32x4 v = {0, 0, 0, 0};
-    if (e0 < s0 + p.P) v = *reinterpret_cast<const u32x4*>(rowp + e0);
+  for (int r = 0; r < NR; ++r) key[r] = words[r < NF ? lane + 64 * r : min(lane + 64 * r, last)];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint16_t b = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
-      const bool in = valid(r, e);
-      key[r][e] = in ? sortable16(b) : 0u;
-      nv += in ? 1 : 0;
+  for (int r = 0; r < NR; ++r) {
+    if (r >= NF - 1) {
+      if (lane + 64 * r > last) key[r] = 0xFFFFFFFFu;  // bits 0xFFFF: order key 0
+      if (lane + 64 * r == last && ((off + p.P) & 1)) key[r] |= 0xFFFF0000u;
     }
+    if (r == 0 && off && lane == 0) key[0] |= 0xFFFFu;
+    const s16x2 b = __builtin_bit_cast(s16x2, key[r]);
+    key[r] ^= __builtin_bit_cast(uint32_t, b >> (short)15) | 0x80008000u;
   }
-  auto count_ge = [&](uint32_t t) {  // keys >= t (t >= 1), wave-wide
+  auto count_ge = [&](uint32_t t) {  // keys >= t (1 <= t <= 0xFFFF), wave-wide
     int c = 0;
 #pragma unroll
-    for (int r = 0; r < RC; ++r)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) c += key[r][e] >= t ? 1 : 0;
-    // per-lane counts summed by ballots of their bits (c <= 8 * RC <= 72)
-    int sum = 0;
-#pragma unroll
-    for (int bit = 0; bit < 7; ++bit) sum += __popcll(__ballot((c >> bit) & 1)) << bit;
-    return sum;
+    for (int r = 0; r < NR; ++r) {
+      c += __popcll(__builtin_amdgcn_ballot_w64((uint16_t)key[r] >= (uint16_t)t));
+      c += __popcll(__builtin_amdgcn_ballot_w64(key[r] >= (t << 16)));
+    }
+    return c;
   };
-  const int k = p.k;
-  // Bracket for the bisection: t is at most the largest key, and for k <= 64 at least the k-th
-  // largest of the lanes' largest keys (k distinct keys reach it), found by a bisection over one
-  // value per lane (a compare and a ballot per step).
-  uint32_t lmax = 0;
-#pragma unroll
-  for (int r = 0; r < RC; ++r)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) lmax = max(lmax, key[r][e]);
-  uint32_t hi = lmax;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) hi = max(hi, (uint32_t)__shfl_xor((int)hi, o));
-  uint32_t lo = 0;  // count(key >= lo) >= k holds for lo = 0
-  const bool any = nv > 0;
-  if (k <= 64 && __popcll(__ballot(any)) >= k) {
-    uint32_t a = 0, b = hi;  // count(lane maxima >= a) >= k
-    while (a < b) {
-      const uint32_t mid = (a + b + 1) >> 1;
-      if (__popcll(__ballot(any && lmax >= mid)) >= k) a = mid;
-      else b = mid - 1;
-    }
-    lo = a;
-  }
-  int c_above = 0;  // count(key >= hi + 1): 0 for the largest key, then the count of the last miss
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi + 1) >> 1;
-    const int c = count_ge(mid);
-    if (c >= k) {
-      lo = mid;
-    } else {
-      hi = mid - 1;
-      c_above = c;
-    }
-  }
-  const uint32_t t = lo;
-  const int need_eq = k - c_above;  // keys equal to t to keep, lowest first
   int32_t* o = p.out + (int64_t)row * p.ors + p.ocol + (int64_t)fs * k;
   uint16_t* ok = p.okey ? p.okey + (int64_t)row * p.ors + (int64_t)fs * k : nullptr;
-  int base = 0, eq_seen = 0;
+  u16x2 mx = __builtin_bit_cast(u16x2, key[0]);
 #pragma unroll
-  for (int r = 0; r < RC; ++r) {
-    int neq = 0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) neq += (valid(r, e) && key[r][e] == t) ? 1 : 0;
-    int eq_tot;
-    const int eq_pre = eq_seen + wave_prefix4(neq, &eq_tot);
-    int nsel = 0, eq_run = 0;
-    bool sel[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const bool in = valid(r, e);
-      const bool eq = in && key[r][e] == t;
-      sel[e] = in && (key[r][e] > t || (eq && eq_pre + eq_run < need_eq));
-      eq_run += eq ? 1 : 0;
-      nsel += sel[e] ? 1 : 0;
+  for (int r = 1; r < NR; ++r) mx = __builtin_elementwise_max(mx, __builtin_bit_cast(u16x2, key[r]));
+  const uint32_t lmax = max((uint32_t)mx[0], (uint32_t)mx[1]);
+  const uint32_t top = wave_reduce_u32(lmax, [](uint32_t a, uint32_t b) { return max(a, b); });
+  uint32_t t = 1;
+  int n = -1;
+  if (k <= kCands) {
+    if (p.P > kCands) {
+      uint32_t a = 1, b = top;
+      t = wave_reduce_u32(lmax, [](uint32_t x, uint32_t y) { return min(x, y); });
+      if (k <= 64) a = max(t, 1u);  // every lane's largest key reaches it
+      t = (a + b + 1) >> 1;
+      for (uint32_t x = a, y = b; x < y;) {
+        const int c = __popcll(__builtin_amdgcn_ballot_w64(lmax >= t));
+        if (c > p.lanes + 2) x = t;
+        else if (c < p.lanes - 2) y = t - 1;
+        else break;
+        t = (x + y + 1) >> 1;
+      }
+      // count(a) >= k unless a = 1; stops with a = b where the counts jump over the window
+      for (;;) {
+        const int c = count_ge(t);
+        if (c >= k && c <= kCands) {
+          n = c;
+          break;
+        }
+        if (c < k) b = t - 1;
+        else a = t;
+        if (a >= b) {  // the one threshold left
+          const int ca = a == t ? c : count_ge(a);
+          if (ca >= k && ca <= kCands) {
+            n = ca;
+            t = a;
+          }
+          break;
+        }
+        t = (a + b + 1) >> 1;
+      }
+    } else {
+      n = count_ge(1);
+      if (n < k) n = -1;  // the k-th key is the lowest order key, which counts leave out
     }
-    int sel_tot;
-    int pos = base + wave_prefix4(nsel, &sel_tot);
-    const int64_t e0 = a0 + 8 * (int64_t)(lane + 64 * r);
+  }
+  if (n >= 0) {
+    uint32_t* cw = cands[w];
+    const int j0 = 2 * lane - off;
+    int base = 0;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      if (sel[e]) {
-        o[pos] = (int32_t)(e0 + e);
-        if (ok) ok[pos] = (uint16_t)key[r][e];
-        ++pos;
+    for (int r = 0; r < NR; ++r) {
+      const bool h0 = (uint16_t)key[r] >= (uint16_t)t, h1 = key[r] >= (t << 16);
+      const uint64_t m0 = __builtin_amdgcn_ballot_w64(h0), m1 = __builtin_amdgcn_ballot_w64(h1);
+      const int at = lanes_before(m1, lanes_before(m0, base));
+      if (h0) cw[at] = (key[r] << 16) | (uint32_t)(j0 + 128 * r);
+      if (h1) cw[at + (h0 ? 1 : 0)] = (key[r] & 0xFFFF0000u) | (uint32_t)(j0 + 128 * r + 1);
+      base += __popcll(m0) + __popcll(m1);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t x0 = lane < n ? cw[lane] : 0u, x1 = 64 + lane < n ? cw[64 + lane] : 0u;
+    uint32_t lo = t, hi = top;  // count(lo) >= k
+    int above = 0;                // keys above hi
+    int c_lo = n;
+    while (lo < hi && c_lo != k) {
+      const uint32_t mid = (lo + hi + 1) >> 1;
+      const int c = __popcll(__builtin_amdgcn_ballot_w64(x0 >= (mid << 16))) +
+                    __popcll(__builtin_amdgcn_ballot_w64(x1 >= (mid << 16)));
+      if (c >= k) {
+        lo = mid;
+        c_lo = c;
+      } else {
+        hi = mid - 1;
+        above = c;
       }
     }
-    base += sel_tot;
-    eq_seen += eq_tot;
-  }
-}
-
-// ---- frame stage for k <= 8: running per-lane top-K lists merged across the wave ----
-// (larger k take the bisection above: at k = 16 over 128 frames of 1369 keys, 4096 rows, 1.23 ms
-// with lists of 16 against about 1 ms)
-constexpr int kSmallMaxK = 8;
-// Composite key (order key << 16 | 0xFFFF - j) of key j of the frame: larger is better, equal
-// scores order by the lower j. Each lane keeps the K best of its keys, a butterfly over the wave
-// merges the lists (bitonic merge of two descending lists), and the K winners are written in
-// increasing key order.
-template <int K>
-__device__ inline void cas_desc(uint32_t (&c)[K], int i, int j) {
-  const uint32_t hi = max(c[i], c[j]), lo = min(c[i], c[j]);
-  c[i] = hi;
-  c[j] = lo;
-}
-
-template <int K>
-__device__ inline void sort_bitonic_desc(uint32_t (&c)[K]) {
-  // c is bitonic: half-cleaners of sizes K, K/2, ..., 2 sort it descending
+    // every candidate at or above lo, except the last of those equal to it where they are too many
+    // (then the search ended with lo = hi, so that `above` counts the keys above lo)
+    int skip_from = c_lo == k ? 0x7FFFFFFF : k - above;  // rank among the equal ones from which they drop out
+    int out_base = 0;
 #pragma unroll
-  for (int len = K; len >= 2; len >>= 1)
-#pragma unroll
-    for (int i = 0; i < K; ++i)
-      if ((i % len) < len / 2) cas_desc<K>(c, i, i + len / 2);
-}
-
-template <int RC, int K>
-__global__ __launch_bounds__(256) void frame_select_small_kernel(FrameTopkParams p) {
-  const int lane = tid_x() & 63, w = tid_x() >> 6;
-  const int row = bid_y();
-  const int nfr = p.F - p.f0;
-  const int fs = bid_x() * 4 + w;
-  if (fs >= nfr) return;
-  const int f = p.f0 + fs;
-  const int64_t s0 = (int64_t)f * p.P;
-  const int64_t a0 = s0 & ~(int64_t)7;
-  const uint16_t* rowp = p.scores + (int64_t)row * p.srs;
-  uint32_t c[K];
-#pragma unroll
-  for (int i = 0; i < K; ++i) c[i] = 0;  // 0 ranks below every key (j < 0xFFFF keeps the low half > 0)
-  const int lo_e = (int)(s0 - a0);  // slot 8 (lane + 64 r) + e holds key (that - lo_e) of the frame
-#pragma unroll
-  for (int r = 0; r < RC; ++r) {
-    const int64_t e0 = a0 + 8 * (int64_t)(lane + 64 * r);
-    u32x4 v = {0, 0, 0, 0};
-    if (e0 < s0 + p.P) v = *reinterpret_cast<const u32x4*>(rowp + e0);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t j = (uint32_t)(8 * (lane + 64 * r) + e - lo_e);  // key of the frame (or out of it)
-      const uint16_t b = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
-      // keys outside the frame: 0, which ranks below every key (its low half is never 0xFFFF - j)
-      const uint32_t y = j < (uint32_t)p.P ? (sortable16(b) << 16) | (0xFFFFu - j) : 0u;
-      // insertion into the descending list: every new slot from the old list (independent steps)
-#pragma unroll
-      for (int i = K - 1; i > 0; --i) c[i] = max(c[i], min(c[i - 1], y));
-      c[0] = max(c[0], y);
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t x = h ? x1 : x0;
+      bool take = x >= (lo << 16);
+      const uint64_t meq = __builtin_amdgcn_ballot_w64(take && (x >> 16) == lo);
+      take = take && ((x >> 16) != lo || lanes_before(meq, 0) < skip_from);
+      if (skip_from != 0x7FFFFFFF) skip_from -= (int)__popcll(meq);
+      const uint64_t mt = __builtin_amdgcn_ballot_w64(take);
+      const int at = lanes_before(mt, out_base);
+      if (take) {
+        o[at] = (int32_t)(s0 + (x & 0xFFFFu));
+        if (ok) ok[at] = (uint16_t)(x >> 16);
+      }
+      out_base += __popcll(mt);
     }
+    return;
   }
-  // butterfly merge: after step d every lane holds the best K of its 2^d-lane group
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    uint32_t o[K];
-#pragma unroll
-    for (int i = 0; i < K; ++i) o[i] = (uint32_t)__shfl_xor((int)c[i], d, 64);
-#pragma unroll
-    for (int i = 0; i < K; ++i) c[i] = max(c[i], o[K - 1 - i]);
-    sort_bitonic_desc<K>(c);
+  // the exact threshold over all keys: the largest t with at least k keys at or above it
+  uint32_t thr = 0;
+#pragma unroll 1
+  for (int bit = 15; bit >= 0; --bit) {
+    const uint32_t c = thr | (1u << bit);
+    if (count_ge(c) >= k) thr = c;
   }
-  // the k winners (k <= K), in increasing key order: reversed order of the low halves
-  const int k = p.k;
-  int32_t* out = p.out + (int64_t)row * p.ors + p.ocol + (int64_t)fs * k;
-  uint16_t* ok = p.okey ? p.okey + (int64_t)row * p.ors + (int64_t)fs * k : nullptr;
-  if (lane < k) {
-    // rank of winner `lane` by key index among the k winners
-    uint32_t mine = 0;
-    int jm = 0;
+  int need = k - (thr < 0xFFFFu ? count_ge(thr + 1) : 0);  // keys equal to thr to keep, lowest first
+  int base = 0;
+  int ln = lane;
+  asm volatile("" : "+v"(ln));  // positions formed here, not held through the search
 #pragma unroll
-    for (int i = 0; i < K; ++i)
-      if (i == lane) mine = c[i];
-    jm = 0xFFFF - (int)(mine & 0xFFFFu);
-    int rank = 0;
-#pragma unroll
-    for (int i = 0; i < K; ++i)
-      if (i < k) rank += (0xFFFF - (int)(c[i] & 0xFFFFu)) < jm ? 1 : 0;
-    out[rank] = (int32_t)(s0 + jm);
-    if (ok) ok[rank] = (uint16_t)(mine >> 16);
+  for (int r = 0; r < NR; ++r) {
+    const int j = 2 * (ln + 64 * r) - off;  // position of the lower half
+    const uint32_t k0 = key[r] & 0xFFFFu, k1 = key[r] >> 16;
+    const bool in0 = (uint32_t)j < (uint32_t)p.P, in1 = (uint32_t)(j + 1) < (uint32_t)p.P;
+    const bool e0 = in0 && k0 == thr, e1 = in1 && k1 == thr;
+    const uint64_t me0 = __builtin_amdgcn_ballot_w64(e0), me1 = __builtin_amdgcn_ballot_w64(e1);
+    const int rank = lanes_before(me1, lanes_before(me0, 0));
+    const bool t0 = k0 > thr || (e0 && rank < need);
+    const bool t1 = k1 > thr || (e1 && rank + (e0 ? 1 : 0) < need);
+    const uint64_t m0 = __builtin_amdgcn_ballot_w64(t0), m1 = __builtin_amdgcn_ballot_w64(t1);
+    const int at = lanes_before(m1, lanes_before(m0, base));
+    if (t0) {
+      o[at] = (int32_t)(s0 + j);
+      if (ok) ok[at] = (uint16_t)k0;
+    }
+    if (t1) {
+      o[at + (t0 ? 1 : 0)] = (int32_t)(s0 + j + 1);
+      if (ok) ok[at + (t0 ? 1 : 0)] = (uint16_t)k1;
+    }
+    base += __popcll(m0) + __popcll(m1);
+    need -= (int)(__popcll(me0) + __popcll(me1));
   }
 }
 
@@ -445,21 +439,22 @@ extern "C" int saf3r_frame_topk_scores(const void* scores, int64_t score_stride,
     p.ocol = capped ? 0 : fsel;
     p.okey = capped ? cand_key : nullptr;
     const dim3 grid((nfr + 3) / 4, rows);
-    const int RC = (per_frame / 8 + 2 + 63) / 64;  // 16-byte chunks per lane
-#define SAF3R_SMALL(RCV)                                                                                  \
-  if (k <= 4) hipLaunchKernelGGL((frame_select_small_kernel<RCV, 4>), grid, dim3(256), 0, st, p);           \
-  else hipLaunchKernelGGL((frame_select_small_kernel<RCV, 8>), grid, dim3(256), 0, st, p);
-    if (k <= kSmallMaxK) {
-      if (RC <= 1) { SAF3R_SMALL(1) }
-      else if (RC <= 2) { SAF3R_SMALL(2) }
-      else if (RC <= 3) { SAF3R_SMALL(3) }
-      else if (RC <= 4) { SAF3R_SMALL(4) }
-      else { SAF3R_SMALL(9) }
-    } else if (RC <= 1) hipLaunchKernelGGL(frame_select_kernel<1>, grid, dim3(256), 0, st, p);
-    else if (RC <= 2) hipLaunchKernelGGL(frame_select_kernel<2>, grid, dim3(256), 0, st, p);
-    else if (RC <= 3) hipLaunchKernelGGL(frame_select_kernel<3>, grid, dim3(256), 0, st, p);
-    else if (RC <= 4) hipLaunchKernelGGL(frame_select_kernel<4>, grid, dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(frame_select_kernel<9>, grid, dim3(256), 0, st, p);
+    // m keys at or above a threshold, spread at random, reach 64 (1 - e^(-m / 64)) of the lane
+    // maxima: aim at the middle of the window
+    p.lanes = (int)(64.0 * (1.0 - std::exp(-std::sqrt((double)std::min(k, kCands) * kCands) / 64.0)));
+    const int words = per_frame / 2 + 1;  // of a frame's span, at most
+#define SAF3R_FRAME(NR, NF) hipLaunchKernelGGL((frame_select_kernel<NR, NF>), grid, dim3(256), 0, st, p)
+    if (words <= 64 * 2) SAF3R_FRAME(2, 0);
+    else if (words <= 64 * 3) SAF3R_FRAME(3, 1);
+    else if (words <= 64 * 5) SAF3R_FRAME(5, 2);
+    else if (words <= 64 * 7) SAF3R_FRAME(7, 4);
+    else if (words <= 64 * 9) SAF3R_FRAME(9, 6);
+    else if (words <= 64 * 11) SAF3R_FRAME(11, 8);
+    else if (words <= 64 * 13) SAF3R_FRAME(13, 10);
+    else if (words <= 64 * 17) SAF3R_FRAME(17, 12);
+    else if (words <= 64 * 25) SAF3R_FRAME(25, 16);
+    else SAF3R_FRAME(33, 24);
+#undef SAF3R_FRAME
     if (int e = check_launch("saf3r_frame_topk_scores")) return e;
     if (!capped) return SAF3R_OK;
   }

@@ -741,11 +741,12 @@ def broadcast_gather(qp: torch.Tensor, kp: torch.Tensor, geom: Geometry, heads: 
 
 
 def frame_topk_scores(scores: torch.Tensor, frames: int, per_frame: int, topk: int, per_frame_mode: bool = True,
-                      exclude_first: bool = False, first_stride: int = 1, cap: int = 0) -> torch.Tensor:
+                      exclude_first: bool = False, first_stride: int = 1, cap: int = 0,
+                      out: torch.Tensor | None = None) -> torch.Tensor:
     """Token top-k of every row of a bf16 score block [rows, frames*per_frame] (``saf3r_frame_topk_scores``):
     int32 [rows, F_sel + kept], F_sel frame-0 samples first when ``exclude_first``, then the kept keys
     (per frame or per row, at most ``cap`` when ``cap`` > 0) in increasing key order. Ties go to the
-    lower key (ref: saf3r/patch/utils.py:54-184)."""
+    lower key (ref: saf3r/patch/utils.py:54-184). ``out`` (optional) receives the result."""
     _need_cuda(scores)
     lib = _lib.load()
     if scores.dtype != torch.bfloat16 or scores.dim() != 2 or scores.stride(1) != 1 or scores.stride(0) % 8:
@@ -761,7 +762,13 @@ def frame_topk_scores(scores: torch.Tensor, frames: int, per_frame: int, topk: i
     else:
         rest = min(topk, nk - f0 * per_frame)
     kept = min(rest, cap) if cap > 0 else rest
-    idx = torch.empty(rows, fsel + kept, dtype=torch.int32, device=scores.device)
+    if out is None:
+        idx = torch.empty(rows, fsel + kept, dtype=torch.int32, device=scores.device)
+    elif (tuple(out.shape) != (rows, fsel + kept) or out.dtype != torch.int32 or out.stride(1) != 1
+          or out.device != scores.device):
+        raise ValueError(f"out must be int32 [{rows}, {fsel + kept}] with unit column stride")
+    else:
+        idx = out
     cand_i = cand_k = None
     if per_frame_mode and kept < rest:
         cand_i = torch.empty(rows, rest, dtype=torch.int32, device=scores.device)
