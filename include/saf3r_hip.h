@@ -168,6 +168,21 @@ int saf3r_pack_qkv(const void* q, const void* k, const void* v, int64_t tok_stri
                    const uint8_t* pool_heads, float* pool_mean, uint16_t* pool_split, float* pool_meta,
                    void* stream);
 
+/* saf3r_pack_qkv with LayerNorm parameters and positions as a module holds them, so that a caller
+ * converts nothing per call: param_flags SAF3R_PACK_LN_BF16 (the four parameter arrays are bf16,
+ * 16-byte aligned; fp32 otherwise), SAF3R_PACK_POS_INT64 (int64 positions, of which the low 32 bits
+ * are read; int32 otherwise). */
+enum saf3r_pack_param_flags { SAF3R_PACK_LN_BF16 = 1, SAF3R_PACK_POS_INT64 = 2 };
+int saf3r_pack_qkv_typed(const void* q, const void* k, const void* v, int64_t tok_stride, int64_t head_stride,
+                   int frames, int tokens_per_frame, int num_special, int num_heads,
+                   const void* q_ln_weight, const void* q_ln_bias, const void* k_ln_weight,
+                   const void* k_ln_bias, float ln_eps, int apply_ln,
+                   const void* pos, const float* rope_cos, const float* rope_sin, int rope_positions,
+                   void* q_packed, void* k_packed, void* v_packed, const uint8_t* token_order,
+                   const uint8_t* fp32_heads, float* qk32, const uint8_t* q_scaled, float q_scale,
+                   const uint8_t* pool_heads, float* pool_mean, uint16_t* pool_split, float* pool_meta,
+                   int param_flags, void* stream);
+
 /*
  * Pooled patch-block means (fp32) of the packed Q and K of the listed heads.
  *   head_ids: host int32 [n_heads_sel]; pooled_q / pooled_k: [n_heads_sel][F*NBf][64].
@@ -263,6 +278,13 @@ int saf3r_probe_scores(const float* q32, const float* k32, int64_t slot_stride, 
                        int n_sel, const int32_t* sample_idx, int n_samples, float scale, float* partial,
                        float* qbar, float* scores, int64_t scores_stride, void* stream);
 
+/* saf3r_probe_scores with `slots` in host memory (at most 64, passed in the kernels' arguments: no copy
+ * to the device, which would wait for the stream) and the score rows they are written to: selected
+ * head i goes to scores + rows[i] * scores_stride (host int32 [n_sel]). */
+int saf3r_probe_scores_host(const float* q32, const float* k32, int64_t slot_stride, int n_tokens, const int32_t* slots, const int32_t* rows,
+                       int n_sel, const int32_t* sample_idx, int n_samples, float scale, float* partial,
+                       float* qbar, float* scores, int64_t scores_stride, void* stream);
+
 /*
  * saf3r_probe_scores without the workspace argument: it allocates nothing (no hipMalloc / hipFree,
  * no allocating library call) and keeps the partial sums in a static device array of the library
@@ -291,6 +313,12 @@ int saf3r_keyset_build(const float* scores, int64_t scores_stride, int n_heads, 
                        int tokens_per_frame, int num_special, int32_t* idx, int64_t idx_stride, int32_t* count,
                        void* stream);
 
+/* saf3r_keyset_build with mode, param, start and include in host memory (at most 64 heads). */
+int saf3r_keyset_build_host(const float* scores, int64_t scores_stride, int n_heads, const int32_t* mode,
+                       const int32_t* param, const int32_t* start, const int32_t* include, int frames,
+                       int tokens_per_frame, int num_special, int32_t* idx, int64_t idx_stride, int32_t* count,
+                       void* stream);
+
 /*
  * Compact K/V of the key sets, in the layout SAF3R_KEYSET heads read: for set s (head head_ids[s]),
  *   keyset_k: bf16 [n_sel][capacity][64], row j = packed K of token idx[s][j];
@@ -301,6 +329,12 @@ int saf3r_keyset_build(const float* scores, int64_t scores_stride, int n_heads, 
  * Replaces: saf3r/patch/sparse_attention.py:181-182, :271-272 (k/v[:, :, idx, :]).
  */
 int saf3r_keyset_gather(const void* k_packed, int frames, int tokens_per_frame, int num_special,
+                        const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
+                        int64_t v_head_stride, const int32_t* idx, int64_t idx_stride, const int32_t* count,
+                        int max_tiles, void* keyset_k, void* keyset_v, int64_t capacity, void* stream);
+
+/* saf3r_keyset_gather with head_ids in host memory (at most 64). */
+int saf3r_keyset_gather_host(const void* k_packed, int frames, int tokens_per_frame, int num_special,
                         const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
                         int64_t v_head_stride, const int32_t* idx, int64_t idx_stride, const int32_t* count,
                         int max_tiles, void* keyset_k, void* keyset_v, int64_t capacity, void* stream);

@@ -19,9 +19,11 @@ EXPORTS = (
     "saf3r_token_topk", "saf3r_probe_scores", "saf3r_keyset_build", "saf3r_keyset_gather",
     "saf3r_frame_topk_scores", "saf3r_probe_scores_noalloc", "saf3r_token_topk_workspace_bytes",
     "saf3r_pooled_prepare", "saf3r_block_select_pooled", "saf3r_block_select_pooled_workspace_bytes",
-    "saf3r_gather_attn_fwd_sliced", "saf3r_gather_attn_workspace_bytes",
+    "saf3r_gather_attn_fwd_sliced", "saf3r_gather_attn_workspace_bytes", "saf3r_pack_qkv_typed",
+    "saf3r_probe_scores_host", "saf3r_keyset_build_host", "saf3r_keyset_gather_host",
 )
 ABI_VERSION = 13
+PACK_LN_BF16, PACK_POS_INT64 = 1, 2  # enum saf3r_pack_param_flags
 GATHER_QK_FP32, GATHER_V_FP32, GATHER_OUT_FP32 = 1, 2, 4  # enum saf3r_gather_dtype
 SAF3R_OK, SAF3R_ERR_INVALID, SAF3R_ERR_UNSUPPORTED, SAF3R_ERR_LAUNCH, SAF3R_ERR_INJECTED = range(5)
 
@@ -62,6 +64,8 @@ def load():
         "saf3r_packed_slots": ([i32, i32, i32], i64),
         "saf3r_pack_qkv": ([p, p, p, i64, i64, i32, i32, i32, i32, p, p, p, p, f32, i32, p, p, p, i32, p, p, p, p, p,
                             p, p, f32, p, p, p, p, p], i32),
+        "saf3r_pack_qkv_typed": ([p, p, p, i64, i64, i32, i32, i32, i32, p, p, p, p, f32, i32, p, p, p, i32, p, p, p, p,
+                                  p, p, p, f32, p, p, p, p, i32, p], i32),
         "saf3r_pooled_prepare": ([p, i64, p, p, p], i32),
         "saf3r_block_select_pooled": ([p, p, p, i32, i32, i32, i32, p, p, i64, p], i32),
         "saf3r_block_select_pooled_workspace_bytes": ([i32, i32, i32, i32], i64),
@@ -79,6 +83,9 @@ def load():
         "saf3r_probe_scores_noalloc": ([p, p, i64, i32, p, i32, p, i32, f32, p, p, i64, p], i32),
         "saf3r_keyset_build": ([p, i64, i32, p, p, p, p, i32, i32, i32, p, i64, p, p], i32),
         "saf3r_keyset_gather": ([p, i32, i32, i32, p, i32, p, i64, i64, p, i64, p, i32, p, p, i64, p], i32),
+        "saf3r_probe_scores_host": ([p, p, i64, i32, p, p, i32, p, i32, f32, p, p, p, i64, p], i32),
+        "saf3r_keyset_build_host": ([p, i64, i32, p, p, p, p, i32, i32, i32, p, i64, p, p], i32),
+        "saf3r_keyset_gather_host": ([p, i32, i32, i32, p, i32, p, i64, i64, p, i64, p, i32, p, p, i64, p], i32),
         "saf3r_frame_topk_scores": ([p, i64, i32, i32, i32, i32, i32, i32, i32, i32, p, i64, p, p, p], i32),
     }
     for name, (args, res) in sig.items():
@@ -97,5 +104,8 @@ def check(rc: int) -> None:
         raise Saf3rError(rc, msg)
 
 
-def stream_ptr(device=None):
+def stream_ptr(device=None) -> ctypes.c_void_p:
+    """Handle of the current stream of ``device`` (default: the current device), without a Stream object."""
+    if device is None:
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)

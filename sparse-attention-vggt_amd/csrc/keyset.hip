@@ -34,6 +34,8 @@ __device__ inline int64_t token_slot(const Geom& g, int64_t t) {
   return (int64_t)g.Sp + f * g.Pp + (r - g.ns);
 }
 
+// Per-head lists come from device arrays, or by value in the kernel's arguments: a caller that holds
+// them on the host then needs no copy to the device, which waits for the stream.
 struct ProbeParams {
   const float* q;  // fp32 q rows of slot s at q + s * slot_stride, token t at + 64 t
   const float* k;  // fp32 k rows, same layout
@@ -43,7 +45,8 @@ struct ProbeParams {
   const int32_t* sample;
   int chunk;
   int nchunks;
-  const int32_t* slots;  // [n_sel] slots of the selected heads
+  const int32_t* slots;  // [n_sel] slots of the selected heads, or null: slot_val
+  int32_t slot_val[kMaxHeads], row_val[kMaxHeads];  // slots and score rows by value (slots null)
   float* partial;        // [n_sel][kProbeChunks][64]
   float* qbar;           // [n_sel][64]
   float* scores;         // [n_sel][scores_stride]
@@ -51,13 +54,15 @@ struct ProbeParams {
   float scale;
 };
 
+__device__ inline int probe_slot(const ProbeParams& p, int hs) { return p.slots ? p.slots[hs] : p.slot_val[hs]; }
+
 // grid (nchunks, n_sel), 64 threads: feature d of chunk c, summed over the chunk's rows in order.
 // Rows are read 64 at a time (independent loads in flight: the chain of adds is cheap, the load
 // latency is not) and added in order, so the sum is the sequential one.
 constexpr int kProbeBatch = 64;
 __global__ __launch_bounds__(64) void probe_partial_kernel(ProbeParams p) {
   const int c = bid_x(), hs = bid_y(), d = tid_x();
-  const float* base = p.q + (int64_t)p.slots[hs] * p.slot_stride + d;
+  const float* base = p.q + (int64_t)probe_slot(p, hs) * p.slot_stride + d;
   const int i0 = c * p.chunk, i1 = min(p.n_samp, i0 + p.chunk);
   float acc = 0.f;
   int i = i0;
@@ -104,7 +109,7 @@ __global__ __launch_bounds__(256) void probe_scores_kernel(ProbeParams p) {
   __syncthreads();
   const int t = bid_x() * 256 + tid_x();
   if (t >= p.n) return;
-  const f32x4* row = reinterpret_cast<const f32x4*>(p.k + (int64_t)p.slots[hs] * p.slot_stride + (int64_t)t * 64);
+  const f32x4* row = reinterpret_cast<const f32x4*>(p.k + (int64_t)probe_slot(p, hs) * p.slot_stride + (int64_t)t * 64);
   float acc = 0.f;
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
@@ -114,16 +119,17 @@ __global__ __launch_bounds__(256) void probe_scores_kernel(ProbeParams p) {
     acc = __builtin_fmaf(qb[4 * j + 2], w[2], acc);
     acc = __builtin_fmaf(qb[4 * j + 3], w[3], acc);
   }
-  p.scores[hs * p.scores_stride + t] = acc * p.scale;
+  p.scores[(p.slots ? hs : p.row_val[hs]) * p.scores_stride + t] = acc * p.scale;
 }
 
 struct BuildParams {
   const float* scores;  // [n_heads][scores_stride] (top-k heads)
   int64_t scores_stride;
-  const int32_t* mode;   // per head: 0 stride, 1 top-k
+  const int32_t* mode;   // per head: 0 stride, 1 top-k (null: every list by value in spec)
   const int32_t* param;  // stride, or k
   const int32_t* start;  // first strided token
   const int32_t* include;
+  int32_t spec[4][kMaxHeads];  // mode, param, start, include
   int n, T, ns;
   int32_t* idx;  // [n_heads][idx_stride]
   int64_t idx_stride;
@@ -142,8 +148,10 @@ __global__ __launch_bounds__(kBuildThreads) void keyset_build_kernel(BuildParams
   __shared__ uint32_t sh_prefix;
   __shared__ int sh_remaining;
   const int hh = bid_x(), tid = tid_x();
-  const int mode = p.mode[hh], param = p.param[hh], start = p.start[hh];
-  const bool include = p.include[hh] != 0;
+  const bool dev = p.mode != nullptr;
+  const int mode = dev ? p.mode[hh] : p.spec[0][hh], param = dev ? p.param[hh] : p.spec[1][hh];
+  const int start = dev ? p.start[hh] : p.spec[2][hh];
+  const bool include = (dev ? p.include[hh] : p.spec[3][hh]) != 0;
   const float* sc = p.scores + (int64_t)hh * p.scores_stride;
 
   // ---- top-k: threshold key by radix select (most significant digit first) ----
@@ -311,7 +319,8 @@ __global__ __launch_bounds__(kBuildThreads) void keyset_build_kernel(BuildParams
 struct GatherKParams {
   const __bf16* k;  // packed K
   Geom g;
-  const int32_t* head_ids;
+  const int32_t* head_ids;  // device array, or null: head_val
+  int32_t head_val[kMaxHeads];
   const __bf16* v;  // natural V rows
   int64_t v_tok_stride, v_head_stride;
   const int32_t* idx;
@@ -329,7 +338,7 @@ __global__ __launch_bounds__(256) void keyset_gather_kernel(GatherKParams p) {
   const int tile = bid_x(), hs = bid_y();
   const int cnt = p.count[hs];
   if (tile * 64 >= cnt) return;
-  const int h = p.head_ids[hs];
+  const int h = p.head_ids ? p.head_ids[hs] : p.head_val[hs];
   const int t = tid_x(), row = t >> 2, c = t & 3;
   const int j = tile * 64 + row;
   const int64_t tok = j < cnt ? p.idx[hs * p.idx_stride + j] : -1;
@@ -376,7 +385,6 @@ __global__ __launch_bounds__(256) void keyset_gather_kernel(GatherKParams p) {
 
 using namespace saf3r;
 
-// Checks the arguments of both probe entries and fills everything but the workspace pointer.
 // Checks the arguments of both probe entries and fills everything but the workspace pointer.
 static int probe_setup(const char* who, const float* q32, const float* k32, int64_t slot_stride, int n_tokens,
                        const int32_t* slots, int n_sel, const int32_t* sample_idx, int n_samples, float scale,
@@ -493,20 +501,46 @@ extern "C" int saf3r_probe_scores_noalloc(const float* q32, const float* k32, in
   return probe_launch(p, n_sel, stream);
 }
 
-extern "C" int saf3r_keyset_build(const float* scores, int64_t scores_stride, int n_heads, const int32_t* mode,
-                                  const int32_t* param, const int32_t* start, const int32_t* include, int frames,
-                                  int tokens_per_frame, int num_special, int32_t* idx, int64_t idx_stride,
-                                  int32_t* count, void* stream) {
-  if (int e = injected("saf3r_keyset_build")) return e;
+// Host lists by value: at most kMaxHeads entries
+static int host_lists(const char* who, int n) {
+  return n > kMaxHeads ? fail(SAF3R_ERR_UNSUPPORTED, "%s: %d heads, at most %d from host lists", who, n, kMaxHeads)
+                       : SAF3R_OK;
+}
+
+extern "C" int saf3r_probe_scores_host(const float* q32, const float* k32, int64_t slot_stride, int n_tokens,
+                                       const int32_t* slots, const int32_t* rows, int n_sel, const int32_t* sample_idx,
+                                       int n_samples, float scale, float* partial, float* qbar, float* scores,
+                                       int64_t scores_stride, void* stream) {
+  const char* who = "saf3r_probe_scores_host";
+  if (int e = injected(who)) return e;
+  ProbeParams p;
+  if (int e = probe_setup(who, q32, k32, slot_stride, n_tokens, slots, n_sel, sample_idx, n_samples, scale, qbar,
+                          scores, scores_stride, &p))
+    return e;
+  if (!partial || !rows) return fail(SAF3R_ERR_INVALID, "%s: null workspace or rows", who);
+  if (int e = host_lists(who, n_sel)) return e;
+  p.slots = nullptr;
+  for (int i = 0; i < n_sel; ++i) {
+    if (slots[i] < 0 || rows[i] < 0) return fail(SAF3R_ERR_INVALID, "%s: negative slot or row", who);
+    p.slot_val[i] = slots[i];
+    p.row_val[i] = rows[i];
+  }
+  p.partial = partial;
+  return probe_launch(p, n_sel, stream);
+}
+
+static int build_launch(const char* who, const float* scores, int64_t scores_stride, int n_heads, const int32_t* mode,
+                        const int32_t* param, const int32_t* start, const int32_t* include, bool host, int frames,
+                        int tokens_per_frame, int num_special, int32_t* idx, int64_t idx_stride, int32_t* count,
+                        void* stream) {
+  if (int e = injected(who)) return e;
   Geom g;
-  if (!make_geom(frames, tokens_per_frame, num_special, &g))
-    return fail(SAF3R_ERR_INVALID, "saf3r_keyset_build: invalid geometry");
+  if (!make_geom(frames, tokens_per_frame, num_special, &g)) return fail(SAF3R_ERR_INVALID, "%s: invalid geometry", who);
   const int64_t n = (int64_t)frames * tokens_per_frame;
-  if (n > 0x7fffffff) return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_keyset_build: too many tokens");
-  if (n_heads <= 0 || n_heads > 65535) return fail(SAF3R_ERR_INVALID, "saf3r_keyset_build: bad n_heads %d", n_heads);
-  if (!mode || !param || !start || !include || !idx || !count)
-    return fail(SAF3R_ERR_INVALID, "saf3r_keyset_build: null pointer");
-  if (idx_stride < n) return fail(SAF3R_ERR_INVALID, "saf3r_keyset_build: idx_stride below the token count");
+  if (n > 0x7fffffff) return fail(SAF3R_ERR_UNSUPPORTED, "%s: too many tokens", who);
+  if (n_heads <= 0 || n_heads > 65535) return fail(SAF3R_ERR_INVALID, "%s: bad n_heads %d", who, n_heads);
+  if (!mode || !param || !start || !include || !idx || !count) return fail(SAF3R_ERR_INVALID, "%s: null pointer", who);
+  if (idx_stride < n) return fail(SAF3R_ERR_INVALID, "%s: idx_stride below the token count", who);
   BuildParams p;
   p.scores = scores;
   p.scores_stride = scores_stride;
@@ -514,6 +548,17 @@ extern "C" int saf3r_keyset_build(const float* scores, int64_t scores_stride, in
   p.param = param;
   p.start = start;
   p.include = include;
+  if (host) {
+    if (int e = host_lists(who, n_heads)) return e;
+    for (int i = 0; i < n_heads; ++i) {
+      if (mode[i] == SAF3R_KEYSET_TOPK && !scores) return fail(SAF3R_ERR_INVALID, "%s: top-k heads need scores", who);
+      p.spec[0][i] = mode[i];
+      p.spec[1][i] = param[i];
+      p.spec[2][i] = start[i];
+      p.spec[3][i] = include[i];
+    }
+    p.mode = p.param = p.start = p.include = nullptr;
+  }
   p.n = (int)n;
   p.T = tokens_per_frame;
   p.ns = num_special;
@@ -521,28 +566,52 @@ extern "C" int saf3r_keyset_build(const float* scores, int64_t scores_stride, in
   p.idx_stride = idx_stride;
   p.count = count;
   hipLaunchKernelGGL(keyset_build_kernel, dim3(n_heads), dim3(kBuildThreads), 0, (hipStream_t)stream, p);
-  return check_launch("saf3r_keyset_build");
+  return check_launch(who);
 }
 
-extern "C" int saf3r_keyset_gather(const void* k_packed, int frames, int tokens_per_frame, int num_special,
+extern "C" int saf3r_keyset_build(const float* scores, int64_t scores_stride, int n_heads, const int32_t* mode,
+                                  const int32_t* param, const int32_t* start, const int32_t* include, int frames,
+                                  int tokens_per_frame, int num_special, int32_t* idx, int64_t idx_stride,
+                                  int32_t* count, void* stream) {
+  return build_launch("saf3r_keyset_build", scores, scores_stride, n_heads, mode, param, start, include, false, frames,
+                      tokens_per_frame, num_special, idx, idx_stride, count, stream);
+}
+
+extern "C" int saf3r_keyset_build_host(const float* scores, int64_t scores_stride, int n_heads, const int32_t* mode,
+                                       const int32_t* param, const int32_t* start, const int32_t* include, int frames,
+                                       int tokens_per_frame, int num_special, int32_t* idx, int64_t idx_stride,
+                                       int32_t* count, void* stream) {
+  return build_launch("saf3r_keyset_build_host", scores, scores_stride, n_heads, mode, param, start, include, true,
+                      frames, tokens_per_frame, num_special, idx, idx_stride, count, stream);
+}
+
+static int gather_launch(const char* who, bool host, const void* k_packed, int frames, int tokens_per_frame, int num_special,
                                    const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
                                    int64_t v_head_stride, const int32_t* idx, int64_t idx_stride,
                                    const int32_t* count, int max_tiles, void* keyset_k, void* keyset_v,
                                    int64_t capacity, void* stream) {
-  if (int e = injected("saf3r_keyset_gather")) return e;
+  if (int e = injected(who)) return e;
   GatherKParams p;
   if (!make_geom(frames, tokens_per_frame, num_special, &p.g))
-    return fail(SAF3R_ERR_INVALID, "saf3r_keyset_gather: invalid geometry");
+    return fail(SAF3R_ERR_INVALID, "%s: invalid geometry", who);
   if (!k_packed || !head_ids || !v || !idx || !count || !keyset_k || !keyset_v)
-    return fail(SAF3R_ERR_INVALID, "saf3r_keyset_gather: null pointer");
+    return fail(SAF3R_ERR_INVALID, "%s: null pointer", who);
   if (n_sel <= 0 || n_sel > 65535 || max_tiles <= 0 || capacity % 64 || (int64_t)max_tiles * 64 > capacity)
-    return fail(SAF3R_ERR_INVALID, "saf3r_keyset_gather: bad n_sel %d, max_tiles %d or capacity %lld", n_sel,
+    return fail(SAF3R_ERR_INVALID, "%s: bad n_sel %d, max_tiles %d or capacity %lld", who, n_sel,
                 max_tiles, (long long)capacity);
   if (v_tok_stride % 8 || v_head_stride % 8 || ((uintptr_t)v | (uintptr_t)k_packed) % 16 ||
       ((uintptr_t)keyset_k | (uintptr_t)keyset_v) % 16)
-    return fail(SAF3R_ERR_INVALID, "saf3r_keyset_gather: 16-byte alignment required");
+    return fail(SAF3R_ERR_INVALID, "%s: 16-byte alignment required", who);
   p.k = (const __bf16*)k_packed;
   p.head_ids = head_ids;
+  if (host) {
+    if (int e = host_lists(who, n_sel)) return e;
+    for (int i = 0; i < n_sel; ++i) {
+      if (head_ids[i] < 0) return fail(SAF3R_ERR_INVALID, "%s: negative head", who);
+      p.head_val[i] = head_ids[i];
+    }
+    p.head_ids = nullptr;
+  }
   p.v = (const __bf16*)v;
   p.v_tok_stride = v_tok_stride;
   p.v_head_stride = v_head_stride;
@@ -553,5 +622,21 @@ extern "C" int saf3r_keyset_gather(const void* k_packed, int frames, int tokens_
   p.vc = (__bf16*)keyset_v;
   p.capacity = capacity;
   hipLaunchKernelGGL(keyset_gather_kernel, dim3(max_tiles, n_sel), dim3(256), 0, (hipStream_t)stream, p);
-  return check_launch("saf3r_keyset_gather");
+  return check_launch(who);
+}
+
+extern "C" int saf3r_keyset_gather(const void* k_packed, int frames, int tokens_per_frame, int num_special,
+                                   const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
+                                   int64_t v_head_stride, const int32_t* idx, int64_t idx_stride,
+                                   const int32_t* count, int max_tiles, void* keyset_k, void* keyset_v,
+                                   int64_t capacity, void* stream) {
+  return gather_launch("saf3r_keyset_gather", false, k_packed, frames, tokens_per_frame, num_special, head_ids, n_sel, v, v_tok_stride, v_head_stride, idx, idx_stride, count, max_tiles, keyset_k, keyset_v, capacity, stream);
+}
+
+extern "C" int saf3r_keyset_gather_host(const void* k_packed, int frames, int tokens_per_frame, int num_special,
+                                   const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
+                                   int64_t v_head_stride, const int32_t* idx, int64_t idx_stride,
+                                   const int32_t* count, int max_tiles, void* keyset_k, void* keyset_v,
+                                   int64_t capacity, void* stream) {
+  return gather_launch("saf3r_keyset_gather_host", true, k_packed, frames, tokens_per_frame, num_special, head_ids, n_sel, v, v_tok_stride, v_head_stride, idx, idx_stride, count, max_tiles, keyset_k, keyset_v, capacity, stream);
 }

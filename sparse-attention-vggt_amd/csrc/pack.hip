@@ -19,14 +19,16 @@ struct PackParams {
   const __bf16* k;
   const __bf16* v;
   int64_t tok_stride, head_stride;
-  const float* qw;
-  const float* qb;
-  const float* kw;
-  const float* kb;
+  const void* qw;  // LayerNorm parameters, fp32 or (ln_bf16) bf16
+  const void* qb;
+  const void* kw;
+  const void* kb;
   float eps;
   int apply_ln;
+  int ln_bf16;
   int apply_rope;
   const int32_t* pos;
+  int pos_step;  // words between positions: 1, or 2 for the low words of int64 ones
   const float* rcos;
   const float* rsin;
   int rpos;
@@ -86,7 +88,7 @@ __global__ __launch_bounds__(512) void pack_qkv_kernel(PackParams p) {
   // angle index e % 16 and, for e < 16, -t[e + 16] (else +t[e - 16]) as its partner term
   float cs[8], sn[8];
   if (p.apply_rope && tok >= 0) {
-    const int pv = min(max(p.pos[tok * 2 + (c8 >> 2)], 0), p.rpos - 1);
+    const int pv = min(max(p.pos[(tok * 2 + (c8 >> 2)) * p.pos_step], 0), p.rpos - 1);
     const f32x4* c4 = reinterpret_cast<const f32x4*>(p.rcos + pv * 16 + 8 * (c8 & 1));
     const f32x4* s4 = reinterpret_cast<const f32x4*>(p.rsin + pv * 16 + 8 * (c8 & 1));
 #pragma unroll
@@ -127,10 +129,27 @@ __global__ __launch_bounds__(512) void pack_qkv_kernel(PackParams p) {
       v2 += __shfl_xor(v2, 2);
       v2 += __shfl_xor(v2, 4);
       const float rstd = 1.0f / sqrtf(v2 * (1.0f / 64.0f) + p.eps);
-      const float* w = which == 0 ? p.qw : p.kw;
-      const float* b = which == 0 ? p.qb : p.kb;
+      const void* w = which == 0 ? p.qw : p.kw;
+      const void* b = which == 0 ? p.qb : p.kb;
+      float wv[8], bv[8];
+      if (p.ln_bf16) {  // the parameters as the module holds them: no fp32 copies per call
+        const u32x4 w4 = reinterpret_cast<const u32x4*>(w)[c8], b4 = reinterpret_cast<const u32x4*>(b)[c8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = (x[j] - mean) * rstd * w[8 * c8 + j] + b[8 * c8 + j];
+        for (int j = 0; j < 4; ++j) {
+          wv[2 * j] = bf16_lo(w4[j]);
+          wv[2 * j + 1] = bf16_hi(w4[j]);
+          bv[2 * j] = bf16_lo(b4[j]);
+          bv[2 * j + 1] = bf16_hi(b4[j]);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          wv[j] = static_cast<const float*>(w)[8 * c8 + j];
+          bv[j] = static_cast<const float*>(b)[8 * c8 + j];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = (x[j] - mean) * rstd * wv[j] + bv[j];
     }
     if (p.apply_rope) {
       float y[8];
@@ -225,30 +244,36 @@ __global__ __launch_bounds__(512) void pack_qkv_kernel(PackParams p) {
 
 using namespace saf3r;
 
-extern "C" int saf3r_pack_qkv(const void* q, const void* k, const void* v, int64_t tok_stride, int64_t head_stride,
+static int pack_launch(const char* who, const void* q, const void* k, const void* v, int64_t tok_stride, int64_t head_stride,
                               int frames, int tokens_per_frame, int num_special, int num_heads,
-                              const float* q_ln_weight, const float* q_ln_bias, const float* k_ln_weight,
-                              const float* k_ln_bias, float ln_eps, int apply_ln, const int32_t* pos,
+                              const void* q_ln_weight, const void* q_ln_bias, const void* k_ln_weight,
+                              const void* k_ln_bias, float ln_eps, int apply_ln, const void* pos,
                               const float* rope_cos, const float* rope_sin, int rope_positions, void* q_packed,
                               void* k_packed, void* v_packed, const uint8_t* token_order, const uint8_t* fp32_heads,
                               float* qk32, const uint8_t* q_scaled, float q_scale, const uint8_t* pool_heads,
-                              float* pool_mean, uint16_t* pool_split, float* pool_meta, void* stream) {
-  if (int e = injected("saf3r_pack_qkv")) return e;
+                              float* pool_mean, uint16_t* pool_split, float* pool_meta, int param_flags,
+                       void* stream) {
+  if (int e = injected(who)) return e;
   PackParams p;
+  if (param_flags & ~(SAF3R_PACK_LN_BF16 | SAF3R_PACK_POS_INT64))
+    return fail(SAF3R_ERR_INVALID, "%s: unknown param_flags 0x%x", who, param_flags);
   if (!make_geom(frames, tokens_per_frame, num_special, &p.g))
-    return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: invalid geometry F=%d T=%d ns=%d", frames, tokens_per_frame,
+    return fail(SAF3R_ERR_INVALID, "%s: invalid geometry F=%d T=%d ns=%d", who, frames, tokens_per_frame,
                 num_special);
-  if (num_heads <= 0 || num_heads > 65535) return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: bad num_heads %d", num_heads);
+  if (num_heads <= 0 || num_heads > 65535) return fail(SAF3R_ERR_INVALID, "%s: bad num_heads %d", who, num_heads);
   if (!q || !k || !v || !q_packed || !k_packed || !v_packed)
-    return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: null tensor pointer");
+    return fail(SAF3R_ERR_INVALID, "%s: null tensor pointer", who);
   if (tok_stride % 8 || head_stride % 8 || ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % 16)
-    return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: inputs must be 16-byte aligned with strides a multiple of 8");
+    return fail(SAF3R_ERR_INVALID, "%s: inputs must be 16-byte aligned with strides a multiple of 8", who);
   if (((uintptr_t)q_packed | (uintptr_t)k_packed | (uintptr_t)v_packed) % 16)
-    return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: packed outputs must be 16-byte aligned");
+    return fail(SAF3R_ERR_INVALID, "%s: packed outputs must be 16-byte aligned", who);
   if (apply_ln && (!q_ln_weight || !q_ln_bias || !k_ln_weight || !k_ln_bias))
-    return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: LayerNorm requested without parameters");
+    return fail(SAF3R_ERR_INVALID, "%s: LayerNorm requested without parameters", who);
+  if (apply_ln && (param_flags & SAF3R_PACK_LN_BF16) &&
+      ((uintptr_t)q_ln_weight | (uintptr_t)q_ln_bias | (uintptr_t)k_ln_weight | (uintptr_t)k_ln_bias) % 16)
+    return fail(SAF3R_ERR_INVALID, "%s: bf16 LayerNorm parameters must be 16-byte aligned", who);
   if (rope_cos && (!pos || !rope_sin || rope_positions <= 0 || ((uintptr_t)rope_cos | (uintptr_t)rope_sin) % 16))
-    return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: RoPE needs positions and 16-byte aligned cos/sin tables");
+    return fail(SAF3R_ERR_INVALID, "%s: RoPE needs positions and 16-byte aligned cos/sin tables", who);
   p.q = (const __bf16*)q;
   p.k = (const __bf16*)k;
   p.v = (const __bf16*)v;
@@ -260,8 +285,10 @@ extern "C" int saf3r_pack_qkv(const void* q, const void* k, const void* v, int64
   p.kb = k_ln_bias;
   p.eps = ln_eps;
   p.apply_ln = apply_ln != 0;
+  p.ln_bf16 = (param_flags & SAF3R_PACK_LN_BF16) != 0;
   p.apply_rope = rope_cos != nullptr;
-  p.pos = pos;
+  p.pos = static_cast<const int32_t*>(pos);
+  p.pos_step = (param_flags & SAF3R_PACK_POS_INT64) ? 2 : 1;
   p.rcos = rope_cos;
   p.rsin = rope_sin;
   p.rpos = rope_positions;
@@ -273,15 +300,15 @@ extern "C" int saf3r_pack_qkv(const void* q, const void* k, const void* v, int64
     for (int h = 0; h < num_heads; ++h) {
       const int lay = token_order[h];
       if (!lay) continue;
-      if (h >= 64) return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_pack_qkv: token order is supported for heads 0..63");
+      if (h >= 64) return fail(SAF3R_ERR_UNSUPPORTED, "%s: token order is supported for heads 0..63", who);
       if (lay == SAF3R_LAYOUT_TOKEN) {
         p.tok_order |= 1ull << h;
       } else if (lay == SAF3R_LAYOUT_FRAMED) {
         if (!framed_fits(p.g))
-          return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_pack_qkv: the framed layout needs ceil(T/64) = ceil(P/64) here");
+          return fail(SAF3R_ERR_UNSUPPORTED, "%s: the framed layout needs ceil(T/64) = ceil(P/64) here", who);
         p.framed |= 1ull << h;
       } else {
-        return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: head %d: unknown layout %d", h, lay);
+        return fail(SAF3R_ERR_INVALID, "%s: head %d: unknown layout %d", who, h, lay);
       }
     }
   }
@@ -291,23 +318,23 @@ extern "C" int saf3r_pack_qkv(const void* q, const void* k, const void* v, int64
     int n32 = 0;
     for (int h = 0; h < num_heads; ++h) {
       if (!fp32_heads[h]) continue;
-      if (h >= 64) return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_pack_qkv: fp32 rows are supported for heads 0..63");
+      if (h >= 64) return fail(SAF3R_ERR_UNSUPPORTED, "%s: fp32 rows are supported for heads 0..63", who);
       p.f32_heads |= 1ull << h;
       p.f32slot[h] = (int8_t)n32++;
     }
     if (n32 > 0 && (!qk32 || (uintptr_t)qk32 % 16))
-      return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: fp32 heads need a 16-byte aligned qk32 buffer");
+      return fail(SAF3R_ERR_INVALID, "%s: fp32 heads need a 16-byte aligned qk32 buffer", who);
   }
   p.q_scaled = 0;
   p.q_scale = q_scale;
   if (q_scaled) {
     for (int h = 0; h < num_heads; ++h) {
       if (!q_scaled[h]) continue;
-      if (h >= 64) return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_pack_qkv: scaled Q is supported for heads 0..63");
+      if (h >= 64) return fail(SAF3R_ERR_UNSUPPORTED, "%s: scaled Q is supported for heads 0..63", who);
       p.q_scaled |= 1ull << h;
     }
     if (p.q_scaled && !(q_scale > 0.f && q_scale < 3.0e38f))
-      return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: q_scale must be positive and finite");
+      return fail(SAF3R_ERR_INVALID, "%s: q_scale must be positive and finite", who);
   }
   p.pool_heads = 0;
   p.pool_mean = pool_mean;
@@ -317,17 +344,39 @@ extern "C" int saf3r_pack_qkv(const void* q, const void* k, const void* v, int64
     int np = 0;
     for (int h = 0; h < num_heads; ++h) {
       if (!pool_heads[h]) continue;
-      if (h >= 64) return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_pack_qkv: pooling is supported for heads 0..63");
+      if (h >= 64) return fail(SAF3R_ERR_UNSUPPORTED, "%s: pooling is supported for heads 0..63", who);
       if (((p.tok_order | p.framed) >> h) & 1)
-        return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: pooled head %d must use the packed layout", h);
+        return fail(SAF3R_ERR_INVALID, "%s: pooled head %d must use the packed layout", who, h);
       p.pool_heads |= 1ull << h;
       p.pool_slot[h] = (int8_t)np++;
     }
     if (np > 0 && (!pool_mean || !pool_split || !pool_meta || ((uintptr_t)pool_mean | (uintptr_t)pool_split |
                                                                 (uintptr_t)pool_meta) % 16))
-      return fail(SAF3R_ERR_INVALID, "saf3r_pack_qkv: pooled heads need 16-byte aligned pool_mean / split / meta");
+      return fail(SAF3R_ERR_INVALID, "%s: pooled heads need 16-byte aligned pool_mean / split / meta", who);
   }
   dim3 grid(p.g.NT, num_heads);
   hipLaunchKernelGGL(pack_qkv_kernel, grid, dim3(512), 0, (hipStream_t)stream, p);
-  return check_launch("saf3r_pack_qkv");
+  return check_launch(who);
+}
+
+extern "C" int saf3r_pack_qkv(const void* q, const void* k, const void* v, int64_t tok_stride, int64_t head_stride,
+                              int frames, int tokens_per_frame, int num_special, int num_heads,
+                              const float* q_ln_weight, const float* q_ln_bias, const float* k_ln_weight,
+                              const float* k_ln_bias, float ln_eps, int apply_ln, const int32_t* pos,
+                              const float* rope_cos, const float* rope_sin, int rope_positions, void* q_packed,
+                              void* k_packed, void* v_packed, const uint8_t* token_order, const uint8_t* fp32_heads,
+                              float* qk32, const uint8_t* q_scaled, float q_scale, const uint8_t* pool_heads,
+                              float* pool_mean, uint16_t* pool_split, float* pool_meta, void* stream) {
+  return pack_launch("saf3r_pack_qkv", q, k, v, tok_stride, head_stride, frames, tokens_per_frame, num_special, num_heads, q_ln_weight, q_ln_bias, k_ln_weight, k_ln_bias, ln_eps, apply_ln, pos, rope_cos, rope_sin, rope_positions, q_packed, k_packed, v_packed, token_order, fp32_heads, qk32, q_scaled, q_scale, pool_heads, pool_mean, pool_split, pool_meta, 0, stream);
+}
+
+extern "C" int saf3r_pack_qkv_typed(const void* q, const void* k, const void* v, int64_t tok_stride, int64_t head_stride,
+                              int frames, int tokens_per_frame, int num_special, int num_heads,
+                              const void* q_ln_weight, const void* q_ln_bias, const void* k_ln_weight,
+                              const void* k_ln_bias, float ln_eps, int apply_ln, const void* pos,
+                              const float* rope_cos, const float* rope_sin, int rope_positions, void* q_packed,
+                              void* k_packed, void* v_packed, const uint8_t* token_order, const uint8_t* fp32_heads,
+                              float* qk32, const uint8_t* q_scaled, float q_scale, const uint8_t* pool_heads,
+                              float* pool_mean, uint16_t* pool_split, float* pool_meta, int param_flags, void* stream) {
+  return pack_launch("saf3r_pack_qkv_typed", q, k, v, tok_stride, head_stride, frames, tokens_per_frame, num_special, num_heads, q_ln_weight, q_ln_bias, k_ln_weight, k_ln_bias, ln_eps, apply_ln, pos, rope_cos, rope_sin, rope_positions, q_packed, k_packed, v_packed, token_order, fp32_heads, qk32, q_scaled, q_scale, pool_heads, pool_mean, pool_split, pool_meta, param_flags, stream);
 }

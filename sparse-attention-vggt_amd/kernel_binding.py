@@ -40,7 +40,7 @@ def _check(rc: int) -> None:
 
 
 def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return _lib.stream_ptr()
 
 
 def fused_sparse_topk_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv_indices: torch.Tensor,

@@ -11,6 +11,7 @@ use the same buffers: token order (DENSE heads, slot t = token t) and the framed
 from __future__ import annotations
 
 from dataclasses import dataclass
+from functools import cached_property, lru_cache
 
 BLOCK = 64
 HEAD_DIM = 64
@@ -30,48 +31,54 @@ class Geometry:
     def from_tokens(cls, num_tokens: int, tokens_per_frame: int, num_special: int = 5) -> "Geometry":
         if num_tokens % tokens_per_frame:
             raise ValueError(f"{num_tokens} tokens is not a whole number of {tokens_per_frame}-token frames")
-        return cls(num_tokens // tokens_per_frame, tokens_per_frame, num_special)
+        return _geometry(cls, num_tokens // tokens_per_frame, tokens_per_frame, num_special)
 
-    @property
+    @cached_property
     def patches(self) -> int:
         return self.tokens_per_frame - self.num_special
 
-    @property
+    @cached_property
     def blocks_per_frame(self) -> int:
         return -(-self.patches // BLOCK)
 
-    @property
+    @cached_property
     def num_blocks(self) -> int:
         return self.frames * self.blocks_per_frame
 
-    @property
+    @cached_property
     def tokens(self) -> int:
         return self.frames * self.tokens_per_frame
 
-    @property
+    @cached_property
     def special_slots(self) -> int:
         return -(-(self.frames * self.num_special) // BLOCK) * BLOCK
 
-    @property
+    @cached_property
     def padded_patches(self) -> int:
         return self.blocks_per_frame * BLOCK
 
-    @property
+    @cached_property
     def slots(self) -> int:
         """Packed slots per head (L)."""
         return self.special_slots + self.frames * self.padded_patches
 
-    @property
+    @cached_property
     def tiles(self) -> int:
         return self.slots // BLOCK
 
-    @property
+    @cached_property
     def frame_tiles(self) -> int:
         """Tiles per frame in the framed layout (NBT = ceil(T/64))."""
         return -(-self.tokens_per_frame // BLOCK)
 
-    @property
+    @cached_property
     def framed_fits(self) -> bool:
         """The framed layout (frame f's T tokens in token order at tile f*NBT) fits the L slots of a
         head: the special tokens fit the padding of a frame's last patch tile, or there are none."""
         return self.frames * self.frame_tiles * BLOCK <= self.slots
+
+
+@lru_cache(maxsize=64)
+def _geometry(cls, frames: int, tokens_per_frame: int, num_special: int) -> Geometry:
+    """Geometries of a model's forwards: one object per size, whose derived counts are computed once."""
+    return cls(frames, tokens_per_frame, num_special)

@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes
 import math
 from dataclasses import dataclass
+from functools import lru_cache
 from typing import Sequence
 
 import torch
@@ -76,8 +77,8 @@ def _mark(name, phase):
         _recorder(name, phase)
 
 
-def _ptr(t: torch.Tensor | None):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def _ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
 def _need_cuda(*ts):
@@ -86,31 +87,49 @@ def _need_cuda(*ts):
             raise ValueError("saf3r kernels take GPU tensors")
 
 
-def _i32_array(vals: Sequence[int]):
-    arr = (ctypes.c_int32 * len(vals))(*[int(v) for v in vals])
-    return arr
+# Host arrays of per-head values, by their values: the C entries only read them, and a model's layers
+# pass the same few tables in every forward.
+@lru_cache(maxsize=1024)
+def _i32_values(vals: tuple):
+    return (ctypes.c_int32 * len(vals))(*[int(v) for v in vals])
 
 
-def _u8_flags(flags: Sequence[bool] | None, n: int):
-    """Host uint8 [n] flag array for the C ABI (None: no array)."""
-    if flags is None:
-        return None
-    flags = list(flags)
+@lru_cache(maxsize=1024)
+def _flag_values(flags: tuple, n: int):
     if len(flags) != n:
         raise ValueError(f"one flag per head: got {len(flags)} for {n} heads")
     return (ctypes.c_uint8 * n)(*[1 if f else 0 for f in flags])
 
 
-def _u8_layouts(layouts: Sequence[int] | None, n: int):
-    """Host uint8 [n] array of per-head layouts (``LAYOUT_*``; True counts as ``LAYOUT_TOKEN``)."""
-    if layouts is None:
-        return None
+@lru_cache(maxsize=1024)
+def _layout_values(layouts: tuple, n: int):
     layouts = [int(x) for x in layouts]
     if len(layouts) != n:
         raise ValueError(f"one layout per head: got {len(layouts)} for {n} heads")
     if any(x not in (LAYOUT_PACKED, LAYOUT_TOKEN, LAYOUT_FRAMED) for x in layouts):
         raise ValueError(f"unknown layout in {layouts}")
     return (ctypes.c_uint8 * n)(*layouts)
+
+
+@lru_cache(maxsize=1024)
+def _pattern_counts(patterns: tuple) -> tuple[int, int, int]:
+    """Heads served from block lists, from key sets and from the broadcast buffers."""
+    return (sum(1 for p in patterns if p == BLOCK_DYNAMIC), sum(1 for p in patterns if p in KEYSET_PATTERNS),
+            sum(1 for p in patterns if p == BROADCAST))
+
+
+def _i32_array(vals: Sequence[int]):
+    return _i32_values(tuple(vals))
+
+
+def _u8_flags(flags: Sequence[bool] | None, n: int):
+    """Host uint8 [n] flag array for the C ABI (None: no array)."""
+    return None if flags is None else _flag_values(tuple(flags), n)
+
+
+def _u8_layouts(layouts: Sequence[int] | None, n: int):
+    """Host uint8 [n] array of per-head layouts (``LAYOUT_*``; True counts as ``LAYOUT_TOKEN``)."""
+    return None if layouts is None else _layout_values(tuple(layouts), n)
 
 
 FRAMED_PATTERNS = (FRAME_LOCAL, ANCHOR_LOCAL, ANCHOR)  # heads that can take the framed layout
@@ -177,6 +196,16 @@ class Pooled:
                       torch.empty(n, 2, nb, 2, dtype=torch.float32, device=device))
 
 
+def _ln_params(params, device):
+    """(the four LayerNorm parameter tensors the pack reads, whether they are bf16)."""
+    if any(t.numel() != HEAD_DIM for t in params):
+        raise ValueError("LayerNorm weight and bias must hold 64 values each")
+    if all(t.dtype == torch.bfloat16 and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0
+           for t in params):
+        return params, True
+    return tuple(t.detach().to(device=device, dtype=torch.float32).contiguous() for t in params), False
+
+
 def pack_qkv(q, k, v, tok_stride: int, head_stride: int, geom: Geometry, num_heads: int,
              ln_q=None, ln_k=None, ln_eps: float = 1e-5, pos=None, rope_base=None, rope_positions=None, out=None,
              token_order: Sequence[int] | None = None, fp32_heads: Sequence[bool] | None = None,
@@ -207,11 +236,11 @@ def pack_qkv(q, k, v, tok_stride: int, head_stride: int, geom: Geometry, num_hea
         qk32 = torch.empty(sum(1 for f in fp32_heads if f), 2, geom.tokens, HEAD_DIM, dtype=torch.float32,
                            device=q.device)
     apply_ln = ln_q is not None
-    if apply_ln:  # fp32 device copies (the kernel reads them as device arrays of 64 floats)
-        qw, qb = (t.detach().to(device=q.device, dtype=torch.float32).contiguous() for t in ln_q)
-        kw, kb = (t.detach().to(device=q.device, dtype=torch.float32).contiguous() for t in ln_k)
-        if any(t.numel() != HEAD_DIM for t in (qw, qb, kw, kb)):
-            raise ValueError("LayerNorm weight and bias must hold 64 values each")
+    param_flags = 0
+    if apply_ln:  # bf16 parameters are read as they are, others as fp32 copies
+        ln, bf16_params = _ln_params((*ln_q, *ln_k), q.device)
+        param_flags = _lib.PACK_LN_BF16 if bf16_params else 0
+        qw, qb, kw, kb = ln
     else:
         qw = qb = kw = kb = None
     rc = rs = None
@@ -219,18 +248,23 @@ def pack_qkv(q, k, v, tok_stride: int, head_stride: int, geom: Geometry, num_hea
     if rope_base is not None:
         if pos is None:
             raise ValueError("RoPE needs positions")
-        pos = pos.to(device=q.device, dtype=torch.int32).contiguous()
+        if pos.dtype == torch.int64 and pos.device == q.device:
+            pos = pos.contiguous()
+            param_flags |= _lib.PACK_POS_INT64
+        else:
+            pos = pos.to(device=q.device, dtype=torch.int32).contiguous()
         npos = int(rope_positions) if rope_positions is not None else int(pos.max().item()) + 1
         rc, rs = rope_tables(npos, rope_base, q.device)
     _mark("pack_qkv", "start")
-    _lib.check(lib.saf3r_pack_qkv(
+    _lib.check(lib.saf3r_pack_qkv_typed(
         _ptr(q), _ptr(k), _ptr(v), tok_stride, head_stride, geom.frames, geom.tokens_per_frame, geom.num_special,
         num_heads, _ptr(qw), _ptr(qb), _ptr(kw), _ptr(kb), float(ln_eps), int(apply_ln),
         _ptr(pos) if rc is not None else None, _ptr(rc), _ptr(rs), npos, _ptr(qp), _ptr(kp), _ptr(vp),
         _u8_layouts(token_order, num_heads), _u8_flags(fp32_heads, num_heads) if qk32 is not None else None,
         _ptr(qk32), _u8_flags(q_scaled, num_heads), float(prescale_factor() if q_scale is None else q_scale),
         _u8_flags(pool_flags, num_heads), _ptr(pooled.mean if pooled else None),
-        _ptr(pooled.split if pooled else None), _ptr(pooled.meta if pooled else None), _lib.stream_ptr()))
+        _ptr(pooled.split if pooled else None), _ptr(pooled.meta if pooled else None), param_flags,
+        _lib.stream_ptr()))
     _mark("pack_qkv", "end")
     res = (qp, kp, vp) + ((qk32,) if fp32_heads is not None else ()) + ((pooled,) if pooled is not None else ())
     return res
@@ -367,7 +401,8 @@ def sparse_attn_fwd(qp, kp, vp, geom: Geometry, patterns: Sequence[int], sel: to
         raise ValueError(f"out must be bf16 [N, >= H*64] with unit column stride, got {tuple(out.shape)}")
     scale = 1.0 / math.sqrt(HEAD_DIM) if scale is None else scale
     width = 0
-    n_dyn = sum(1 for p in patterns if p == BLOCK_DYNAMIC)
+    patterns = tuple(patterns)
+    n_dyn, n_ks, n_bc = _pattern_counts(patterns)
     if n_dyn:
         if sel is None:
             raise ValueError("block-dynamic heads need a selection list")
@@ -378,14 +413,12 @@ def sparse_attn_fwd(qp, kp, vp, geom: Geometry, patterns: Sequence[int], sel: to
         width = sel.shape[-1]
     else:
         sel = None
-    n_ks = sum(1 for p in patterns if p in KEYSET_PATTERNS)
     ks_k = ks_v = ks_n = None
     ks_cap = 0
     if n_ks:
         if keysets is None or keysets.k.shape[0] != n_ks:
             raise ValueError(f"{n_ks} key-set heads need {n_ks} gathered key sets")
         ks_k, ks_v, ks_n, ks_cap = keysets.k, keysets.v, keysets.count, keysets.capacity
-    n_bc = sum(1 for p in patterns if p == BROADCAST)
     bq = bk = bv = None
     if n_bc:
         if broadcast is None or broadcast.q.shape[0] != n_bc:
@@ -565,6 +598,7 @@ def token_topk(q: torch.Tensor, k: torch.Tensor, frames: int, per_frame: int, to
 # Shared key sets of the stride and q_probe_topk modes
 # ----------------------------------------------------------------------------------------
 KEYSET_STRIDE, KEYSET_TOPK = 0, 1
+MAX_HEADS = 64  # of the C entries that take their lists from host memory
 
 
 @dataclass
@@ -605,12 +639,14 @@ class KeySets:
 
 
 def probe_scores(qk32: torch.Tensor, slots: Sequence[int], scale: float | None = None,
-                 sample: torch.Tensor | None = None, noalloc: bool = False):
+                 sample: torch.Tensor | None = None, noalloc: bool = False, out: torch.Tensor | None = None,
+                 rows: Sequence[int] | None = None):
     """Mean query and probe scores (``saf3r/patch/sparse_attention.py:150-168``) of the heads stored at
     ``slots`` of ``qk32`` (fp32 [n, 2, N, 64], q and k rows in token order, as ``pack_qkv`` writes them
     for ``fp32_heads``): returns (qbar fp32 [n_sel][64], scores fp32 [n_sel][N]). ``sample`` (int tokens)
     restricts the mean to those query rows, in list order (the reference's ``q_sample_ratio < 1``).
-    ``noalloc`` uses the allocation-free entry (its partial sums in the library's static workspace)."""
+    ``noalloc`` uses the allocation-free entry (its partial sums in the library's static workspace).
+    ``out`` (fp32 [.., >= N], contiguous) with ``rows`` receives head i's scores in row ``rows[i]``."""
     _need_cuda(qk32)
     lib = _lib.load()
     if qk32.dtype != torch.float32 or qk32.dim() != 4 or qk32.shape[1] != 2 or qk32.shape[3] != HEAD_DIM \
@@ -619,25 +655,43 @@ def probe_scores(qk32: torch.Tensor, slots: Sequence[int], scale: float | None =
     N = qk32.shape[2]
     n = len(slots)
     dev = qk32.device
-    hs = torch.tensor(list(slots), dtype=torch.int32, device=dev)
+    slots = list(slots)
+    rows = list(range(n)) if rows is None else list(rows)
     qbar = torch.empty(n, HEAD_DIM, dtype=torch.float32, device=dev)
-    scores = torch.empty(n, N, dtype=torch.float32, device=dev)
+    if out is None:
+        scores = torch.empty(max(rows) + 1 if rows else 0, N, dtype=torch.float32, device=dev)
+    else:
+        scores = out
+        if (out.dtype != torch.float32 or out.dim() != 2 or not out.is_contiguous() or out.shape[1] < N
+                or (rows and max(rows) >= out.shape[0])):
+            raise ValueError("out must be contiguous fp32 [> max(rows), >= N]")
     scale = 1.0 / math.sqrt(HEAD_DIM) if scale is None else scale
     if sample is not None:
         sample = sample.to(device=dev, dtype=torch.int32).contiguous()
         if sample.dim() != 1 or not 1 <= sample.numel() <= N:
             raise ValueError("sample must list between 1 and N tokens")
     stride = qk32.stride(0)
-    args = (_ptr(qk32), ctypes.c_void_p(qk32.data_ptr() + 4 * qk32.stride(1)), stride, N, _ptr(hs), n, _ptr(sample),
-            0 if sample is None else sample.numel(), float(scale))
+    kptr = qk32.data_ptr() + 4 * qk32.stride(1)
+    n_samp = 0 if sample is None else sample.numel()
+    by_value = n <= MAX_HEADS and not noalloc  # the lists go with the launch
+    hs = None if by_value else torch.tensor(slots, dtype=torch.int32, device=dev)
+    if not by_value and rows != list(range(n)):
+        raise ValueError("rows need at most 64 heads and the allocating entry")
     _mark("probe", "start")
     if noalloc:
-        _lib.check(lib.saf3r_probe_scores_noalloc(*args, _ptr(qbar), _ptr(scores), scores.stride(0),
+        _lib.check(lib.saf3r_probe_scores_noalloc(_ptr(qk32), kptr, stride, N, _ptr(hs), n, _ptr(sample), n_samp,
+                                                  float(scale), _ptr(qbar), _ptr(scores), scores.stride(0),
                                                   _lib.stream_ptr()))
     else:
         partial = torch.empty(n, 256, HEAD_DIM, dtype=torch.float32, device=dev)
-        _lib.check(lib.saf3r_probe_scores(*args, _ptr(partial), _ptr(qbar), _ptr(scores), scores.stride(0),
-                                          _lib.stream_ptr()))
+        if by_value:
+            _lib.check(lib.saf3r_probe_scores_host(_ptr(qk32), kptr, stride, N, _i32_array(slots), _i32_array(rows), n,
+                                                   _ptr(sample), n_samp, float(scale), _ptr(partial), _ptr(qbar),
+                                                   _ptr(scores), scores.stride(0), _lib.stream_ptr()))
+        else:
+            _lib.check(lib.saf3r_probe_scores(_ptr(qk32), kptr, stride, N, _ptr(hs), n, _ptr(sample), n_samp,
+                                              float(scale), _ptr(partial), _ptr(qbar), _ptr(scores), scores.stride(0),
+                                              _lib.stream_ptr()))
     _mark("probe", "end")
     return qbar, scores
 
@@ -659,8 +713,8 @@ def keyset_build(specs: Sequence[KeySetSpec], geom: Geometry, scores: torch.Tens
     n = len(specs)
     if any(s.param <= 0 for s in specs):
         raise ValueError("key-set stride / k must be positive")
-    arr = torch.tensor([[s.mode, s.param, s.start, int(bool(s.include))] for s in specs], dtype=torch.int32)
-    arr = arr.t().contiguous().to(device)
+    lists = [[s.mode for s in specs], [s.param for s in specs], [s.start for s in specs],
+             [int(bool(s.include)) for s in specs]]
     idx = torch.empty(n, geom.tokens, dtype=torch.int32, device=device)
     count = torch.empty(n, dtype=torch.int32, device=device)
     if scores is not None:
@@ -669,9 +723,15 @@ def keyset_build(specs: Sequence[KeySetSpec], geom: Geometry, scores: torch.Tens
             raise ValueError("scores must be fp32 [n_specs, >= N]")
         scores = scores.contiguous()
     _mark("keyset_build", "start")
-    _lib.check(lib.saf3r_keyset_build(_ptr(scores), 0 if scores is None else scores.stride(0), n, _ptr(arr[0]),
-                                      _ptr(arr[1]), _ptr(arr[2]), _ptr(arr[3]), geom.frames, geom.tokens_per_frame,
-                                      geom.num_special, _ptr(idx), idx.stride(0), _ptr(count), _lib.stream_ptr()))
+    # (top-k heads without scores keep the device-list entry's behaviour)
+    if n <= MAX_HEADS and (scores is not None or KEYSET_TOPK not in lists[0]):
+        entry, args = lib.saf3r_keyset_build_host, [_i32_array(x) for x in lists]
+    else:
+        arr = torch.tensor(lists, dtype=torch.int32, device=device)
+        entry, args = lib.saf3r_keyset_build, [_ptr(arr[i]) for i in range(4)]
+    _lib.check(entry(_ptr(scores), 0 if scores is None else scores.stride(0), n, *args, geom.frames,
+                     geom.tokens_per_frame, geom.num_special, _ptr(idx), idx.stride(0), _ptr(count),
+                     _lib.stream_ptr()))
     _mark("keyset_build", "end")
     return idx, count
 
@@ -687,11 +747,16 @@ def keyset_gather(kp: torch.Tensor, geom: Geometry, specs: Sequence[KeySetSpec],
     dev = kp.device
     kc = torch.empty(n, cap, HEAD_DIM, dtype=torch.bfloat16, device=dev)
     vc = torch.empty(n, cap // 64, 64, 64, dtype=torch.bfloat16, device=dev)
-    hs = torch.tensor([s.head for s in specs], dtype=torch.int32, device=dev)
+    heads = [s.head for s in specs]
     _mark("keyset_gather", "start")
-    _lib.check(lib.saf3r_keyset_gather(_ptr(kp), geom.frames, geom.tokens_per_frame, geom.num_special, _ptr(hs), n,
-                                       _ptr(v), v_tok_stride, v_head_stride, _ptr(idx), idx.stride(0), _ptr(count),
-                                       cap // 64, _ptr(kc), _ptr(vc), cap, _lib.stream_ptr()))
+    if n <= MAX_HEADS:
+        entry, hs = lib.saf3r_keyset_gather_host, _i32_array(heads)
+    else:
+        dev_heads = torch.tensor(heads, dtype=torch.int32, device=dev)
+        entry, hs = lib.saf3r_keyset_gather, _ptr(dev_heads)
+    _lib.check(entry(_ptr(kp), geom.frames, geom.tokens_per_frame, geom.num_special, hs, n, _ptr(v), v_tok_stride,
+                     v_head_stride, _ptr(idx), idx.stride(0), _ptr(count), cap // 64, _ptr(kc), _ptr(vc), cap,
+                     _lib.stream_ptr()))
     _mark("keyset_gather", "end")
     return KeySets(kc, vc, count, idx, cap)
 

@@ -125,9 +125,8 @@ def update_args_per_forward(model, img_h, img_w):
             continue
         if not isinstance(attn, BaseHeadwiseSparseAttentionWrapper):
             continue
-        attn.patch_height = patch_height
-        attn.patch_width = patch_width
-        attn.first_dino_flag = False
+        # plain values, straight into the instance (nn.Module's attribute checks cost 3 us a layer)
+        attn.__dict__.update(patch_height=patch_height, patch_width=patch_width, first_dino_flag=False)
 
 
 def set_dino_topk_from_features(model, patch_tokens: Tensor, model_cfg):

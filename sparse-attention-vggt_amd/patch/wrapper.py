@@ -15,6 +15,8 @@ Instead of a Python loop over heads, every head runs in the single attention lau
 """
 from __future__ import annotations
 
+from functools import lru_cache
+
 import torch
 from torch import nn
 
@@ -41,6 +43,12 @@ def _get(cfg, key, default=None):
     if isinstance(cfg, dict):
         return cfg.get(key, default)
     return getattr(cfg, key, default)
+
+
+@lru_cache(maxsize=1024)
+def _head_layouts(patterns: tuple, geom: Geometry) -> tuple:
+    """``ops.token_order_heads`` of a head table, by value (a model's layers repeat a few tables)."""
+    return tuple(ops.token_order_heads(patterns, geom))
 
 
 class BaseHeadwiseSparseAttentionWrapper(nn.Module):
@@ -121,20 +129,21 @@ class BaseHeadwiseSparseAttentionWrapper(nn.Module):
         C = H * HEAD_DIM
         ln_q = ln_k = None
         eps = 1e-5
-        if isinstance(om.q_norm, nn.LayerNorm):
-            ln_q = (om.q_norm.weight, om.q_norm.bias)
-            ln_k = (om.k_norm.weight, om.k_norm.bias)
-            eps = om.q_norm.eps
-        elif not isinstance(om.q_norm, nn.Identity):
-            raise NotImplementedError(f"q_norm {type(om.q_norm).__name__} is not LayerNorm / Identity")
+        q_norm, k_norm, rope = om.q_norm, om.k_norm, om.rope
+        if isinstance(q_norm, nn.LayerNorm):
+            ln_q = (q_norm.weight, q_norm.bias)
+            ln_k = (k_norm.weight, k_norm.bias)
+            eps = q_norm.eps
+        elif not isinstance(q_norm, nn.Identity):
+            raise NotImplementedError(f"q_norm {type(q_norm).__name__} is not LayerNorm / Identity")
         base = p2 = npos = None
-        if om.rope is not None and pos is not None:
-            base = float(om.rope.base_frequency)
+        if rope is not None and pos is not None:
+            base = float(rope.base_frequency)
             p2 = pos.reshape(-1, 2)
             # table length: the patch grid bounds every position ((y+1, x+1) with specials at 0)
             npos = max(self.patch_height, self.patch_width) + 1 if self.patch_height else None
         # dense heads: unpadded token-order tiles; frame-relative heads: whole frames per tile run
-        tord = ops.token_order_heads(self.patterns, geom)
+        tord = _head_layouts(tuple(self.patterns), geom)
         f32 = [h in self.fp32_slot for h in range(H)] if self.fp32_heads else None
         # block_topk heads: the pack also writes their pooled block records (means of bf16 q / k)
         return ops.pack_qkv(qkv, qkv[:, C:], qkv[:, 2 * C:], 3 * C, HEAD_DIM, geom, H, ln_q=ln_q, ln_k=ln_k,
@@ -147,7 +156,7 @@ class BaseHeadwiseSparseAttentionWrapper(nn.Module):
         om = self.orig_module
         H = self.num_heads
         C = H * HEAD_DIM
-        tord = ops.token_order_heads(self.patterns, geom)
+        tord = _head_layouts(tuple(self.patterns), geom)
         qs = self.q_scaled_heads()
         packed = self.pack(qkv, pos, geom)
         qp, kp, vp = packed[:3]
@@ -160,13 +169,15 @@ class BaseHeadwiseSparseAttentionWrapper(nn.Module):
             else:
                 sel = ops.block_select(pooled.mean[:, 0], pooled.mean[:, 1], geom.frames, geom.blocks_per_frame,
                                        self.layer_block_topk, self.topk_scope)
-        self.last_selection = sel  # block lists of the block_topk heads, in head order
+        # (straight into the instance: nn.Module's attribute checks cost more than a launch)
+        kept = self.__dict__
+        kept["last_selection"] = sel  # block lists of the block_topk heads, in head order
         if self.dino_heads:
             self._lazy_token_topk(qp, kp, geom)
         keysets = None
         if self.keyset_heads:
             keysets = self._keysets(qk32, kp, qkv, geom, C)
-        self.last_keysets = keysets
+        kept["last_keysets"] = keysets
         bcast = None
         if self.broadcast_heads:  # broadcast_first: frame 0's Q/K rows and every frame's V tiles
             bcast = ops.broadcast_gather(qp, kp, geom, self.broadcast_heads, qkv[:, 2 * C:], qkv.stride(0), HEAD_DIM)
@@ -182,7 +193,7 @@ class BaseHeadwiseSparseAttentionWrapper(nn.Module):
                 vr = ops.rows(qkv, 3 * C, ns, P, T, offset=2 * C + h * HEAD_DIM)
                 orr = ops.rows(out, C, ns, P, T, offset=h * HEAD_DIM)
                 ops.gather_attn_rows(qr, kr, vr, est, W, geom.frames * P, W, geom.frames * P, None, orr, qk_fp32=True)
-        self.last_attention = out if self.keep_attention else None
+        kept["last_attention"] = out if self.keep_attention else None
         return out
 
     def _keysets(self, qk32, kp, qkv, geom: Geometry, C: int):
@@ -197,13 +208,12 @@ class BaseHeadwiseSparseAttentionWrapper(nn.Module):
             if len(ratios) == 1 and len(probe_rows) == len(specs):
                 _, scores = ops.probe_scores(qk32, [self.fp32_slot[specs[i].head] for i in probe_rows],
                                              sample=ops.probe_sample(geom.tokens, ratios[0]))
-            else:  # one call per sample ratio; rows of stride heads stay unused zeros
-                scores = torch.zeros(len(specs), geom.tokens, dtype=torch.float32, device=kp.device)
+            else:  # one call per sample ratio; rows of stride heads are not read
+                scores = torch.empty(len(specs), geom.tokens, dtype=torch.float32, device=kp.device)
                 for r in ratios:
                     rows_r = [i for i in probe_rows if specs[i].sample_ratio == r]
-                    _, sc = ops.probe_scores(qk32, [self.fp32_slot[specs[i].head] for i in rows_r],
-                                             sample=ops.probe_sample(geom.tokens, r))
-                    scores[rows_r] = sc
+                    ops.probe_scores(qk32, [self.fp32_slot[specs[i].head] for i in rows_r],
+                                     sample=ops.probe_sample(geom.tokens, r), out=scores, rows=rows_r)
         idx, count = ops.keyset_build(specs, geom, scores, kp.device)
         ks = ops.keyset_gather(kp, geom, specs, qkv[:, 2 * C:], qkv.stride(0), HEAD_DIM, idx, count)
         ks.scores = scores
