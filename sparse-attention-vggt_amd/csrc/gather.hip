@@ -8,10 +8,12 @@
 // bandwidth of those row reads, not by arithmetic (a list is one query's own, so there is no
 // matrix product to share between queries). A wave owns two query rows (32 lanes each) and walks
 // their lists in steps of ENT entries with an fp32 online softmax, so any list length is handled by
-// the same kernel. Lane l of a row's 32 serves key slot ks = l / 8 of every group of 4 keys and dims
-// 8 dg .. 8 dg + 7 (dg = l % 8): 8 lanes read a K or V row together (32 bytes each of an fp32 K row,
-// 16 of a bf16 row), so one load instruction moves 8 whole rows (4 of each query), and the 8 partial
-// dot products of a row are summed by three DPP steps inside the 8 lanes. Entries < 0 or >= num_keys are skipped. q and k
+// the same kernel. Lane l of a row's 32 serves key slot ks = l / 8 of every group of 4 keys and 8 dims
+// (dg = l % 8: dims 8 dg .. of a bf16 row; 4 dg .. 4 dg + 3 and 32 + 4 dg .. of an fp32 row): 8 lanes
+// read a K or V row together, 16 bytes each per load, so that one load instruction covers 8 whole
+// 128-byte lines, one per row (32 adjacent bytes of an fp32 row per lane, as two loads, touched 16
+// lines in each: 404 against 398 us at 64 x 1036 fp32 rows, lists of 256), and the 8 partial dot products of a row are summed by three DPP steps inside
+// the 8 lanes. Entries < 0 or >= num_keys are skipped. q and k
 // are bf16 or fp32 rows (the reference's kernel upcasts either); v and out are bf16 or fp32 rows
 // (the reference writes out in v.dtype from its fp32 accumulator).
 //
@@ -67,10 +69,21 @@ struct GatherParams {
   int64_t nk;
   float c;          // scale * log2(e)
   int64_t resident; // C: waves resident on the GPU at once (walk order only)
+  // narrow row addressing (see narrow_rows): key id sits at byte row32(id) * stride of either tensor
+  const char* kb;
+  const char* vb;
+  int nshift;       // frame of id = (mulhi(nmagic, id) + id) >> nshift; -1: one frame
+  uint32_t nmagic;
+  int ndelta;       // rows from frame to frame beyond the frame's own
+  uint32_t kbytes, vbytes;  // row strides
   float* part;      // sliced mode: partial results [n][kGatherSlices][66] of the rows of this launch
   int64_t r0;       // sliced mode: the first row of this launch (rows r0 .. r0 + n - 1)
 };
 
+// high word of a 32 x 32-bit product as one instruction (the __umulhi library routine is a call)
+__device__ __forceinline__ uint32_t mulhi32(uint32_t a, uint32_t b) { return (uint32_t)(((uint64_t)a * b) >> 32); }
+
+constexpr int kGatherWaves = 4;   // per work-group
 constexpr int kGatherSlices = 8;  // sliced mode: list slices, a multiple of the 8 XCDs
 
 // sum of x over the 8 lanes of this lane's group (quad swaps, then the mirrored quad of the group)
@@ -99,8 +112,10 @@ __device__ inline float slots_sum(float x) {
 // L2 serves more reads of the step's key rows between two fetches of them. QK32: q and k rows are
 // fp32 (the reference's gather reads the fp32 q / k of the autocast forward and multiplies in fp32);
 // otherwise bf16. V32 / O32: v / out rows are fp32; otherwise bf16.
-template <bool QK32, bool V32, bool O32, int ENT, bool SLICED, int QPW>
-__global__ __launch_bounds__(256) void gather_attn_kernel(GatherParams p) {
+// (8 waves per SIMD in sliced mode, 6 with fp32 V rows or wide addresses: 5 - 10% faster there than what the registers
+// ask for by themselves; the one-pass form loses by it)
+template <bool QK32, bool V32, bool O32, bool NARROW, int ENT, bool SLICED, int QPW>
+__global__ __launch_bounds__(64 * kGatherWaves, SLICED ? (V32 || !NARROW ? 6 : 8) : (QK32 || V32 ? 4 : 5)) void gather_attn_kernel(GatherParams p) {
   static_assert(QPW == 1 || QPW == 2, "one or two rows per wave");
   constexpr int LANES = 64 / QPW;       // lanes of one row
   constexpr int SLOTS = LANES / 8;      // key slots of one row
@@ -108,7 +123,7 @@ __global__ __launch_bounds__(256) void gather_attn_kernel(GatherParams p) {
   static_assert(ENT <= LANES && ENT % SLOTS == 0, "a step's entries sit in the row's lanes");
   const int lane = tid_x() & 63, w = tid_x() >> 6, dg = lane & 7;
   const int qh = lane / LANES, qbase = qh * LANES, ks = (lane - qbase) >> 3;
-  constexpr int RPW = 4 * QPW;  // rows per workgroup
+  constexpr int RPW = kGatherWaves * QPW;  // rows per workgroup
   // sliced: workgroup b takes rows RPW g .. RPW g + RPW - 1, g = (b / 8) % G (G = ceil(n / RPW)),
   // of slice (b % 8) + 8 (b / 8G): slice s runs on XCD s % 8, the XCD's slices one after the other
   const int64_t ng = (p.n + RPW - 1) / RPW;
@@ -120,12 +135,12 @@ __global__ __launch_bounds__(256) void gather_attn_kernel(GatherParams p) {
   const int64_t rl = rvalid ? rl_raw : rw;
   const int64_t r = SLICED ? p.r0 + rl : rl;
 
-  // this lane's 8 dims of q: fp32 values (QK32) or bf16 pairs
+  // this lane's 8 dims of q: fp32 values (QK32: dims 4 dg .. and 32 + 4 dg ..) or bf16 pairs (8 dg ..)
   float qv[8];
   uint32_t qw[4];
   if constexpr (QK32) {
-    const f32x4* q4 = reinterpret_cast<const f32x4*>(p.q.row<float>(r) + 8 * dg);
-    const f32x4 a = q4[0], b = q4[1];
+    const f32x4* q4 = reinterpret_cast<const f32x4*>(p.q.row<float>(r) + 4 * dg);
+    const f32x4 a = q4[0], b = q4[8];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       qv[e] = a[e];
@@ -138,7 +153,8 @@ __global__ __launch_bounds__(256) void gather_attn_kernel(GatherParams p) {
     qw[2] = x.z;
     qw[3] = x.w;
   }
-  float acc[8];
+  float acc[8];  // output dims d0 .. d0 + 3 and d1 .. d1 + 3
+  const int d0 = V32 ? 4 * dg : 8 * dg, d1 = V32 ? 32 + 4 * dg : 8 * dg + 4;
 #pragma unroll
   for (int d = 0; d < 8; ++d) acc[d] = 0.f;
   float m_run = -__builtin_inff(), l_run = 0.f;
@@ -170,17 +186,28 @@ __global__ __launch_bounds__(256) void gather_attn_kernel(GatherParams p) {
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
       const int id = __shfl(myid, qbase + SLOTS * it + ks);
-      const int64_t rid = id >= 0 ? id : 0;  // a masked entry reads row 0; its score is dropped
+      const int rid = id >= 0 ? id : 0;  // a masked entry reads row 0; its score is dropped
+      const char *kr, *vr;               // this lane's first dims of the K and the V row
+      if constexpr (NARROW) {
+        uint32_t row = (uint32_t)rid;
+        if (p.nshift >= 0)  // uniform
+          row += (uint32_t)__mul24((int)((mulhi32(p.nmagic, row) + row) >> p.nshift), p.ndelta);
+        kr = p.kb + (__umul24(row, p.kbytes) + 16 * dg);
+        vr = p.vb + (__umul24(row, p.vbytes) + 16 * dg);
+      } else {
+        kr = reinterpret_cast<const char*>(QK32 ? (const void*)(p.k.row<float>(rid) + 4 * dg) : (const void*)(p.k.row(rid) + 8 * dg));
+        vr = reinterpret_cast<const char*>(V32 ? (const void*)(p.v.row<float>(rid) + 4 * dg) : (const void*)(p.v.row(rid) + 8 * dg));
+      }
       float part = 0.f;
       if constexpr (QK32) {
-        const f32x4* k4 = reinterpret_cast<const f32x4*>(p.k.row<float>(rid) + 8 * dg);
-        const f32x4 a = k4[0], b = k4[1];
+        const f32x4* k4 = reinterpret_cast<const f32x4*>(kr);
+        const f32x4 a = k4[0], b = k4[8];
 #pragma unroll
         for (int e = 0; e < 4; ++e) part = __builtin_fmaf(qv[e], a[e], part);
 #pragma unroll
         for (int e = 0; e < 4; ++e) part = __builtin_fmaf(qv[4 + e], b[e], part);
       } else {
-        const u32x4 kx = *reinterpret_cast<const u32x4*>(p.k.row(rid) + 8 * dg);
+        const u32x4 kx = *reinterpret_cast<const u32x4*>(kr);
         // elements are copied to scalars before the bf16x2 bit_cast: a bit_cast applied directly to
         // a vector element (kx[e]) was lowered to element 0 for every e by this compiler
         const uint32_t kw[4] = {kx.x, kx.y, kx.z, kx.w};
@@ -190,15 +217,15 @@ __global__ __launch_bounds__(256) void gather_attn_kernel(GatherParams p) {
                                                  part, false);
       }
       if constexpr (V32) {
-        const f32x4* v4 = reinterpret_cast<const f32x4*>(p.v.row<float>(rid) + 8 * dg);
-        const f32x4 a = v4[0], b = v4[1];
+        const f32x4* v4 = reinterpret_cast<const f32x4*>(vr);
+        const f32x4 a = v4[0], b = v4[8];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           vf[it][e] = a[e];
           vf[it][4 + e] = b[e];
         }
       } else {
-        const u32x4 vx = *reinterpret_cast<const u32x4*>(p.v.row(rid) + 8 * dg);
+        const u32x4 vx = *reinterpret_cast<const u32x4*>(vr);
         vw[it][0] = vx.x;
         vw[it][1] = vx.y;
         vw[it][2] = vx.z;
@@ -243,8 +270,8 @@ __global__ __launch_bounds__(256) void gather_attn_kernel(GatherParams p) {
   if constexpr (SLICED) {  // the slice's unnormalised sum, its maximum and its sum of weights
     float* pr = p.part + (rl * kGatherSlices + slice) * 66;
     if (ks == 0) {
-      *reinterpret_cast<f32x4*>(pr + 8 * dg) = f32x4{acc[0], acc[1], acc[2], acc[3]};
-      *reinterpret_cast<f32x4*>(pr + 8 * dg + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
+      *reinterpret_cast<f32x4*>(pr + d0) = f32x4{acc[0], acc[1], acc[2], acc[3]};
+      *reinterpret_cast<f32x4*>(pr + d1) = f32x4{acc[4], acc[5], acc[6], acc[7]};
     }
     if (lane == qbase) {
       pr[64] = m_run;
@@ -255,9 +282,9 @@ __global__ __launch_bounds__(256) void gather_attn_kernel(GatherParams p) {
   if (ks == 0) {
     const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
     if constexpr (O32) {
-      float* orow = const_cast<float*>(p.out.row<float>(r)) + 8 * dg;
-      *reinterpret_cast<f32x4*>(orow) = f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
-      *reinterpret_cast<f32x4*>(orow + 4) = f32x4{acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv};
+      float* orow = const_cast<float*>(p.out.row<float>(r));
+      *reinterpret_cast<f32x4*>(orow + d0) = f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
+      *reinterpret_cast<f32x4*>(orow + d1) = f32x4{acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv};
     } else {
       uint32_t o[4];
 #pragma unroll
@@ -266,7 +293,8 @@ __global__ __launch_bounds__(256) void gather_attn_kernel(GatherParams p) {
         o[e] = __builtin_bit_cast(uint32_t, pr);
       }
       __bf16* orow = const_cast<__bf16*>(p.out.row<__bf16>(r));
-      *reinterpret_cast<u32x4*>(orow + 8 * dg) = u32x4{o[0], o[1], o[2], o[3]};
+      *reinterpret_cast<u32x2*>(orow + d0) = u32x2{o[0], o[1]};
+      *reinterpret_cast<u32x2*>(orow + d1) = u32x2{o[2], o[3]};
     }
   }
 }
@@ -338,8 +366,9 @@ static bool to_dev(const saf3r_rows* s, RowsDev* d, const char* name, bool fp32 
   return true;
 }
 
-constexpr int kGatherStep = 32;        // list entries per walk step
-constexpr int kGatherStepSliced = 16;  // the same in sliced mode (a slice's 64 entries in 4 steps)
+// list entries per walk step: 32 held 96 to 120 registers (one pass, 64 x 1036 rows, lists of 256: bf16
+// 351 -> 277 us, fp32 q / k 640 -> 372), 8 gave the loads too little to overlap (3 to 20% slower)
+constexpr int kGatherStep = 16;
 constexpr int kGatherRows = 2;  // rows per wave (both modes)
 constexpr int64_t kGatherChunkRows = 65536;  // sliced mode: rows per pair of launches
 
@@ -349,38 +378,72 @@ static int64_t resident_waves(K kernel) {
   int dev = 0, cus = 0, blocks = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, 256, 0) != hipSuccess || cus <= 0 || blocks <= 0)
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, 64 * kGatherWaves, 0) != hipSuccess || cus <= 0 || blocks <= 0)
     return 1;
-  return (int64_t)cus * blocks * 4;
+  return (int64_t)cus * blocks * kGatherWaves;
 }
 
-template <bool QK32, bool V32, bool O32>
-static void launch_gather_o(GatherParams p, bool sliced, hipStream_t st) {
+template <bool QK32, bool V32, bool O32, bool NARROW>
+static void launch_gather_n(GatherParams p, bool sliced, hipStream_t st) {
+  constexpr int RPW = kGatherWaves * kGatherRows;
   if (sliced) {
-    auto kernel = gather_attn_kernel<QK32, V32, O32, kGatherStepSliced, true, kGatherRows>;
+    auto kernel = gather_attn_kernel<QK32, V32, O32, NARROW, kGatherStep, true, kGatherRows>;
     p.resident = resident_waves(kernel);
-    // rows in chunks: one chunk's partial results (138 MB) stay in the memory-side cache between
-    // its two kernels, and the workspace holds one chunk
-    const int64_t n = p.n;
-    for (int64_t r0 = 0; r0 < n; r0 += kGatherChunkRows) {
+    // rows in equal chunks, so that the workspace holds one chunk
+    const int64_t n = p.n, chunks = (n + kGatherChunkRows - 1) / kGatherChunkRows;
+    const int64_t per = ((n + chunks - 1) / chunks + RPW - 1) / RPW * RPW;
+    for (int64_t r0 = 0; r0 < n; r0 += per) {
       p.r0 = r0;
-      p.n = (int)(n - r0 < kGatherChunkRows ? n - r0 : kGatherChunkRows);
-      const unsigned gs = (unsigned)((p.n + 4 * kGatherRows - 1) / (4 * kGatherRows));
+      p.n = (int)(n - r0 < per ? n - r0 : per);
+      const unsigned gs = (unsigned)((p.n + RPW - 1) / RPW);
       const unsigned g4 = (unsigned)((p.n + 3) / 4);
-      hipLaunchKernelGGL(kernel, dim3(gs * kGatherSlices), dim3(256), 0, st, p);
+      hipLaunchKernelGGL(kernel, dim3(gs * kGatherSlices), dim3(64 * kGatherWaves), 0, st, p);
       hipLaunchKernelGGL(gather_merge_kernel<O32>, dim3(g4), dim3(256), 0, st, p);
     }
   } else {
-    auto kernel = gather_attn_kernel<QK32, V32, O32, kGatherStep, false, kGatherRows>;
+    auto kernel = gather_attn_kernel<QK32, V32, O32, NARROW, kGatherStep, false, kGatherRows>;
     p.resident = resident_waves(kernel);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((p.n + 4 * kGatherRows - 1) / (4 * kGatherRows))), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((p.n + RPW - 1) / RPW)), dim3(64 * kGatherWaves), 0, st, p);
   }
 }
 
+template <bool QK32, bool V32, bool O32>
+static void launch_gather_o(const GatherParams& p, bool narrow, bool sliced, hipStream_t st) {
+  if (narrow) launch_gather_n<QK32, V32, O32, true>(p, sliced, st);
+  else launch_gather_n<QK32, V32, O32, false>(p, sliced, st);
+}
+
 template <bool QK32, bool V32>
-static void launch_gather(const GatherParams& p, bool o32, bool sliced, hipStream_t st) {
-  if (o32) launch_gather_o<QK32, V32, true>(p, sliced, st);
-  else launch_gather_o<QK32, V32, false>(p, sliced, st);
+static void launch_gather(const GatherParams& p, bool o32, bool narrow, bool sliced, hipStream_t st) {
+  if (o32) launch_gather_o<QK32, V32, true>(p, narrow, sliced, st);
+  else launch_gather_o<QK32, V32, false>(p, narrow, sliced, st);
+}
+
+// Narrow row addressing: K and V rows map ids to frames alike, every row number and row stride fits
+// 24 bits and every byte offset 32, so a lane forms both addresses with a few 24- and 32-bit
+// instructions on uniform bases. The general form's 64-bit multiplies were about 20 of 55 VALU
+// instructions per gathered key (sliced, 64 x 1036 rows, lists of 256: bf16 313 -> 278 us, fp32
+// 422 -> 404; the rest is the rate at which the L1 delivers the rows, 64 bytes a clock and CU).
+static bool narrow_rows(GatherParams* p, bool qk32, bool v32) {
+  const RowsDev &k = p->k, &v = p->v;
+  const bool mapped = k.shift >= 0;
+  if (k.shift != v.shift || k.magic != v.magic) return false;
+  if (mapped && (k.rows_per_frame != v.rows_per_frame || k.frame_row_stride != v.frame_row_stride)) return false;
+  const int64_t kbytes = k.row_stride * (qk32 ? 4 : 2), vbytes = v.row_stride * (v32 ? 4 : 2);
+  const int64_t delta = mapped ? k.frame_row_stride - k.rows_per_frame : 0;
+  const int64_t lim = (int64_t)1 << 24;
+  if (p->nk > lim || kbytes < 0 || vbytes < 0 || kbytes >= lim || vbytes >= lim || delta < 0 || delta >= lim / 2)
+    return false;
+  const int64_t last = p->nk - 1 + (mapped ? (p->nk - 1) / k.rows_per_frame * delta : 0);  // the largest row
+  if (last >= lim || (last + 1) * kbytes > 0xFFFFFFFFll || (last + 1) * vbytes > 0xFFFFFFFFll) return false;
+  p->kb = static_cast<const char*>(k.ptr) + k.base_row * kbytes;
+  p->vb = static_cast<const char*>(v.ptr) + v.base_row * vbytes;
+  p->nshift = k.shift;
+  p->nmagic = k.magic;
+  p->ndelta = (int)delta;
+  p->kbytes = (uint32_t)kbytes;
+  p->vbytes = (uint32_t)vbytes;
+  return true;
 }
 
 // shared by both entries: argument checks and the launch
@@ -407,13 +470,14 @@ static int gather_run(const char* who, const saf3r_rows* q, const saf3r_rows* k,
   p.part = part;
   p.r0 = 0;
   const bool sliced = part != nullptr;
+  const bool narrow = narrow_rows(&p, qk32, v32);
   hipStream_t st = (hipStream_t)stream;
   if (qk32) {
-    if (v32) launch_gather<true, true>(p, o32, sliced, st);
-    else launch_gather<true, false>(p, o32, sliced, st);
+    if (v32) launch_gather<true, true>(p, o32, narrow, sliced, st);
+    else launch_gather<true, false>(p, o32, narrow, sliced, st);
   } else {
-    if (v32) launch_gather<false, true>(p, o32, sliced, st);
-    else launch_gather<false, false>(p, o32, sliced, st);
+    if (v32) launch_gather<false, true>(p, o32, narrow, sliced, st);
+    else launch_gather<false, false>(p, o32, narrow, sliced, st);
   }
   return check_launch(who);
 }

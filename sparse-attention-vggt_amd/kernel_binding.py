@@ -77,7 +77,7 @@ def fused_sparse_topk_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     lib = _lib.load()
     args = (ctypes.byref(_rows(q)), ctypes.byref(_rows(k)), ctypes.byref(_rows(v)), ctypes.c_void_p(idx.data_ptr()),
             idx.stride(0), N, idx.shape[1], k.shape[0], float(scale), flags, ctypes.byref(_rows(out)))
-    if ops.gather_sliced(N, idx.shape[1]):  # many rows with long lists: the two-pass kernels
+    if ops.gather_sliced(N, idx.shape[1], flags):  # many rows with long lists: the two-pass kernels
         nbytes = lib.saf3r_gather_attn_workspace_bytes(N, idx.shape[1])
         if nbytes < 0:
             raise RuntimeError(lib.saf3r_last_error().decode(errors="replace"))

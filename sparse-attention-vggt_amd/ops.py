@@ -495,22 +495,29 @@ def gather_attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, idx: torc
 _gather_ws = {}  # (device, bytes) -> the sliced gather's workspace, kept for the next call of the same size
 
 
-def gather_sliced(n: int, topk: int) -> bool:
-    """Whether a gather of ``n`` rows with ``topk``-entry lists takes the two-pass sliced kernels (many
-    rows with long lists, where the rows the lists touch exceed one XCD's L2)."""
-    return topk >= 128 and n * topk >= (1 << 22)
+def gather_sliced(n: int, topk: int, dtype_flags: int = _lib.GATHER_QK_FP32) -> bool:
+    """Whether a gather of ``n`` rows with ``topk``-entry lists takes the two-pass sliced kernels: many rows with
+    long lists, from fewer on the more bytes a key has. Measured (us, one pass / sliced) with lists of 128 at
+    33152 rows (4.2 M entries): bf16 61 / 93, fp32 q / k 89 / 91, all fp32 138 / 105; lists of 512 at 8288 rows (the
+    same entries) 67 / 62, 70 / 67, 93 / 79; lists of 256 at 66304 rows (17 M) 269 / 250, 377 / 303, 700 / 388; all
+    fp32 with lists of 128 at 16576 rows (2.1 M) 55 / 56."""
+    if topk < 128 or n * topk < (1 << 22):
+        return False
+    if dtype_flags & _lib.GATHER_V_FP32 or topk >= 512:
+        return True
+    return n * topk >= (1 << (23 if dtype_flags & _lib.GATHER_QK_FP32 else 24))
 
 
 def gather_attn_rows(qr, kr, vr, idx, idx_row_stride, n, topk, num_keys, scale, outr, keep=None, qk_fp32=False,
                      dtype_flags=None, sliced=None):
     """``saf3r_gather_attn_fwd`` on row descriptors; ``qk_fp32``: q and k rows are fp32 (or give the
-    full ``dtype_flags``). ``sliced`` (default: ``gather_sliced(n, topk)``) runs
+    full ``dtype_flags``). ``sliced`` (default: ``gather_sliced``) runs
     ``saf3r_gather_attn_fwd_sliced`` with a workspace kept per device and size."""
     lib = _lib.load()
     scale = 1.0 / math.sqrt(HEAD_DIM) if scale is None else scale
     flags = (_lib.GATHER_QK_FP32 if qk_fp32 else 0) if dtype_flags is None else dtype_flags
     if sliced is None:
-        sliced = gather_sliced(n, topk)
+        sliced = gather_sliced(n, topk, flags)
     _mark("gather_attn", "start")
     if sliced and n > 0:
         nbytes = int(lib.saf3r_gather_attn_workspace_bytes(n, topk))
