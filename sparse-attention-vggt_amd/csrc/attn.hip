@@ -36,6 +36,7 @@
 // step, points to: all resident work-groups then touch nearby key frames at the same moment. The
 // walk order changes only the summation order; the host can turn it off for run-to-run identical
 // output.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -77,6 +78,7 @@ struct AttnParams {
   uint64_t tok_order;    // DENSE heads (bit h) packed in token order: tile t = tokens 64t .. 64t+63
   uint64_t framed;       // frame-relative heads (bit h) in the framed layout: frame f = tiles f*NBT ..
   uint64_t q_pre;        // heads (bit h) whose Q rows hold q * scale * log2(e)
+  uint64_t split;        // heads (bit h) whose single-range walks run in split mode (short launches)
   int n_items;           // fixup launch: items in the segments, work-groups of the launch
   int fix_groups;
   int ntok;              // F*T tokens
@@ -578,6 +580,8 @@ struct Item {
   bool tokord, framed;
 };
 
+// SPLIT: a launch in which some heads' single-range walks are split (AttnParams.split)
+template <bool SPLIT>
 __device__ inline Item decode_item(const AttnParams& p, int item) {
   const Geom& g = p.g;
   Item d;
@@ -592,7 +596,11 @@ __device__ inline Item decode_item(const AttnParams& p, int item) {
   const int groups_pf = (g.NBf + 3) >> 2;
   d.tokord = pat == SAF3R_DENSE && ((p.tok_order >> d.h) & 1);
   d.framed = d.h < 64 && ((p.framed >> d.h) & 1);
-  if (d.framed) {
+  if (SPLIT && d.h < 64 && ((p.split >> d.h) & 1)) {  // one query tile per item, in tile order
+    d.qt0 = it;
+    d.nw = 4;
+    d.kind = kSplit;
+  } else if (d.framed) {
     // four consecutive query tiles of one frame (the frame's last item may hold fewer)
     const int gpf = (g.NBT + 3) >> 2, f = it / gpf, gg = it - f * gpf;
     d.qt0 = f * g.NBT + 4 * gg;
@@ -644,7 +652,7 @@ __device__ inline uint16_t* item_marker(const AttnParams& p, const Item& d) {
 
 // The kernel body for work item `item` (uniform). FIXUP: walked again, exactly, because the main
 // launch marked it.
-template <bool FIXUP>
+template <bool FIXUP, bool SPLIT>
 __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
   __shared__ __align__(16) char ring[kRing];
   __shared__ int list[kMaxList];
@@ -665,7 +673,7 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
   }
 
   // ---- decode the work item (uniform) ----
-  const Item d = decode_item(p, item);
+  const Item d = decode_item<SPLIT>(p, item);
   const int h = d.h, pat = d.pat, qt0 = d.qt0, nw = d.nw, kind = d.kind;
   const int bfr = d.bfr;  // BROADCAST: the frame whose rows the item writes
   const bool tokord = d.tokord, framed = d.framed;
@@ -1083,25 +1091,50 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
 
   // ================= split mode: one query tile, block list split across the four waves ======
   {
-    // compact the selection row into LDS (drop invalid entries, keep order); an entry holds the
-    // key tile and the number of valid keys of its block: tile << 7 | valid (1..64)
-    const int32_t* srow = p.sel + ((int64_t)p.slot[h] * ((int64_t)g.F * g.NBf) + (qt - g.nst)) * p.sel_width;
+    // The tile list in LDS; an entry holds the key tile and its number of valid keys: tile << 7 | valid
+    // (1..64).
     int total = 0;
-    for (int c0 = 0; c0 < p.sel_width; c0 += 256) {
-      const int j = c0 + tid;
-      const int v = j < p.sel_width ? srow[j] : -1;
-      const bool ok = v >= 0 && v < g.F * g.NBf;
-      const uint64_t m = __ballot(ok);
-      const int pre = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-      if (lane == 0) wcnt[w] = __popcll(m);
-      __syncthreads();
-      int off = total;
-      for (int i = 0; i < w; ++i) off += wcnt[i];
-      if (ok && off + pre < kMaxList) list[off + pre] = ((g.nst + v) << 7) | min(64, g.P - 64 * (v % g.NBf));
-      total += wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
+    const bool kset = SPLIT && (pat == SAF3R_KEYSET || pat == SAF3R_TOKEN_DYNAMIC_KEYSET);
+    if (!SPLIT || (pat == SAF3R_BLOCK_DYNAMIC && qt >= g.nst)) {
+      // a block-dynamic patch tile: its selection row (invalid entries dropped, order kept)
+      const int32_t* srow = p.sel + ((int64_t)p.slot[h] * ((int64_t)g.F * g.NBf) + (qt - g.nst)) * p.sel_width;
+      for (int c0 = 0; c0 < p.sel_width; c0 += 256) {
+        const int j = c0 + tid;
+        const int v = j < p.sel_width ? srow[j] : -1;
+        const bool ok = v >= 0 && v < g.F * g.NBf;
+        const uint64_t m = __ballot(ok);
+        const int pre = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+        if (lane == 0) wcnt[w] = __popcll(m);
+        __syncthreads();
+        int off = total;
+        for (int i = 0; i < w; ++i) off += wcnt[i];
+        if (ok && off + pre < kMaxList) list[off + pre] = ((g.nst + v) << 7) | min(64, g.P - 64 * (v % g.NBf));
+        total += wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
+        __syncthreads();
+      }
+      total = min(total, kMaxList);
+    } else {
+      // single-range walks of short launches: tiles 0 .. of the key set, the tokens or the packed rows,
+      // or a framed head's one or two frames (at most kSplitMaxTiles, which fit the list)
+      const int keys = kset ? min(p.ks_count[p.slot[h]], (int)p.ks_cap) : p.ntok;
+      const int nbt = g.NBT, own = framed && pat != SAF3R_ANCHOR ? qf * nbt : 0;
+      const bool two = framed && pat == SAF3R_ANCHOR_LOCAL && qf != 0;
+      total = __builtin_amdgcn_readfirstlane(framed ? (two ? 2 * nbt : nbt) : (kset || tokord) ? (keys + 63) / 64 : g.NT);
+      for (int i = tid; i < total; i += 256) {
+        int kt = i, valid;
+        if (framed) {
+          const int j = i >= nbt ? i - nbt : i;  // tile of its frame
+          kt = two && i < nbt ? j : own + j;
+          valid = j == nbt - 1 ? g.T - 64 * (nbt - 1) : 64;
+        } else if (kset || tokord) {
+          valid = min(64, keys - 64 * i);
+        } else {
+          valid = i < g.nst ? min(64, g.S - 64 * i) : min(64, g.P - 64 * ((i - g.nst) % g.NBf));
+        }
+        list[i] = (kt << 7) | valid;
+      }
       __syncthreads();
     }
-    total = min(total, kMaxList);
     // wave w takes list positions w, w + 4, w + 8, ...: with lists in frame-major order, the four
     // waves (and, through the clock phase, every resident work-group) advance through the key
     // frames together
@@ -1147,8 +1180,9 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
       vo = (uint32_t)(i * 128 + (((lane & 3) ^ swz4(i)) << 4));
     }
     const uint32_t vo1 = vo + 1024;
-    const char* kbase = reinterpret_cast<const char*>(p.k + head_base * 64);
-    const char* vbase = reinterpret_cast<const char*>(p.v + head_base * 64);
+    const int64_t kv_base = kset ? (int64_t)p.slot[h] * p.ks_cap * 64 : head_base * 64;
+    const char* kbase = reinterpret_cast<const char*>((kset ? p.kc : p.k) + kv_base);
+    const char* vbase = reinterpret_cast<const char*>((kset ? p.vc : p.v) + kv_base);
     char* slots = ring + w * 16384;
     auto issue_k = [&](int e, int hh) {
       const char* kb = kbase + (int64_t)(e >> 7) * 8192 + hh * 4096;
@@ -1305,9 +1339,17 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
     }
     __syncthreads();
     const int row = tid >> 2, d0 = (tid & 3) * 16;
-    int64_t tok;
-    if (qspecial) tok = -1;  // split mode only serves patch tiles
-    else {
+    int64_t tok;  // of the thread's row, as row_info (whose own rows the compiler needs in its form)
+    if (SPLIT && tokord) {
+      const int i = qt * 64 + row;
+      tok = i < p.ntok ? (int64_t)i : -1;
+    } else if (SPLIT && framed) {
+      const int i = qb * 64 + row;
+      tok = i < g.T ? (int64_t)qf * g.T + i : -1;
+    } else if (qspecial) {
+      const int sl = qt * 64 + row;
+      tok = SPLIT && sl < g.S ? (int64_t)(sl / g.ns) * g.T + sl % g.ns : -1;
+    } else {
       const int pp = qb * 64 + row;
       tok = pp < g.P ? (int64_t)qf * g.T + g.ns + pp : -1;
     }
@@ -1353,12 +1395,17 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
   }
 }
 
+// Launches without split walks keep a kernel of their own: with the split walks' code in it the compiler
+// spills 28 bytes a lane instead of 20, which a layer of 48 x 1301 tokens and 24 heads took 3 % longer with
+// (9.76 -> 10.10 ms), one of 32 x 1374 tokens 1.4 % (1.85 -> 1.88 ms).
+template <bool SPLIT>
 __global__ __launch_bounds__(256, 2) void sparse_attn_kernel(AttnParams p) {
-  attn_body<false>(p, __builtin_amdgcn_workgroup_id_x());
+  attn_body<false, SPLIT>(p, __builtin_amdgcn_workgroup_id_x());
 }
 
 // Work-group g reads the markers of items g, g + G, g + 2G, ... (G = fix_groups), 64 at a time on
 // wave 0's lanes, and walks the marked ones exactly, one after the other.
+template <bool SPLIT>
 __global__ __launch_bounds__(256, 2) void sparse_attn_fixup_kernel(AttnParams p) {
   __shared__ uint64_t marked;
   const int tid = __builtin_amdgcn_workitem_id_x();
@@ -1368,7 +1415,7 @@ __global__ __launch_bounds__(256, 2) void sparse_attn_fixup_kernel(AttnParams p)
       const int item = base + G * tid;
       bool m = false;
       if (item < p.n_items) {
-        const Item d = decode_item(p, item);
+        const Item d = decode_item<SPLIT>(p, item);
         m = d.kind != kSkip && *reinterpret_cast<const volatile uint16_t*>(item_marker(p, d)) == 0xFFFFu;
       }
       const uint64_t b = __ballot(m);
@@ -1382,7 +1429,7 @@ __global__ __launch_bounds__(256, 2) void sparse_attn_fixup_kernel(AttnParams p)
     while (b) {
       const int l = __builtin_ctzll(b);
       b &= b - 1;
-      attn_body<true>(p, base + G * l);
+      attn_body<true, SPLIT>(p, base + G * l);
       __syncthreads();  // the next item reuses the LDS
     }
   }
@@ -1394,15 +1441,50 @@ __global__ __launch_bounds__(256, 2) void sparse_attn_fixup_kernel(AttnParams p)
 struct Seg {
   int h, base, items;
   int64_t steps;
+  int64_t cost;  // the same with a split-mode item's fixed part (choose_split)
 };
 
-static int head_segments(int h, int pat, bool tokord, bool framed, int ntt, const Geom& g, int sel_width,
+// Key tiles of the longest walk of a head that split mode can take over from the shared walks (0: none)
+static int64_t split_tiles(int pat, bool tokord, bool framed, int ntt, const Geom& g, int64_t ks_cap) {
+  if (framed) return (int64_t)g.NBT * (pat == SAF3R_ANCHOR_LOCAL ? 2 : 1);
+  switch (pat) {
+    case SAF3R_DENSE: return tokord ? ntt : g.NT;
+    case SAF3R_KEYSET:
+    case SAF3R_TOKEN_DYNAMIC_KEYSET: return ks_cap / 64;
+    case SAF3R_TOKEN_DYNAMIC:
+    case SAF3R_BLOCK_DYNAMIC: return g.nst > 0 ? g.NT : 0;
+    default: return 0;
+  }
+}
+
+// Steps of a split-mode item of n key tiles: a wave's quarter of them, plus what its work-group spends
+// on the list, the first loads and the merge of the four partial results, in steps (fitted: with 2
+// the choice below also split the key-set heads of small profile layers, 46 -> 59 us).
+constexpr int64_t kSplitFixed = 8;
+// Walks whose K and V (16 KB a tile) an XCD's 4 MB of L2 holds: a split walk reads them once per query tile,
+// a shared one once per four, and the clock-paced order of longer dense walks is for shared ones.
+constexpr int64_t kSplitMaxTiles = 256;
+static int64_t split_steps(int64_t n) { return (n + 3) / 4 + kSplitFixed; }
+
+static int head_segments(int h, int pat, bool tokord, bool framed, bool split, int ntt, const Geom& g, int sel_width,
                          int64_t ks_cap, Seg* out) {
   const int ns4 = (g.nst + 3) / 4, groups_pf = (g.NBf + 3) / 4;
   int n = 0;
-  auto add = [&](int base, int items, int64_t steps) {
-    if (items > 0) out[n++] = Seg{h, base, items, steps};
+  auto add = [&](int base, int items, int64_t steps, int64_t cost = 0) {
+    if (items > 0) out[n++] = Seg{h, base, items, steps, cost > 0 ? cost : steps};
   };
+  if (split) {  // one query tile per item
+    const int64_t n4 = split_steps(split_tiles(pat, tokord, framed, ntt, g, ks_cap));
+    if (pat == SAF3R_TOKEN_DYNAMIC || pat == SAF3R_TOKEN_DYNAMIC_KEYSET) {
+      add(0, g.nst, n4);
+    } else if (pat == SAF3R_BLOCK_DYNAMIC) {
+      add(0, g.nst, n4);
+      add(g.nst, g.F * g.NBf, max(1, sel_width / 2), split_steps(sel_width));
+    } else {
+      add(0, framed ? g.F * g.NBT : tokord ? ntt : g.NT, n4);
+    }
+    return n;
+  }
   if (framed) {  // four query tiles of one frame per item; one or two frames of key tiles
     add(0, g.F * ((g.NBT + 3) / 4), (int64_t)g.NBT * (pat == SAF3R_ANCHOR_LOCAL ? 2 : 1));
     return n;
@@ -1423,7 +1505,7 @@ static int head_segments(int h, int pat, bool tokord, bool framed, int ntt, cons
     case SAF3R_TOKEN_DYNAMIC_KEYSET: add(0, ns4, ks_cap / 64); break;
     case SAF3R_BLOCK_DYNAMIC:
       add(0, ns4, g.NT);
-      add(ns4, g.F * g.NBf, max(1, sel_width / 2));
+      add(ns4, g.F * g.NBf, max(1, sel_width / 2), split_steps(sel_width));
       break;
     default: {  // frame-relative patterns: one special tile per item, four patch tiles per item
       const int64_t mult = pat == SAF3R_ANCHOR_LOCAL ? 2 : 1;
@@ -1433,6 +1515,52 @@ static int head_segments(int h, int pat, bool tokord, bool framed, int ntt, cons
     }
   }
   return n;
+}
+
+// The heads whose single-range walks run in split mode (a bit each). A wave takes 1.4 us for a key tile
+// however few work-groups there are, so a short launch takes as long as its longest walk: a dense head
+// of two 1041-token frames is 33 tiles on 9 work-groups. A launch's time is estimated as the larger of its
+// work over the resident work-groups and its longest item; from the longest walk down, heads are split
+// as far as that falls by 5 % and a split item's fixed part. Launches that fill the chip split nothing
+// (the fixed part of every item adds to their work), nor do heads of many short walks.
+// Measured, attention and fixup, us, nothing split / this rule / every walk split: seeded block mix of 16
+// heads, 1041-token frames, 2 frames 62 / 40 / 41, 4 105 / 64 / 70, 8 192 / 145 / 160, 12 294 / 250 / 280;
+// profile layer 11 (dino special rows), 4 frames 96 / 57 / 64; layers 3, 9, 20 (anchor and key-set
+// heads), 4 frames 44 / 44 / 59, 64 / 63 / 70, 65 / 64 / 74. The sum of the two instead of the larger split
+// dense heads of full launches: 32 x 1374 tokens 1870 -> 2010, 128 x 1374 25100 -> 27970.
+struct HeadWork {
+  Seg shared[2], split[2];
+  int n_shared, n_split;
+  bool can_split;
+  int64_t tiles;
+};
+static uint64_t choose_split(const HeadWork* hw, int heads, int64_t slots) {
+  double best = 0;  // of the masks tried so far
+  uint64_t chosen = 0, mask = 0;
+  bool used[kMaxHeads] = {};
+  for (int k = 0;; ++k) {
+    int64_t work = 0, longest = 0;
+    for (int h = 0; h < heads; ++h) {
+      const Seg* s = (mask >> h) & 1 ? hw[h].split : hw[h].shared;
+      const int n = (mask >> h) & 1 ? hw[h].n_split : hw[h].n_shared;
+      for (int i = 0; i < n; ++i) {
+        work += s[i].items * s[i].cost;
+        longest = std::max(longest, s[i].cost);
+      }
+    }
+    const double span = std::max((double)work / (double)slots, (double)longest);
+    if (k == 0) best = span;
+    if (span < 0.95 * best - kSplitFixed) {
+      best = span;
+      chosen = mask;
+    }
+    int next = -1;
+    for (int h = 0; h < heads; ++h)
+      if (hw[h].can_split && !used[h] && (next < 0 || hw[h].tiles > hw[next].tiles)) next = h;
+    if (next < 0) return chosen;
+    used[next] = true;
+    mask |= 1ull << next;
+  }
 }
 
 // the K + V bytes of the block-dynamic heads above which split-mode walks are clock-paced
@@ -1578,11 +1706,26 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   p.pace_read = (int)(pace_seq % 3u);
   p.pace_acc = (int)((pace_seq + 1u) % 3u);
   p.pace_zero = (int)((pace_seq + 2u) % 3u);
+  int cus = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  HeadWork hw[kMaxHeads];
+  for (int h = 0; h < num_heads; ++h) {
+    HeadWork& x = hw[h];
+    const bool to = (p.tok_order >> h) & 1, fr = (p.framed >> h) & 1;
+    x.tiles = split_tiles(p.pattern[h], to, fr, p.ntt, p.g, keyset_capacity);
+    x.can_split = x.tiles > 0 && x.tiles <= kSplitMaxTiles;
+    x.n_shared = head_segments(h, p.pattern[h], to, fr, false, p.ntt, p.g, sel_width, keyset_capacity, x.shared);
+    x.n_split = head_segments(h, p.pattern[h], to, fr, x.can_split, p.ntt, p.g, sel_width, keyset_capacity, x.split);
+  }
+  p.split = choose_split(hw, num_heads, 2 * (int64_t)cus);
   Seg segs[kMaxSegs];
   int nseg = 0;
-  for (int h = 0; h < num_heads; ++h)
-    nseg += head_segments(h, p.pattern[h], (p.tok_order >> h) & 1, (p.framed >> h) & 1, p.ntt, p.g, sel_width,
-                          keyset_capacity, segs + nseg);
+  for (int h = 0; h < num_heads; ++h) {
+    const bool sp = (p.split >> h) & 1;
+    for (int i = 0; i < (sp ? hw[h].n_split : hw[h].n_shared); ++i) segs[nseg++] = (sp ? hw[h].split : hw[h].shared)[i];
+  }
   for (int i = 1; i < nseg; ++i) {  // stable: longest item first
     const Seg x = segs[i];
     int j = i;
@@ -1603,7 +1746,8 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   }
   p.item_start[p.n_order] = (int)total;
   if (total == 0) return SAF3R_OK;
-  hipLaunchKernelGGL(sparse_attn_kernel, dim3((unsigned)total), dim3(256), 0, (hipStream_t)stream, p);
+  hipLaunchKernelGGL(p.split ? sparse_attn_kernel<true> : sparse_attn_kernel<false>, dim3((unsigned)total), dim3(256), 0,
+                     (hipStream_t)stream, p);
   if (int e = check_launch("saf3r_sparse_attn_fwd")) return e;
   // the exact walk of the items that left the FAST range: the same items of the prescaled heads,
   // in the fixed order; every other item returns after reading its marker
@@ -1622,12 +1766,9 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   }
   f.item_start[f.n_order] = (int)ftotal;
   if (ftotal == 0) return SAF3R_OK;
-  int cus = 0, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
   f.n_items = (int)ftotal;
   f.fix_groups = (int)std::min<int64_t>(ftotal, 2 * (int64_t)cus);  // one resident round
-  hipLaunchKernelGGL(sparse_attn_fixup_kernel, dim3((unsigned)f.fix_groups), dim3(256), 0, (hipStream_t)stream, f);
+  hipLaunchKernelGGL(f.split ? sparse_attn_fixup_kernel<true> : sparse_attn_fixup_kernel<false>,
+                     dim3((unsigned)f.fix_groups), dim3(256), 0, (hipStream_t)stream, f);
   return check_launch("saf3r_sparse_attn_fwd");
 }
