@@ -60,7 +60,6 @@ struct AttnParams {
   Geom g;
   int sel_width;
   float c;  // softmax scale * log2(e)
-  uint32_t nsmagic;  // ceil(2^32 / ns): frame of a special slot = umulhi(slot, nsmagic); 0 for ns <= 1
   uint64_t phase_dense;  // default wall-clock ticks per key-tile step of a dense walk (0: fixed order)
   uint64_t phase_split;  // default wall-clock ticks per list position of a split-mode wave (0: fixed order)
   unsigned long long* pace;  // caller's pacing state [2 kinds][3 slots][ticks, steps] (may be null)
@@ -107,7 +106,6 @@ __device__ inline float partner_sum(float x) {
 
 // high word of a 32 x 32-bit product as one multiply instruction (the __umulhi library routine is
 // an out-of-line call here, with the call's register saves, once per use)
-__device__ __forceinline__ uint32_t mulhi_u32(uint32_t a, uint32_t b) { return (uint32_t)(((uint64_t)a * b) >> 32); }
 
 struct Acc {
   f32x16 o[2][2];  // [dh][gq]: O^T rows 32*dh + (16*half + a), query 32*gq + col
@@ -147,56 +145,79 @@ struct TileMask {
   int eff;       // pattern whose frame relation applies (DENSE / BLOCK_DYNAMIC: none)
 };
 
-// One staged key tile (NKH = 2: 64 keys, K rows 128 B, V rows 128 B) or half tile (NKH = 1:
-// 32 keys, V rows 64 B); key0 is the first key of the staged keys within their 64-slot tile.
-template <int NKH, typename Hook>
+// bits 0 .. n - 1 (none below 0, all from 64 up)
+__device__ __forceinline__ uint64_t keys_below(int n) {
+  return n >= 64 ? ~0ull : (1ull << (n < 0 ? 0 : n)) - 1;
+}
+
+// a row without a reference maximum yet uses -2^127: unmasked keys then give +inf (and the exact
+// path), masked keys 0, and no inf - inf (NaN) ever forms
+__device__ __forceinline__ float ref_mc(float m, float c) { return m == -__builtin_inff() ? -0x1p127f : m * c; }
+
+// P = exp2(s*c - mc) of one query group's 16 keys and their partial row sum over the bf16-rounded
+// values the PV product uses (exact path)
+__device__ __forceinline__ float exps_half(const f32x16& s, float c, float mc, bf16x8 (&p)[2]) {
+  const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
+  float t = 0.f;
+#pragma unroll
+  for (int u = 0; u < 16; u += 2) {
+    const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u], c, -mc));
+    const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u + 1], c, -mc));
+    const bf16x2 pr = {(__bf16)e0, (__bf16)e1};
+    p[u >> 3][u & 7] = pr[0];
+    p[u >> 3][(u & 7) + 1] = pr[1];
+    t = __builtin_amdgcn_fdot2_f32_bf16(pr, ones, t, false);
+  }
+  return t;
+}
+
+// Keys 32 kh .. 32 kh + 31 of a staged key tile (K and V rows of 128 B). Half a tile at a time: with the
+// scores and P of a whole one the kernel ran out of registers and kept its Q fragments in scratch
+// memory, in the pipelined walks too (64 frames of 24 x 32 patches 2.95 -> 3.63 ms; with this 2.87).
+template <typename Hook>
 __device__ __forceinline__ void attend(const char* __restrict__ kst, const char* __restrict__ vst,
                                        const bf16x8 (&qfrag)[2][4], Acc& A, const int (&frow)[2],
-                                       const TileMask& tm, const Geom& g, uint32_t nsmagic, int key0, int half,
-                                       int col, float c, Hook&& hook) {
-  f32x16 s[NKH][2];
-  // S^T of the staged keys, masked; also re-run by the exact path below, which keeps s from
-  // having to stay live next to P
+                                       const TileMask& tm, const Geom& g, int kh, int half, int col, float c,
+                                       Hook&& hook) {
+  f32x16 s[2];
+  // S^T of the keys, masked; also re-run by the exact path below, which keeps s from having to stay
+  // live next to P
   auto scores = [&]() {
-#pragma unroll
-    for (int kh = 0; kh < NKH; ++kh) s[kh][0] = s[kh][1] = f32x16{};
+    s[0] = s[1] = f32x16{};
+    const int r = 32 * kh + col;
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
-      const int chn = 4 * half + st;
-#pragma unroll
-      for (int kh = 0; kh < NKH; ++kh) {
-        const int r = 32 * kh + col;
-        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kst + r * 128 + ((chn ^ swz8(r)) << 4));
-        s[kh][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qfrag[0][st], s[kh][0], 0, 0, 0);
-        s[kh][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qfrag[1][st], s[kh][1], 0, 0, 0);
-      }
+      const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kst + r * 128 + (((4 * half + st) ^ swz8(r)) << 4));
+      s[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qfrag[0][st], s[0], 0, 0, 0);
+      s[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qfrag[1][st], s[1], 0, 0, 0);
     }
     if (tm.need) {
+      // The keys a row may see are one run of the tile, and for the anchor patterns also the frame-0
+      // specials: a bit mask per row, from which an element takes two instructions and neither branch nor
+      // lane mask. (Frame relations tested per element, with a multiply-high for the key's frame and a
+      // branch on the pattern, made 20 KB of code a tile, which ran at the speed of instruction
+      // fetches, 9.3 us a tile of 64 keys, now 2.4: block mix of 16 heads, 12 frames of 24 x 32
+      // patches 1371 -> 352 us, 16 x 16 patches, 4 frames 168 -> 51, 12 frames 474 -> 131.)
+      const bool own = tm.eff == SAF3R_FRAME_LOCAL || tm.eff == SAF3R_ANCHOR_LOCAL;
+      const bool any = !own && tm.eff != SAF3R_ANCHOR;  // no frame relation
+      const int base = tm.kt * 64, end = tm.kspecial ? min(g.S - base, 64) : tm.kvalid;
+      const uint64_t anc = tm.kspecial && !any && tm.eff != SAF3R_FRAME_LOCAL ? keys_below(min(g.ns - base, 64)) : 0;
 #pragma unroll
-      for (int kh = 0; kh < NKH; ++kh) {
+      for (int gq = 0; gq < 2; ++gq) {
+        int b = 0, e = end;
+        if (tm.kspecial && !any) {
+          b = frow[gq] * g.ns - base;
+          e = own ? min(b + g.ns, end) : b;
+        } else if (!tm.kspecial) {
+          const bool see = any || (own && tm.kframe == frow[gq]) || (tm.eff != SAF3R_FRAME_LOCAL && tm.kframe == 0);
+          if (!see) e = 0;
+        }
+        const uint32_t ok = (uint32_t)(((keys_below(e) & ~keys_below(b)) | anc) >> (32 * kh + 4 * half));
 #pragma unroll
         for (int a = 0; a < 16; ++a) {
-          const int key = key0 + 32 * kh + 8 * (a >> 2) + 4 * half + (a & 3);
-          bool ok;
-          int fc;
-          if (tm.kspecial) {
-            // frame = slot / ns as a multiply-high with ceil(2^32 / ns), exact below 2^32 / ns
-            // (magic 0: ns = 1)
-            const uint32_t sl = (uint32_t)(tm.kt * 64 + key);
-            ok = sl < (uint32_t)g.S;
-            fc = nsmagic ? (int)mulhi_u32(sl, nsmagic) : (int)sl;
-          } else {
-            ok = key < tm.kvalid;
-            fc = tm.kframe;
-          }
-#pragma unroll
-          for (int gq = 0; gq < 2; ++gq) {
-            bool okg = ok;
-            if (tm.eff == SAF3R_FRAME_LOCAL) okg = okg && fc == frow[gq];
-            else if (tm.eff == SAF3R_ANCHOR_LOCAL) okg = okg && (fc == 0 || fc == frow[gq]);
-            else if (tm.eff == SAF3R_ANCHOR) okg = okg && fc == 0;
-            if (!okg) s[kh][gq][a] = -__builtin_inff();
-          }
+          const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)ok, 8 * (a >> 2) + (a & 3), 1);
+          const float x = s[gq][a];  // (a vector element cannot be bit-cast in place)
+          s[gq][a] = __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, x) & m) | (~m & 0xFF800000u));
         }
       }
     }
@@ -207,45 +228,24 @@ __device__ __forceinline__ void attend(const char* __restrict__ kst, const char*
   hook();
   __builtin_amdgcn_sched_barrier(0);
 
-  // P = exp2(s*c - m*c) against the row's reference maximum m, and this tile's partial row sums.
-  // m is raised only when a tile's partial sum exceeds 2^64 (the first tile of a row with an
-  // unmasked key, whose m is still -inf, always does): values up to 2^64 keep every bf16 P, every
-  // fp32 sum and O finite, so no per-tile maximum is needed. The exact path then takes the tile's
-  // row maximum, rescales O and l, and recomputes P.
-  bf16x8 pf[2][2 * NKH];
+  // P = exp2(s*c - m*c) against the row's reference maximum m, and the partial row sums. m is raised
+  // only when a partial sum exceeds 2^64 (the first of a row with an unmasked key, whose m is still
+  // -inf, always does): values up to 2^64 keep every bf16 P, every fp32 sum and O finite, so no
+  // maximum is needed otherwise. The exact path then takes the row maximum, rescales O and l, and
+  // recomputes P. Row sums run over the bf16-rounded P that the PV product uses, so l and O agree.
+  // A row without a reference yet uses -2^127: unmasked keys then give +inf (and the exact path),
+  // masked keys 0, and no inf - inf (NaN) ever forms.
+  bf16x8 pf[2][2];
   float ts[2];
-  // row sums over the bf16-rounded P that the PV product uses, so l and O agree
-  const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
-  auto exps = [&](int gq, float mc) {
-    float t = 0.f;
 #pragma unroll
-    for (int j = 0; j < 2 * NKH; ++j) {
-      const int a0 = 8 * (j & 1);
-#pragma unroll
-      for (int u = 0; u < 8; u += 2) {
-        const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j >> 1][gq][a0 + u], c, -mc));
-        const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j >> 1][gq][a0 + u + 1], c, -mc));
-        const bf16x2 pr = {(__bf16)e0, (__bf16)e1};
-        pf[gq][j][u] = pr[0];
-        pf[gq][j][u + 1] = pr[1];
-        t = __builtin_amdgcn_fdot2_f32_bf16(pr, ones, t, false);
-      }
-    }
-    ts[gq] = t;
-  };
-  // a row without a reference yet uses -2^127: unmasked keys then give +inf (and the exact
-  // path), masked keys 0, and no inf - inf (NaN) ever forms
-#pragma unroll
-  for (int gq = 0; gq < 2; ++gq) exps(gq, A.m[gq] == -__builtin_inff() ? -0x1p127f : A.m[gq] * c);
+  for (int gq = 0; gq < 2; ++gq) ts[gq] = exps_half(s[gq], c, ref_mc(A.m[gq], c), pf[gq]);
   if (__ballot(ts[0] > 0x1p64f || ts[1] > 0x1p64f) != 0) {
     scores();
 #pragma unroll
     for (int gq = 0; gq < 2; ++gq) {
-      float mx = s[0][gq][0];
+      float mx = s[gq][0];
 #pragma unroll
-      for (int kh = 0; kh < NKH; ++kh)
-#pragma unroll
-        for (int a = 0; a < 16; ++a) mx = fmaxf(mx, s[kh][gq][a]);
+      for (int a = 0; a < 16; ++a) mx = fmaxf(mx, s[gq][a]);
       mx = partner_max(mx);
       const float m_new = fmaxf(A.m[gq], mx);
       const float alpha = A.m[gq] == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f((A.m[gq] - m_new) * c);
@@ -256,20 +256,19 @@ __device__ __forceinline__ void attend(const char* __restrict__ kst, const char*
         A.o[1][gq][a] *= alpha;
       }
       A.m[gq] = m_new;
-      exps(gq, m_new == -__builtin_inff() ? 0.f : m_new * c);
+      ts[gq] = exps_half(s[gq], c, m_new == -__builtin_inff() ? 0.f : m_new * c, pf[gq]);
     }
   }
   A.l[0] += ts[0];
   A.l[1] += ts[1];
 
 #pragma unroll
-  for (int j = 0; j < 2 * NKH; ++j) {
-    const int chn = 2 * j + half;
+  for (int j = 0; j < 2; ++j) {
+    const int chn = 2 * (2 * kh + j) + half;
 #pragma unroll
     for (int dh = 0; dh < 2; ++dh) {
       const int r = 32 * dh + col;
-      const bf16x8 vf = NKH == 2 ? *reinterpret_cast<const bf16x8*>(vst + r * 128 + ((chn ^ swz8(r)) << 4))
-                                 : *reinterpret_cast<const bf16x8*>(vst + r * 64 + ((chn ^ swz4(r)) << 4));
+      const bf16x8 vf = *reinterpret_cast<const bf16x8*>(vst + r * 128 + ((chn ^ swz8(r)) << 4));
       A.o[dh][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[0][j], A.o[dh][0], 0, 0, 0);
       A.o[dh][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[1][j], A.o[dh][1], 0, 0, 0);
     }
@@ -307,27 +306,6 @@ __device__ __forceinline__ void mask_valid(f32x16 (&s)[2], int kvalid, int key0,
     const int key = key0 + 8 * (a >> 2) + 4 * half + (a & 3);
     if (key >= kvalid) s[0][a] = s[1][a] = -__builtin_inff();
   }
-}
-
-// a row without a reference maximum yet uses -2^127: unmasked keys then give +inf (and the exact
-// path), masked keys 0, and no inf - inf (NaN) ever forms
-__device__ __forceinline__ float ref_mc(float m, float c) { return m == -__builtin_inff() ? -0x1p127f : m * c; }
-
-// P = exp2(s*c - mc) of one query group's 16 keys and their partial row sum over the bf16-rounded
-// values the PV product uses (exact path)
-__device__ __forceinline__ float exps_half(const f32x16& s, float c, float mc, bf16x8 (&p)[2]) {
-  const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
-  float t = 0.f;
-#pragma unroll
-  for (int u = 0; u < 16; u += 2) {
-    const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u], c, -mc));
-    const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u + 1], c, -mc));
-    const bf16x2 pr = {(__bf16)e0, (__bf16)e1};
-    p[u >> 3][u & 7] = pr[0];
-    p[u >> 3][(u & 7) + 1] = pr[1];
-    t = __builtin_amdgcn_fdot2_f32_bf16(pr, ones, t, false);
-  }
-  return t;
 }
 
 // The block of half step h: O += V(h-1) P(h-1), sn = K(h+1) Q^T, pn = P(h) from s with row sums ts.
@@ -760,7 +738,8 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
   asm volatile("" : "+s"(qtq));
 #pragma unroll
   for (int gq = 0; gq < 2; ++gq) {
-    const u32x4* qsrc = reinterpret_cast<const u32x4*>(qrows + ((int64_t)qtq * 64 + 32 * gq + col) * 64 + 32 * half);
+    const char* qb = reinterpret_cast<const char*>(qrows + ((int64_t)qtq * 64 + 32 * gq) * 64);
+    const u32x4* qsrc = reinterpret_cast<const u32x4*>(qb + (uint32_t)(col * 128 + 64 * half));
 #pragma unroll
     for (int s = 0; s < 4; ++s) qfrag[gq][s] = __builtin_bit_cast(bf16x8, qsrc[s]);
   }
@@ -807,10 +786,7 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
       }
       store(A);
     };
-    // ---- key-tile sequence (uniform) ----
-    Walk wk;
-    bool frame_rel = false, rel_patch = false;
-    int seg_s = 0, seg_l = 0;  // own-frame patch tiles of a frame-relative patch-row item
+    // ---- single-range part of the walk (uniform): cnt tiles from sbeg on ----
     constexpr bool keyset = decltype(ks_tag)::value;
     const int eff = (pat == SAF3R_DENSE || pat == SAF3R_TOKEN_DYNAMIC || pat == SAF3R_BLOCK_DYNAMIC || keyset)
                         ? SAF3R_DENSE
@@ -826,59 +802,37 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
     // framed heads: frame 0's tiles (ANCHOR, and first for ANCHOR_LOCAL), then the query frame's
     // (FRAME_LOCAL, and ANCHOR_LOCAL from frame 1 on), each frame NBT tiles with only its last partial
     const bool two = framed && pat == SAF3R_ANCHOR_LOCAL && qf != 0;
+    // frame-relative heads in the packed layout: a patch-row item (one frame) walks its own frame's patch
+    // tiles here and the other ranges in the frame-relative walk, which serves the other items alone
+    const bool frame_rel = !keyset && eff != SAF3R_DENSE && !framed;
+    const bool rel_patch = frame_rel && qt0 >= g.nst && pat != SAF3R_ANCHOR;
+    int sbeg = 0, cnt;
     if constexpr (keyset) {
-      wk.init(0, (ks_keys + 63) / 64, 0, 0, 0, 0, 0, 0);
+      cnt = (ks_keys + 63) / 64;
     } else if (eff == SAF3R_DENSE) {
-      wk.init(0, g.NT, 0, 0, 0, 0, 0, 0);
+      cnt = g.NT;
     } else if (framed) {
-      wk.init(pat == SAF3R_FRAME_LOCAL ? qf * g.NBT : 0, g.NBT, two ? qf * g.NBT : 0, two ? g.NBT : 0, 0, 0, 0, 0);
+      sbeg = pat == SAF3R_FRAME_LOCAL ? qf * g.NBT : 0;
+      cnt = two ? 2 * g.NBT : g.NBT;
     } else {
-      frame_rel = true;
-      int f0, f1;
-      if (qt0 < g.nst) {
-        const int last = min(g.S, (qt0 + nw) * 64) - 1;
-        f0 = (qt0 * 64) / g.ns;
-        f1 = last / g.ns;
-      } else {
-        f0 = f1 = (qt0 - g.nst) / g.NBf;
-      }
-      const bool need_anchor = (pat == SAF3R_ANCHOR_LOCAL || pat == SAF3R_ANCHOR);
-      const bool need_local = (pat != SAF3R_ANCHOR);
-      const bool has_sp = g.ns > 0;
-      const int ls0 = has_sp ? (f0 * g.ns) / 64 : 0;
-      const int ls1 = has_sp ? ((f1 + 1) * g.ns - 1) / 64 : -1;
-      const bool anc_sp = has_sp && need_anchor && !(need_local && ls0 == 0);
-      const bool anc_pt = need_anchor && !(need_local && f0 == 0);
-      // ranges: frame 0's special tiles, the item's frames' special tiles, frame 0's patch tiles,
-      // the item's frames' patch tiles. A patch-row item (one frame) walks its own frame's patch
-      // tiles (only the last one partial) in the pipelined single-range walk and the other ranges
-      // here, with per-key frame masks.
-      rel_patch = qt0 >= g.nst && need_local;
-      wk.init(0, anc_sp ? (g.ns - 1) / 64 + 1 : 0,
-              ls0, (has_sp && need_local) ? ls1 - ls0 + 1 : 0,
-              g.nst, anc_pt ? g.NBf : 0,
-              g.nst + f0 * g.NBf, need_local && !rel_patch ? (f1 - f0 + 1) * g.NBf : 0);
-      if (rel_patch) {
-        seg_s = __builtin_amdgcn_readfirstlane(g.nst + f0 * g.NBf);
-        seg_l = __builtin_amdgcn_readfirstlane(g.NBf);
-      }
+      sbeg = g.nst + (qt0 - g.nst) / g.NBf * g.NBf;
+      cnt = g.NBf;
     }
-    const int count = wk.count;
+    sbeg = __builtin_amdgcn_readfirstlane(sbeg);
+    cnt = __builtin_amdgcn_readfirstlane(cnt);
     int rot = 0;
-    const bool paced = eff == SAF3R_DENSE && p.phase_dense > 0 && count > 0;
+    const bool paced = eff == SAF3R_DENSE && p.phase_dense > 0 && cnt > 0;
     if (paced) {
       // one clock reading per work-group: the four waves share the ring and must agree; the start
       // time waits in LDS for the pace update at the end (no registers held through the walk)
       if (tid == 0) {
         const uint64_t t = __builtin_amdgcn_s_memrealtime();
         t_start = t;
-        wcnt[0] = (int)((t / pace_phase(p, 0)) % (uint64_t)count);
+        wcnt[0] = (int)((t / pace_phase(p, 0)) % (uint64_t)cnt);
       }
       __syncthreads();
       rot = __builtin_amdgcn_readfirstlane(wcnt[0]);  // an LDS value, uniform: keep the walk scalar
     }
-    if (count > 0) wk.seek(rot, g);
-    Walk wi = wk;  // the tiles to load run two steps ahead of the tiles consumed
 
     // thread tid owns 16-byte chunks tid and tid + 256 of the K and the V tile (64 rows of 128 B,
     // same offsets for both); LDS chunk position P holds row P/8, global chunk (P % 8) ^ swz8(row)
@@ -902,23 +856,7 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
         vbase = reinterpret_cast<const char*>(p.vc + (int64_t)p.slot[h] * p.ks_cap * 64);
       }
     }
-    auto issue = [&](int stage) {
-      const char* kb = kbase + (int64_t)wi.kt * 8192;
-      const char* vb = vbase + (int64_t)wi.kt * 8192;
-      char* st = ring + stage * 16384 + 64 * w * 16;
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        uint32_t o = dofs;
-        const char* bk = kb + 4096 * u;
-        const char* bv = vb + 4096 * u;
-        asm volatile("" : "+v"(o), "+s"(bk), "+s"(bv));  // scalar-base address form (see split mode)
-        __builtin_amdgcn_global_load_lds((const void*)(bk + o), (lds_void*)(st + 4096 * u), 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((const void*)(bv + o), (lds_void*)(st + 8192 + 4096 * u), 16, 0, 0);
-      }
-      wi.next(g);
-    };
-
-    if (keyset || eff == SAF3R_DENSE || rel_patch || framed) {
+    if (!frame_rel || rel_patch) {
       // ---- single-range walk: tiles rot, rot + 1, ... (mod count), only partial tiles masked ----
       // (dense and key-set walks: tiles 0 .. count-1 entered at rot; patch-row items of
       // frame-relative heads: their own frame's patch tiles, then the frame-relative walk below)
@@ -929,11 +867,9 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
       // (framed heads: no special tiles, NBT tiles per frame, T - 64 (NBT - 1) valid keys in the last)
       const int nst = framed ? 0 : g.nst, NBf = framed ? g.NBT : g.NBf;
       const int lastv = framed ? g.T - 64 * (NBf - 1) : g.P - 64 * (NBf - 1);  // valid keys, last tile of a frame
-      const int sbeg = rel_patch ? seg_s : framed ? wk.s0 : 0;
-      const int cnt = rel_patch ? seg_l : count;
       // the tile after which the walk continues at jto: the end of the range (wrapping to its start),
       // or for a framed two-frame walk the end of frame 0 (continuing at the query frame)
-      const int jfrom = two ? g.NBT : sbeg + cnt, jto = two ? wk.s1 : sbeg;
+      const int jfrom = two ? g.NBT : sbeg + cnt, jto = two ? qf * g.NBT : sbeg;
       int kt = (rel_patch || framed) ? sbeg : rot, bk = -1;  // consumed tile and its block within its frame
       if constexpr (!keyset) bk = kt >= nst ? (kt - nst) % NBf : -1;
       auto kvalid_of = [&]() -> int {
@@ -1012,7 +948,9 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
           barrier_only();
           if (t + 3 < cnt) issue_at((v + 3) & 3);
           // half step 2t+1: PV of tile t keys 0..31, scores of tile t + 1 keys 0..31
-          load_v(ring + v * 16384 + 8192, 0, vf, half, col);
+          int vcol = col;  // without FAST the loop is one register short: the V rows' offset is found anew
+          if constexpr (!FAST) asm volatile("" : "+v"(vcol));
+          load_v(ring + v * 16384 + 8192, 0, vf, half, vcol);
           load_k(ring + ((v + 1) & 3) * 16384, 0, kf, half, col);
           half_block<FAST>(kf, vf, qfrag, s_nxt, s_cur, pn, pc, ts, A, c);
           if (kv_nxt < 64) mask_valid(s_cur, kv_nxt, 0, half);
@@ -1049,6 +987,50 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
     }
 
     // ---- frame-relative walks (up to four ranges, frame masks): one tile per attend step ----
+    // the ranges: frame 0's special tiles, the item's frames' special tiles, frame 0's patch tiles, the
+    // item's frames' patch tiles (of a patch-row item walked above). Found here, not before the walk
+    // above, whose loops have no scalar registers to spare for them (qt0 through an empty asm, so that
+    // nothing is hoisted there)
+    int q0 = qt0, hl = half, cl = col;
+    asm volatile("" : "+s"(q0), "+v"(hl), "+v"(cl));
+    int f0, f1;
+    if (q0 < g.nst) {
+      f0 = q0 * 64 / g.ns;
+      f1 = (min(g.S, (q0 + nw) * 64) - 1) / g.ns;
+    } else {
+      f0 = f1 = (q0 - g.nst) / g.NBf;
+    }
+    const bool need_anchor = (pat == SAF3R_ANCHOR_LOCAL || pat == SAF3R_ANCHOR);
+    const bool need_local = (pat != SAF3R_ANCHOR);
+    const bool has_sp = g.ns > 0;
+    const int ls0 = has_sp ? (f0 * g.ns) / 64 : 0;
+    const int ls1 = has_sp ? ((f1 + 1) * g.ns - 1) / 64 : -1;
+    const bool anc_sp = has_sp && need_anchor && !(need_local && ls0 == 0);
+    const bool anc_pt = need_anchor && !(need_local && f0 == 0);
+    Walk wk;
+    wk.init(0, anc_sp ? (g.ns - 1) / 64 + 1 : 0,
+            ls0, (has_sp && need_local) ? ls1 - ls0 + 1 : 0,
+            g.nst, anc_pt ? g.NBf : 0,
+            g.nst + f0 * g.NBf, need_local && q0 < g.nst ? (f1 - f0 + 1) * g.NBf : 0);
+    const int count = wk.count;
+    if (count > 0) wk.seek(0, g);
+    Walk wi = wk;  // the tiles to load run two steps ahead of the tiles consumed
+    auto issue = [&](int stage) {
+      const char* kb = kbase + (int64_t)wi.kt * 8192;
+      const char* vb = vbase + (int64_t)wi.kt * 8192;
+      char* st = ring + stage * 16384 + 64 * w * 16;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        uint32_t o = dofs;
+        const char* bk = kb + 4096 * u;
+        const char* bv = vb + 4096 * u;
+        asm volatile("" : "+v"(o), "+s"(bk), "+s"(bv));  // scalar-base address form (see split mode)
+        __builtin_amdgcn_global_load_lds((const void*)(bk + o), (lds_void*)(st + 4096 * u), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void*)(bv + o), (lds_void*)(st + 8192 + 4096 * u), 16, 0, 0);
+      }
+      wi.next(g);
+    };
+
     int64_t qtok_unused[2];
     int frow[2];
     row_info(qtok_unused, frow);
@@ -1068,11 +1050,13 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         if (n + u < count) {
-          const TileMask tm = wk.mask(g, eff, frame_rel, qspecial);
+          const TileMask tm = wk.mask(g, eff, true, qspecial);
           const char* kst = ring + ((n + u) % kStages) * 16384;
-          attend<2>(kst, kst + 8192, qfrag, A, frow, tm, g, p.nsmagic, 0, half, col, c, [&]() {
-            if (n + 2 + u < count) issue((n + 2 + u) % kStages);
-          });
+#pragma unroll 1
+          for (int kh = 0; kh < 2; ++kh)
+            attend(kst, kst + 8192, qfrag, A, frow, tm, g, kh, hl, cl, c, [&]() {
+              if (kh == 0 && n + 2 + u < count) issue((n + 2 + u) % kStages);
+            });
           wk.next(g);
         }
       }
@@ -1396,7 +1380,7 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
 }
 
 // Launches without split walks keep a kernel of their own: with the split walks' code in it the compiler
-// spills 28 bytes a lane instead of 20, which a layer of 48 x 1301 tokens and 24 heads took 3 % longer with
+// spilled 28 bytes a lane instead of 20, which a layer of 48 x 1301 tokens and 24 heads took 3 % longer with
 // (9.76 -> 10.10 ms), one of 32 x 1374 tokens 1.4 % (1.85 -> 1.88 ms).
 template <bool SPLIT>
 __global__ __launch_bounds__(256, 2) void sparse_attn_kernel(AttnParams p) {
@@ -1524,7 +1508,8 @@ static int head_segments(int h, int pat, bool tokord, bool framed, bool split, i
 // as far as that falls by 5 % and a split item's fixed part. Launches that fill the chip split nothing
 // (the fixed part of every item adds to their work), nor do heads of many short walks.
 // Measured, attention and fixup, us, nothing split / this rule / every walk split: seeded block mix of 16
-// heads, 1041-token frames, 2 frames 62 / 40 / 41, 4 105 / 64 / 70, 8 192 / 145 / 160, 12 294 / 250 / 280;
+// heads, 1041-token frames, 2 frames 62 / 40 / 41, 4 105 / 64 / 70, 8 192 / 145 / 160, 12 294 / 250 / 280 (this
+// rule 35, 55, 134 and 245 since the masked walk's code is smaller);
 // profile layer 11 (dino special rows), 4 frames 96 / 57 / 64; layers 3, 9, 20 (anchor and key-set
 // heads), 4 frames 44 / 44 / 59, 64 / 63 / 70, 65 / 64 / 74. The sum of the two instead of the larger split
 // dense heads of full launches: 32 x 1374 tokens 1870 -> 2010, 128 x 1374 25100 -> 27970.
@@ -1685,7 +1670,6 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   if (p.g.ns > 0 && (uint64_t)p.g.Sp * (uint64_t)p.g.ns >= 0x100000000ull)
     return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_sparse_attn_fwd: too many special tokens");
   // ceil(2^32 / ns) fits 32 bits for ns >= 2 only: ns = 1 is magic 0, which the kernel tests for
-  p.nsmagic = p.g.ns > 1 ? (uint32_t)((0x100000000ull + (uint64_t)p.g.ns - 1) / (uint64_t)p.g.ns) : 0u;
   if (flags & ~SAF3R_ATTN_FIXED_ORDER) return fail(SAF3R_ERR_INVALID, "saf3r_sparse_attn_fwd: unknown flags 0x%x", flags);
   if ((uintptr_t)pace % 8) return fail(SAF3R_ERR_INVALID, "saf3r_sparse_attn_fwd: pace must be 8-byte aligned");
   const bool fixed = (flags & SAF3R_ATTN_FIXED_ORDER) != 0;
@@ -1746,8 +1730,8 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   }
   p.item_start[p.n_order] = (int)total;
   if (total == 0) return SAF3R_OK;
-  hipLaunchKernelGGL(p.split ? sparse_attn_kernel<true> : sparse_attn_kernel<false>, dim3((unsigned)total), dim3(256), 0,
-                     (hipStream_t)stream, p);
+  auto kernel = p.split ? sparse_attn_kernel<true> : sparse_attn_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(256), 0, (hipStream_t)stream, p);
   if (int e = check_launch("saf3r_sparse_attn_fwd")) return e;
   // the exact walk of the items that left the FAST range: the same items of the prescaled heads,
   // in the fixed order; every other item returns after reading its marker
@@ -1768,7 +1752,7 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   if (ftotal == 0) return SAF3R_OK;
   f.n_items = (int)ftotal;
   f.fix_groups = (int)std::min<int64_t>(ftotal, 2 * (int64_t)cus);  // one resident round
-  hipLaunchKernelGGL(f.split ? sparse_attn_fixup_kernel<true> : sparse_attn_fixup_kernel<false>,
-                     dim3((unsigned)f.fix_groups), dim3(256), 0, (hipStream_t)stream, f);
+  auto fixup = p.split ? sparse_attn_fixup_kernel<true> : sparse_attn_fixup_kernel<false>;
+  hipLaunchKernelGGL(fixup, dim3((unsigned)f.fix_groups), dim3(256), 0, (hipStream_t)stream, f);
   return check_launch("saf3r_sparse_attn_fwd");
 }
