@@ -1007,9 +1007,11 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
     const int ls1 = has_sp ? ((f1 + 1) * g.ns - 1) / 64 : -1;
     const bool anc_sp = has_sp && need_anchor && !(need_local && ls0 == 0);
     const bool anc_pt = need_anchor && !(need_local && f0 == 0);
+    const int na = anc_sp ? (g.ns - 1) / 64 + 1 : 0;
+    const int sp0 = max(ls0, na);  // the ranges may meet (ns > 64): a tile both hold is walked once, with both masks
     Walk wk;
-    wk.init(0, anc_sp ? (g.ns - 1) / 64 + 1 : 0,
-            ls0, (has_sp && need_local) ? ls1 - ls0 + 1 : 0,
+    wk.init(0, na,
+            sp0, (has_sp && need_local) ? ls1 - sp0 + 1 : 0,
             g.nst, anc_pt ? g.NBf : 0,
             g.nst + f0 * g.NBf, need_local && q0 < g.nst ? (f1 - f0 + 1) * g.NBf : 0);
     const int count = wk.count;

@@ -18,7 +18,7 @@ ATOL_MAX, ATOL_MEAN = 2e-2, 2e-3
 
 @pytest.mark.parametrize("prescaled", [False, True])
 @pytest.mark.parametrize("F,T,ns", [(13, 69, 5), (30, 69, 5), (64, 65, 1), (4, 80, 16), (2, 128, 64), (2, 193, 128),
-                                    (1, 133, 5), (5, 261, 5)])
+                                    (1, 133, 5), (5, 261, 5), (3, 129, 65), (3, 200, 70), (4, 130, 66)])
 def test_packed_frame_relative(pkg, F, T, ns, prescaled):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
