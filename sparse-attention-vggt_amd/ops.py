@@ -91,7 +91,10 @@ def _need_cuda(*ts):
 # pass the same few tables in every forward.
 @lru_cache(maxsize=1024)
 def _i32_values(vals: tuple):
-    return (ctypes.c_int32 * len(vals))(*[int(v) for v in vals])
+    vals = [int(v) for v in vals]
+    if any(not -2 ** 31 <= v < 2 ** 31 for v in vals):  # (ctypes would keep the low 32 bits)
+        raise RuntimeError(f"{vals}: not int32 values")
+    return (ctypes.c_int32 * len(vals))(*vals)
 
 
 @lru_cache(maxsize=1024)
