@@ -88,10 +88,10 @@ def _need_cuda(*ts):
 
 
 # Host arrays of per-head values, by their values: the C entries only read them, and a model's layers
-# pass the same few tables in every forward.
+# pass the same few tables in every forward. Callers turn elements into Python numbers first: a 0-dim tensor
+# is a key by its identity, under which its value can change.
 @lru_cache(maxsize=1024)
 def _i32_values(vals: tuple):
-    vals = [int(v) for v in vals]
     if any(not -2 ** 31 <= v < 2 ** 31 for v in vals):  # (ctypes would keep the low 32 bits)
         raise RuntimeError(f"{vals}: not int32 values")
     return (ctypes.c_int32 * len(vals))(*vals)
@@ -101,12 +101,11 @@ def _i32_values(vals: tuple):
 def _flag_values(flags: tuple, n: int):
     if len(flags) != n:
         raise ValueError(f"one flag per head: got {len(flags)} for {n} heads")
-    return (ctypes.c_uint8 * n)(*[1 if f else 0 for f in flags])
+    return (ctypes.c_uint8 * n)(*flags)
 
 
 @lru_cache(maxsize=1024)
 def _layout_values(layouts: tuple, n: int):
-    layouts = [int(x) for x in layouts]
     if len(layouts) != n:
         raise ValueError(f"one layout per head: got {len(layouts)} for {n} heads")
     if any(x not in (LAYOUT_PACKED, LAYOUT_TOKEN, LAYOUT_FRAMED) for x in layouts):
@@ -122,17 +121,17 @@ def _pattern_counts(patterns: tuple) -> tuple[int, int, int]:
 
 
 def _i32_array(vals: Sequence[int]):
-    return _i32_values(tuple(vals))
+    return _i32_values(tuple(map(int, vals)))
 
 
 def _u8_flags(flags: Sequence[bool] | None, n: int):
     """Host uint8 [n] flag array for the C ABI (None: no array)."""
-    return None if flags is None else _flag_values(tuple(flags), n)
+    return None if flags is None else _flag_values(tuple(map(bool, flags)), n)
 
 
 def _u8_layouts(layouts: Sequence[int] | None, n: int):
     """Host uint8 [n] array of per-head layouts (``LAYOUT_*``; True counts as ``LAYOUT_TOKEN``)."""
-    return None if layouts is None else _layout_values(tuple(layouts), n)
+    return None if layouts is None else _layout_values(tuple(map(int, layouts)), n)
 
 
 FRAMED_PATTERNS = (FRAME_LOCAL, ANCHOR_LOCAL, ANCHOR)  # heads that can take the framed layout
@@ -404,7 +403,7 @@ def sparse_attn_fwd(qp, kp, vp, geom: Geometry, patterns: Sequence[int], sel: to
         raise ValueError(f"out must be bf16 [N, >= H*64] with unit column stride, got {tuple(out.shape)}")
     scale = 1.0 / math.sqrt(HEAD_DIM) if scale is None else scale
     width = 0
-    patterns = tuple(patterns)
+    patterns = tuple(map(int, patterns))
     n_dyn, n_ks, n_bc = _pattern_counts(patterns)
     if n_dyn:
         if sel is None:

@@ -19,3 +19,34 @@ def test_int32_lists_refuse_what_does_not_fit(ops, pkg, bad):
         geom = pkg.Geometry(2, 20, 5)
         with pytest.raises(RuntimeError, match="int32"):
             ops.keyset_build([ops.KeySetSpec(0, ops.KEYSET_STRIDE, bad)], geom, None, "cpu")
+
+
+def test_lists_of_tensors_are_read_each_time(ops):
+    """Elements that can change under the same identity (0-dim tensors) are read in every call, and not held."""
+    import torch
+    t = torch.tensor([3, 1])
+    vals = [t[0], t[1]]
+    assert list(ops._i32_array(vals)) == [3, 1]
+    assert list(ops._u8_flags(vals, 2)) == [1, 1]
+    assert list(ops._u8_layouts([t[1], t[1]], 2)) == [1, 1]
+    same = [vals[1], vals[1]]
+    assert list(ops._u8_layouts(same, 2)) == [1, 1]
+    t[0], t[1] = 5, 0
+    assert list(ops._i32_array(vals)) == [5, 0]
+    assert list(ops._u8_flags(vals, 2)) == [1, 0]
+    assert list(ops._u8_layouts(same, 2)) == [0, 0]
+
+
+def test_pattern_tensors_are_read_each_time(ops, pkg, monkeypatch):
+    """The head counts that ``sparse_attn_fwd`` checks come from the patterns of the call."""
+    import torch
+    geom = pkg.Geometry(1, 20, 5)
+    qp, kp, vp = ops.packed_buffers(geom, 1, "cpu")
+    monkeypatch.setattr(ops, "_need_cuda", lambda *a: None)
+    t = torch.tensor([ops.DENSE])
+    pat = [t[0]]
+    ops._pattern_counts.cache_clear()
+    for p, what in ((ops.BLOCK_DYNAMIC, "selection list"), (ops.KEYSET, "key-set heads"), (ops.BROADCAST, "broadcast")):
+        t[0] = p
+        with pytest.raises(ValueError, match=what):
+            ops.sparse_attn_fwd(qp, kp, vp, geom, pat)
