@@ -46,7 +46,7 @@ def test_pattern_tensors_are_read_each_time(ops, pkg, monkeypatch):
     t = torch.tensor([ops.DENSE])
     pat = [t[0]]
     ops._pattern_counts.cache_clear()
-    for p, what in ((ops.BLOCK_DYNAMIC, "selection list"), (ops.KEYSET, "key-set heads"), (ops.BROADCAST, "broadcast")):
+    for p, what in ((ops.BLOCK_DYNAMIC, "selection list"), (ops.KEYSET, "key-set heads"), (ops.BROADCAST, "BROADCAST")):
         t[0] = p
         with pytest.raises(ValueError, match=what):
             ops.sparse_attn_fwd(qp, kp, vp, geom, pat)
