@@ -78,7 +78,8 @@ class Geometry:
         return self.frames * self.frame_tiles * BLOCK <= self.slots
 
 
-@lru_cache(maxsize=64)
+@lru_cache(maxsize=64, typed=True)
 def _geometry(cls, frames: int, tokens_per_frame: int, num_special: int) -> Geometry:
-    """Geometries of a model's forwards: one object per size, whose derived counts are computed once."""
+    """Geometries of a model's forwards: one object per size, whose derived counts are computed once (typed: 2.0
+    frames are not the 2 frames of another call)."""
     return cls(frames, tokens_per_frame, num_special)

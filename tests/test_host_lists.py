@@ -50,3 +50,15 @@ def test_pattern_tensors_are_read_each_time(ops, pkg, monkeypatch):
         t[0] = p
         with pytest.raises(ValueError, match=what):
             ops.sparse_attn_fwd(qp, kp, vp, geom, pat)
+
+
+def test_geometry_of_one_type_is_not_kept_for_another(pkg):
+    """Geometries are shared by size; sizes of another type (which the C entries refuse) must not become those of a
+    later call with the same integers."""
+    a = pkg.Geometry.from_tokens(2 * 1043.0, 1043.0)
+    b = pkg.Geometry.from_tokens(2 * 1043, 1043)
+    c = pkg.Geometry.from_tokens(2 * 1043, 1043, True)
+    d = pkg.Geometry.from_tokens(2 * 1043, 1043, 1)
+    assert isinstance(a.frames, float) and c.num_special is True
+    assert [type(x) for g in (b, d) for x in (g.frames, g.tokens_per_frame, g.num_special, g.slots)] == [int] * 8
+    assert b is pkg.Geometry.from_tokens(2 * 1043, 1043)
