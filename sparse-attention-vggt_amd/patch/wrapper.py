@@ -208,8 +208,9 @@ class BaseHeadwiseSparseAttentionWrapper(nn.Module):
             if len(ratios) == 1 and len(probe_rows) == len(specs):
                 _, scores = ops.probe_scores(qk32, [self.fp32_slot[specs[i].head] for i in probe_rows],
                                              sample=ops.probe_sample(geom.tokens, ratios[0]))
-            else:  # one call per sample ratio; rows of stride heads are not read
-                scores = torch.empty(len(specs), geom.tokens, dtype=torch.float32, device=kp.device)
+            else:  # one call per sample ratio; rows of stride heads are not read, and stay zeros in ks.scores
+                new = torch.empty if len(probe_rows) == len(specs) else torch.zeros
+                scores = new(len(specs), geom.tokens, dtype=torch.float32, device=kp.device)
                 for r in ratios:
                     rows_r = [i for i in probe_rows if specs[i].sample_ratio == r]
                     ops.probe_scores(qk32, [self.fp32_slot[specs[i].head] for i in rows_r],
