@@ -658,15 +658,19 @@ def probe_scores(qk32: torch.Tensor, slots: Sequence[int], scale: float | None =
     N = qk32.shape[2]
     n = len(slots)
     dev = qk32.device
-    slots = list(slots)
-    rows = list(range(n)) if rows is None else list(rows)
+    slots = [int(s) for s in slots]
+    rows = list(range(n)) if rows is None else [int(r) for r in rows]
+    if any(not 0 <= s < qk32.shape[0] for s in slots):
+        raise ValueError(f"slots {slots} of {qk32.shape[0]}")
+    if len(rows) != n or any(r < 0 for r in rows) or (out is not None and any(r >= out.shape[0] for r in rows)):
+        raise ValueError(f"rows {rows}: one per slot, inside out")
     qbar = torch.empty(n, HEAD_DIM, dtype=torch.float32, device=dev)
     if out is None:
         scores = torch.empty(max(rows) + 1 if rows else 0, N, dtype=torch.float32, device=dev)
     else:
         scores = out
         if (out.dtype != torch.float32 or out.dim() != 2 or not out.is_contiguous() or out.shape[1] < N
-                or (rows and max(rows) >= out.shape[0])):
+                or out.device != dev):
             raise ValueError("out must be contiguous fp32 [> max(rows), >= N]")
     scale = 1.0 / math.sqrt(HEAD_DIM) if scale is None else scale
     if sample is not None:

@@ -62,3 +62,26 @@ def test_geometry_of_one_type_is_not_kept_for_another(pkg):
     assert isinstance(a.frames, float) and c.num_special is True
     assert [type(x) for g in (b, d) for x in (g.frames, g.tokens_per_frame, g.num_special, g.slots)] == [int] * 8
     assert b is pkg.Geometry.from_tokens(2 * 1043, 1043)
+
+
+def test_probe_scores_checks_its_rows_and_output(ops, monkeypatch):
+    """Output rows, one per slot and inside ``out``, are checked before anything is launched."""
+    import torch
+    monkeypatch.setattr(ops, "_need_cuda", lambda *a: None)
+    qk32, out = torch.zeros(3, 2, 10, 64), torch.zeros(4, 10)
+
+    def refused(match, **kw):
+        with pytest.raises(ValueError, match=match):
+            ops.probe_scores(qk32, [2, 0], **kw)
+    refused("rows", out=out, rows=[1])          # the kernels read a row per slot
+    refused("rows", out=out, rows=[1, 2, 3])
+    refused("rows", out=out, rows=[1, -1])
+    refused("rows", rows=[-1, 0])
+    refused("rows", out=out, rows=[1, 4])
+    refused("rows", out=torch.zeros(1, 10))     # no rows given: 0 and 1
+    refused("out", out=torch.zeros(4, 10, device="meta"), rows=[0, 1])  # another device's memory
+    refused("out", out=out.t().contiguous().t(), rows=[0, 1])
+    refused("out", out=torch.zeros(4, 9), rows=[0, 1])
+    for slots in ([0, 3], [-1, 0]):
+        with pytest.raises(ValueError, match="slots"):
+            ops.probe_scores(qk32, slots)
