@@ -720,6 +720,8 @@ def keyset_build(specs: Sequence[KeySetSpec], geom: Geometry, scores: torch.Tens
     n = len(specs)
     if any(s.param <= 0 for s in specs):
         raise ValueError("key-set stride / k must be positive")
+    if scores is None and any(s.mode == KEYSET_TOPK for s in specs):
+        raise ValueError("top-k key sets need scores")
     lists = [[s.mode for s in specs], [s.param for s in specs], [s.start for s in specs],
              [int(bool(s.include)) for s in specs]]
     idx = torch.empty(n, geom.tokens, dtype=torch.int32, device=device)
@@ -730,8 +732,7 @@ def keyset_build(specs: Sequence[KeySetSpec], geom: Geometry, scores: torch.Tens
             raise ValueError("scores must be fp32 [n_specs, >= N]")
         scores = scores.contiguous()
     _mark("keyset_build", "start")
-    # (top-k heads without scores keep the device-list entry's behaviour)
-    if n <= MAX_HEADS and (scores is not None or KEYSET_TOPK not in lists[0]):
+    if n <= MAX_HEADS:
         entry, args = lib.saf3r_keyset_build_host, [_i32_array(x) for x in lists]
     else:
         arr = torch.tensor(lists, dtype=torch.int32, device=device)

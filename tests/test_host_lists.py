@@ -85,3 +85,13 @@ def test_probe_scores_checks_its_rows_and_output(ops, monkeypatch):
     for slots in ([0, 3], [-1, 0]):
         with pytest.raises(ValueError, match="slots"):
             ops.probe_scores(qk32, slots)
+
+
+def test_topk_key_sets_need_scores(ops, pkg):
+    """Refused on the host: the kernel reads a score row for every top-k head."""
+    geom = pkg.Geometry(2, 20, 5)
+    stride = ops.KeySetSpec(0, ops.KEYSET_STRIDE, 3)
+    for specs in ([ops.KeySetSpec(0, ops.KEYSET_TOPK, 3)], [stride, ops.KeySetSpec(1, ops.KEYSET_TOPK, 3)],
+                  [stride] * 70 + [ops.KeySetSpec(1, ops.KEYSET_TOPK, 3)]):
+        with pytest.raises(ValueError, match="scores"):
+            ops.keyset_build(specs, geom, None, "cpu")
