@@ -23,7 +23,10 @@ int fail(int code, const char* fmt, ...) {
 int injected(const char* entry) {
   const char* e = getenv("SAF3R_FAULT_INJECT");
   if (e == nullptr || e[0] == '\0') return SAF3R_OK;
-  if (strcmp(e, "all") == 0 || strcmp(e, entry) == 0)
+  // an entry's name also names its host-list and typed-parameter forms
+  const size_t n = strlen(e);
+  const bool form = strncmp(e, entry, n) == 0 && (strcmp(entry + n, "_host") == 0 || strcmp(entry + n, "_typed") == 0);
+  if (strcmp(e, "all") == 0 || strcmp(e, entry) == 0 || form)
     return fail(SAF3R_ERR_INJECTED, "%s: failure injected through SAF3R_FAULT_INJECT", entry);
   return SAF3R_OK;
 }

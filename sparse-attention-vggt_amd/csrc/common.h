@@ -91,8 +91,8 @@ constexpr int kPoolGroup = 16;
 // ---------------------------------------------------------------------------------------
 void set_error(const char* fmt, ...);
 int fail(int code, const char* fmt, ...);
-// Returns SAF3R_ERR_INJECTED when the environment variable SAF3R_FAULT_INJECT names `entry`
-// (or is "all"); used by the error-path tests to force a failure before any launch.
+// Returns SAF3R_ERR_INJECTED when the environment variable SAF3R_FAULT_INJECT names `entry`, or the
+// entry that it is the _host or _typed form of (or is "all"); used by the error-path tests to force a failure before any launch.
 int injected(const char* entry);
 int check_launch(const char* what);
 
