@@ -88,12 +88,14 @@ def load():
         "saf3r_keyset_gather_host": ([p, i32, i32, i32, p, i32, p, i64, i64, p, i64, p, i32, p, p, i64, p], i32),
         "saf3r_frame_topk_scores": ([p, i64, i32, i32, i32, i32, i32, i32, i32, i32, p, i64, p, p, p], i32),
     }
+    if lib.saf3r_abi_version() != ABI_VERSION:  # (no arguments, int result: ctypes' defaults)
+        raise RuntimeError(f"libsaf3r_hip.so ABI {lib.saf3r_abi_version()} != expected {ABI_VERSION}")
     for name, (args, res) in sig.items():
-        fn = getattr(lib, name)
+        fn = getattr(lib, name, None)
+        if fn is None:  # entries are added within an ABI version
+            raise RuntimeError(f"libsaf3r_hip.so has no {name}: built from older sources, build it again")
         fn.argtypes = args
         fn.restype = res
-    if lib.saf3r_abi_version() != ABI_VERSION:
-        raise RuntimeError(f"libsaf3r_hip.so ABI {lib.saf3r_abi_version()} != expected {ABI_VERSION}")
     _lib = lib
     return lib
 
