@@ -393,6 +393,15 @@ int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed, const void
                           const void* bcast_v, const uint8_t* token_order, const uint8_t* q_scaled, int flags,
                           unsigned long long* pace, unsigned int pace_seq, void* stream);
 
+/* The heads (bit h) whose walks over one range of keys a saf3r_sparse_attn_fwd call with these arguments runs in
+ * split mode, one query tile per work-group with the key tiles split over its four waves (short launches): a
+ * host computation, nothing is launched. compute_units: of the GPU (0: the current device's). For tests and
+ * profiles. */
+int saf3r_sparse_attn_split_heads(int frames, int tokens_per_frame, int num_special, int num_heads,
+                                  const int32_t* head_pattern, int sel_width, int64_t keyset_capacity,
+                                  const uint8_t* token_order, int compute_units, uint64_t* split_heads);
+
+
 /*
  * Gather attention: out[r] = sum_j softmax_j(q[r] . k[idx[r][j]] * scale) v[idx[r][j]], fp32
  * scores and accumulation, head_dim 64 (q, k, v and out rows of 64 elements); idx entries < 0 or

@@ -21,6 +21,7 @@ EXPORTS = (
     "saf3r_pooled_prepare", "saf3r_block_select_pooled", "saf3r_block_select_pooled_workspace_bytes",
     "saf3r_gather_attn_fwd_sliced", "saf3r_gather_attn_workspace_bytes", "saf3r_pack_qkv_typed",
     "saf3r_probe_scores_host", "saf3r_keyset_build_host", "saf3r_keyset_gather_host",
+    "saf3r_sparse_attn_split_heads",
 )
 ABI_VERSION = 13
 PACK_LN_BF16, PACK_POS_INT64 = 1, 2  # enum saf3r_pack_param_flags
@@ -74,6 +75,7 @@ def load():
         "saf3r_block_select": ([p, p, i32, i32, i32, i32, i32, i32, p, p], i32),
         "saf3r_sparse_attn_fwd": ([p, p, p, i32, i32, i32, i32, p, p, i32, f32, p, i64, p, p, p, i64, p, p, p, p, p,
                                    i32, p, ctypes.c_uint, p], i32),
+        "saf3r_sparse_attn_split_heads": ([i32, i32, i32, i32, p, i32, i64, p, i32, p], i32),
         "saf3r_gather_attn_fwd": ([rows, rows, rows, p, i64, i32, i32, i64, f32, i32, rows, p], i32),
         "saf3r_gather_attn_fwd_sliced": ([rows, rows, rows, p, i64, i32, i32, i64, f32, i32, rows, p, i64, p], i32),
         "saf3r_gather_attn_workspace_bytes": ([i32, i32], i64),

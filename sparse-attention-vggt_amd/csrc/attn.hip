@@ -1550,6 +1550,53 @@ static uint64_t choose_split(const HeadWork* hw, int heads, int64_t slots) {
   }
 }
 
+static int compute_units() {
+  int cus = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  return cus;
+}
+
+// Both forms of every head's work items and the heads that run split (two work-groups a CU are resident)
+static uint64_t plan_split(HeadWork* hw, int heads, const int8_t* pattern, uint64_t tok_order, uint64_t framed, int ntt,
+                           const Geom& g, int sel_width, int64_t ks_cap, int cus) {
+  for (int h = 0; h < heads; ++h) {
+    HeadWork& x = hw[h];
+    const bool to = (tok_order >> h) & 1, fr = (framed >> h) & 1;
+    x.tiles = split_tiles(pattern[h], to, fr, ntt, g, ks_cap);
+    x.can_split = x.tiles > 0 && x.tiles <= kSplitMaxTiles;
+    x.n_shared = head_segments(h, pattern[h], to, fr, false, ntt, g, sel_width, ks_cap, x.shared);
+    x.n_split = head_segments(h, pattern[h], to, fr, x.can_split, ntt, g, sel_width, ks_cap, x.split);
+  }
+  return choose_split(hw, heads, 2 * (int64_t)cus);
+}
+
+// The heads in token order and in the framed layout from an array of saf3r_layout (null: none)
+static int head_layouts(const char* who, const uint8_t* layouts, int heads, const int8_t* pattern, const Geom& g,
+                        uint64_t* tok_order, uint64_t* framed) {
+  *tok_order = *framed = 0;
+  for (int h = 0; layouts && h < heads; ++h) {
+    const int lay = layouts[h], pt = pattern[h];
+    if (!lay) continue;
+    if (lay == SAF3R_LAYOUT_TOKEN) {
+      if (pt != SAF3R_DENSE)
+        return fail(SAF3R_ERR_INVALID, "%s: head %d: only DENSE heads take the token-order layout", who, h);
+      *tok_order |= 1ull << h;
+    } else if (lay == SAF3R_LAYOUT_FRAMED) {
+      if (pt != SAF3R_FRAME_LOCAL && pt != SAF3R_ANCHOR_LOCAL && pt != SAF3R_ANCHOR)
+        return fail(SAF3R_ERR_INVALID, "%s: head %d: only FRAME_LOCAL / ANCHOR_LOCAL / ANCHOR heads take the framed layout",
+                    who, h);
+      if (!framed_fits(g))
+        return fail(SAF3R_ERR_UNSUPPORTED, "%s: the framed layout does not fit this geometry", who);
+      *framed |= 1ull << h;
+    } else {
+      return fail(SAF3R_ERR_INVALID, "%s: head %d: unknown layout %d", who, h, lay);
+    }
+  }
+  return SAF3R_OK;
+}
+
 // the K + V bytes of the block-dynamic heads above which split-mode walks are clock-paced
 constexpr int64_t kSplitPacedMinBytes = (int64_t)256 << 20;
 
@@ -1632,31 +1679,12 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
       return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_sparse_attn_fwd: sel_width must be in [1, %d] (got %d)", kMaxList,
                   sel_width);
   }
-  p.tok_order = p.framed = 0;
   if ((int64_t)frames * tokens_per_frame > 0x7fffffc0ll)
     return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_sparse_attn_fwd: too many tokens");
   p.ntok = frames * tokens_per_frame;
   p.ntt = (p.ntok + 63) / 64;
-  if (token_order) {
-    for (int h = 0; h < num_heads; ++h) {
-      const int lay = token_order[h], pt = p.pattern[h];
-      if (!lay) continue;
-      if (lay == SAF3R_LAYOUT_TOKEN) {
-        if (pt != SAF3R_DENSE)
-          return fail(SAF3R_ERR_INVALID, "saf3r_sparse_attn_fwd: head %d: only DENSE heads take the token-order layout", h);
-        p.tok_order |= 1ull << h;
-      } else if (lay == SAF3R_LAYOUT_FRAMED) {
-        if (pt != SAF3R_FRAME_LOCAL && pt != SAF3R_ANCHOR_LOCAL && pt != SAF3R_ANCHOR)
-          return fail(SAF3R_ERR_INVALID,
-                      "saf3r_sparse_attn_fwd: head %d: only FRAME_LOCAL / ANCHOR_LOCAL / ANCHOR heads take the framed layout", h);
-        if (!framed_fits(p.g))
-          return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_sparse_attn_fwd: the framed layout does not fit this geometry");
-        p.framed |= 1ull << h;
-      } else {
-        return fail(SAF3R_ERR_INVALID, "saf3r_sparse_attn_fwd: head %d: unknown layout %d", h, lay);
-      }
-    }
-  }
+  if (int e = head_layouts("saf3r_sparse_attn_fwd", token_order, num_heads, p.pattern, p.g, &p.tok_order, &p.framed))
+    return e;
   p.q_pre = 0;
   if (q_scaled)
     for (int h = 0; h < num_heads; ++h)
@@ -1692,20 +1720,9 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   p.pace_read = (int)(pace_seq % 3u);
   p.pace_acc = (int)((pace_seq + 1u) % 3u);
   p.pace_zero = (int)((pace_seq + 2u) % 3u);
-  int cus = 0, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
+  const int cus = compute_units();
   HeadWork hw[kMaxHeads];
-  for (int h = 0; h < num_heads; ++h) {
-    HeadWork& x = hw[h];
-    const bool to = (p.tok_order >> h) & 1, fr = (p.framed >> h) & 1;
-    x.tiles = split_tiles(p.pattern[h], to, fr, p.ntt, p.g, keyset_capacity);
-    x.can_split = x.tiles > 0 && x.tiles <= kSplitMaxTiles;
-    x.n_shared = head_segments(h, p.pattern[h], to, fr, false, p.ntt, p.g, sel_width, keyset_capacity, x.shared);
-    x.n_split = head_segments(h, p.pattern[h], to, fr, x.can_split, p.ntt, p.g, sel_width, keyset_capacity, x.split);
-  }
-  p.split = choose_split(hw, num_heads, 2 * (int64_t)cus);
+  p.split = plan_split(hw, num_heads, p.pattern, p.tok_order, p.framed, p.ntt, p.g, sel_width, keyset_capacity, cus);
   Seg segs[kMaxSegs];
   int nseg = 0;
   for (int h = 0; h < num_heads; ++h) {
@@ -1757,4 +1774,29 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   auto fixup = p.split ? sparse_attn_fixup_kernel<true> : sparse_attn_fixup_kernel<false>;
   hipLaunchKernelGGL(fixup, dim3((unsigned)f.fix_groups), dim3(256), 0, (hipStream_t)stream, f);
   return check_launch("saf3r_sparse_attn_fwd");
+}
+
+extern "C" int saf3r_sparse_attn_split_heads(int frames, int tokens_per_frame, int num_special, int num_heads,
+                                             const int32_t* head_pattern, int sel_width, int64_t keyset_capacity,
+                                             const uint8_t* token_order, int cus, uint64_t* split_heads) {
+  const char* who = "saf3r_sparse_attn_split_heads";
+  Geom g;
+  if (!make_geom(frames, tokens_per_frame, num_special, &g) || (int64_t)frames * tokens_per_frame > 0x7fffffc0ll)
+    return fail(SAF3R_ERR_INVALID, "%s: invalid geometry", who);
+  if (num_heads <= 0 || num_heads > kMaxHeads || !head_pattern || !split_heads || cus < 0 || sel_width < 0 ||
+      keyset_capacity < 0)
+    return fail(SAF3R_ERR_INVALID, "%s: bad argument", who);
+  int8_t pattern[kMaxHeads];
+  for (int h = 0; h < num_heads; ++h) {
+    if (head_pattern[h] < SAF3R_DENSE || head_pattern[h] > SAF3R_TOKEN_DYNAMIC_KEYSET)
+      return fail(SAF3R_ERR_INVALID, "%s: head %d has unknown pattern %d", who, h, head_pattern[h]);
+    pattern[h] = (int8_t)head_pattern[h];
+  }
+  uint64_t tok_order, framed;
+  if (int e = head_layouts(who, token_order, num_heads, pattern, g, &tok_order, &framed)) return e;
+  HeadWork hw[kMaxHeads];
+  *split_heads = plan_split(hw, num_heads, pattern, tok_order, framed, (frames * tokens_per_frame + 63) / 64, g, sel_width,
+                            keyset_capacity, cus > 0 ? cus : compute_units());
+  set_error("");
+  return SAF3R_OK;
 }

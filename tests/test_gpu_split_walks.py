@@ -1,9 +1,8 @@
-"""Short attention launches, whose long single-range walks run one query tile per work-group, the key
-tiles split over its four waves: every walk kind that takes that route, at partial last tiles and at key
-sets smaller than a tile, against the oracle on the inputs the kernels consumed (bf16 inputs, fp64
-oracle; the bars of the other attention tests, which bound the bf16 rounding of P and of the output).
-
-A launch as short as these splits walks of 24 key tiles or more: the cases have a few tiles more.
+"""Short attention launches of mixed heads, some of whose long single-range walks run one query tile per
+work-group, the key tiles split over its four waves, against the oracle on the inputs the kernels consumed
+(bf16 inputs, fp64 oracle; the bars of the other attention tests, which bound the bf16 rounding of P and of
+the output). Which heads split depends on the mix: ANCHOR_LOCAL alone, DENSE and KEYSET, or none where a
+packed frame-relative head has the longest walk. Each kind on the split route: test_gpu_split_kinds.py.
 """
 import importlib
 
