@@ -125,12 +125,13 @@ __device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t x, Op op) {
 //   2. Those candidates, (order key, position) in one word, into LDS in key order, two per lane.
 //   3. The exact k-th key by bisection over the candidates, and the k kept ones written out in key
 //      order, equal keys lowest first.
-// A row whose counts jump over the window (many equal scores), or k > kCands, bisects over all its
-// keys instead. Bound by VALU issue (the loads alone would take half the time): about 260 instructions per row
-// and frame of 1036 keys at k = 64. It replaced one bisection over unpacked keys (24 registers for
-// 1036 keys, 9 rounds of two instructions per key) for k > 8, and per-lane sorted lists with a
-// butterfly merge for k <= 8: 4096 rows x 32 frames x 1036 keys,
-// top-64 279 -> 97 us, top-4 111 -> 90 us; 128 x 1369 keys 1070 -> 392 and 475 -> 364 us (3.9 TB/s).
+// A row whose counts jump over the window (many equal scores) takes every key above the one they jump at
+// and the first of those equal to it; k > kCands bisects over all keys instead.
+// Bound by VALU issue (the loads alone would take half the time): about 260 instructions per row and
+// frame of 1036 keys at k = 64. It replaced one bisection over unpacked keys (24 registers for 1036
+// keys, 9 rounds of two instructions per key) for k > 8, and per-lane sorted lists with a butterfly
+// merge for k <= 8: 4096 rows x 32 frames x 1036 keys, top-64 279 -> 97 us, top-4 111 -> 90 us; 128 x
+// 1369 keys 1070 -> 392 and 475 -> 364 us (3.9 TB/s).
 constexpr int kCands = 128;
 template <int NR, int NF>
 __global__ __launch_bounds__(256) void frame_select_kernel(FrameTopkParams p) {
@@ -176,6 +177,7 @@ __global__ __launch_bounds__(256) void frame_select_kernel(FrameTopkParams p) {
   const uint32_t lmax = max((uint32_t)mx[0], (uint32_t)mx[1]);
   const uint32_t top = wave_reduce_u32(lmax, [](uint32_t a, uint32_t b) { return max(a, b); });
   uint32_t t = 1;
+  uint32_t thr = 0;  // the k-th largest key, where the counts jump over the window at it (0: the lowest key)
   int n = -1;
   if (k <= kCands) {
     if (p.P > kCands) {
@@ -204,6 +206,8 @@ __global__ __launch_bounds__(256) void frame_select_kernel(FrameTopkParams p) {
           if (ca >= k && ca <= kCands) {
             n = ca;
             t = a;
+          } else if (ca >= k) {
+            thr = a;  // count(a + 1) < k
           }
           break;
         }
@@ -267,12 +271,13 @@ __global__ __launch_bounds__(256) void frame_select_kernel(FrameTopkParams p) {
     }
     return;
   }
-  // the exact threshold over all keys: the largest t with at least k keys at or above it
-  uint32_t thr = 0;
+  // k > kCands: the exact threshold over all keys, the largest t with at least k keys at or above it
+  if (k > kCands) {
 #pragma unroll 1
-  for (int bit = 15; bit >= 0; --bit) {
-    const uint32_t c = thr | (1u << bit);
-    if (count_ge(c) >= k) thr = c;
+    for (int bit = 15; bit >= 0; --bit) {
+      const uint32_t c = thr | (1u << bit);
+      if (count_ge(c) >= k) thr = c;
+    }
   }
   int need = k - (thr < 0xFFFFu ? count_ge(thr + 1) : 0);  // keys equal to thr to keep, lowest first
   int base = 0;
