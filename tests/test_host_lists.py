@@ -37,6 +37,25 @@ def test_lists_of_tensors_are_read_each_time(ops):
     assert list(ops._u8_layouts(same, 2)) == [0, 0]
 
 
+def test_lists_of_other_numbers(ops):
+    """Whatever int() or bool() takes counts by its value."""
+    import numpy as np
+    import torch
+    assert list(ops._i32_array([1.0, np.int64(2), np.float32(3), True, torch.tensor(4.0), torch.tensor(True)])) \
+        == [1, 2, 3, 1, 4, 1]
+    assert list(ops._i32_array(np.array([7, 8]))) == [7, 8] and list(ops._i32_array(iter([5, 6]))) == [5, 6]
+    some = [2, -1, 0, 0.5, None, "x", 256, np.bool_(True), np.array(True), torch.tensor(0.0), torch.tensor(False)]
+    assert list(ops._u8_flags(some, len(some))) == [1, 1, 0, 1, 0, 1, 1, 1, 1, 0, 0]
+    assert list(ops._u8_flags(np.array([0, 3]), 2)) == [0, 1] and list(ops._u8_flags(torch.tensor([2, 0]), 2)) == [1, 0]
+    assert list(ops._u8_layouts([1.0, True, np.int32(0), torch.tensor(1)], 4)) == [1, 1, 0, 1]
+    for bad in (-1, 3, 256, 300.0):
+        with pytest.raises(ValueError, match="layout"):
+            ops._u8_layouts([0, bad], 2)
+    for fn in (ops._u8_flags, ops._u8_layouts):
+        with pytest.raises(ValueError, match="heads"):
+            fn([1, 1, 1], 2)
+
+
 def test_pattern_tensors_are_read_each_time(ops, pkg, monkeypatch):
     """The head counts that ``sparse_attn_fwd`` checks come from the patterns of the call."""
     import torch
