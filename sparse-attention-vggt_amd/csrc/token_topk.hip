@@ -445,10 +445,11 @@ __device__ __forceinline__ uint64_t lane_xor(uint64_t x, int lane) {
   return ((uint64_t)lane_xor<D>((uint32_t)(x >> 32), lane) << 32) | lane_xor<D>((uint32_t)x, lane);
 }
 
-template <typename Op>
-__device__ __forceinline__ float wave_reduce32(float x, Op op) {
-  auto at = [](uint32_t y) { return __builtin_bit_cast(float, y); };
-  auto bits = [](float y) { return __builtin_bit_cast(uint32_t, y); };
+// x of 32 bits over the wave, as a wave-uniform value
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce32(T x, Op op) {
+  auto at = [](uint32_t y) { return __builtin_bit_cast(T, y); };
+  auto bits = [](T y) { return __builtin_bit_cast(uint32_t, y); };
   x = op(x, at(dpp32<0xB1>(bits(x))));
   x = op(x, at(dpp32<0x4E>(bits(x))));
   x = op(x, at(dpp32<0x141>(bits(x))));
@@ -457,7 +458,7 @@ __device__ __forceinline__ float wave_reduce32(float x, Op op) {
   x = op(at((uint32_t)a[0]), at((uint32_t)a[1]));
   const auto b = __builtin_amdgcn_permlane32_swap(bits(x), bits(x), false, false);
   x = op(at((uint32_t)b[0]), at((uint32_t)b[1]));
-  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane((int)bits(x)));
+  return at((uint32_t)__builtin_amdgcn_readfirstlane((int)bits(x)));
 }
 
 // One compare-exchange of a bitonic network over the wave: runs of M lanes, distance D
@@ -515,9 +516,9 @@ __device__ __forceinline__ int lanes_before(uint64_t m, int base) {
 //     the window, which mostly takes one or two;
 //   - those candidates, as composite keys, into the row's own LDS space, then a bitonic sort over
 //     the wave (DPP exchanges) and the k best written out in order.
-// A row whose counts jump over the window (more than CAP - k equal scores, or infinities), or that holds
-// a NaN, takes the exact threshold by 32 counts on the sortable keys, equal keys from the lowest index
-// on (the matrix core hands every NaN on as -NaN, the lowest key).
+// A row whose counts jump over the window (more than CAP - k equal scores, or infinities), or that holds a NaN
+// (the matrix core hands every NaN on as -NaN, the lowest key), takes the exact threshold on the sortable
+// keys, equal keys from the lowest index on.
 // CAP is 64 for k <= 32 (one sorted register per lane), else 128 (two, merged).
 // The next frame's fragments load while the rows of this one are selected (NV <= 24; longer frames
 // have no registers for it).
@@ -644,6 +645,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void topk_rows_kernel(TopkParams p)
       for (int i = 0; i < NV; i += 2) nans |= __builtin_amdgcn_ballot_w64(__builtin_isunordered(v[i], v[i + 1]));
       float t = -0x1.fffffep127f;  // P <= cap: every finite score is a candidate
       bool found = false;
+      float lo = -__builtin_inff(), hi = __builtin_inff();
       if (!nans && p.P <= cap) {
         const int c = count(t);
         found = c >= p.ke && c <= cap;
@@ -651,8 +653,8 @@ __global__ __launch_bounds__(64 * kRowWaves) void topk_rows_kernel(TopkParams p)
         float lmax = v[0];
 #pragma unroll
         for (int i = 1; i < NV; ++i) lmax = fmaxf(lmax, v[i]);
-        float hi = wave_reduce32(lmax, [](float a, float b) { return fmaxf(a, b); });
-        float lo = wave_reduce32(lmax, [](float a, float b) { return fminf(a, b); });
+        hi = wave_reduce32(lmax, [](float a, float b) { return fmaxf(a, b); });
+        lo = wave_reduce32(lmax, [](float a, float b) { return fminf(a, b); });
         if (p.ke > 64) lo -= 2.f * (hi - lo);  // 64 scores reach the least lane maximum: look below it
         // first guess: the value that about `lanes` of the 64 lane maxima reach
         float a = lo, b = hi;
@@ -677,7 +679,9 @@ __global__ __launch_bounds__(64 * kRowWaves) void topk_rows_kernel(TopkParams p)
         }
       }
       int n = 0;  // candidates, in increasing key index
-      if (found) {
+      // (likely: otherwise the exact path's values take registers of this one: 6 x 1369 tokens, top-32 115 us
+      // against 100, 2 x 4096 219 against 127)
+      if (__builtin_expect(found, 1)) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
           const bool take = !(v[i] < t);
@@ -691,14 +695,34 @@ __global__ __launch_bounds__(64 * kRowWaves) void topk_rows_kernel(TopkParams p)
         uint32_t u[NV];  // sortable keys, 0 past the frame's end
 #pragma unroll
         for (int i = 0; i < NV; ++i) u[i] = ln + 64 * i < p.P ? fkey(v[i]) : 0;
-        uint32_t thr = 0;  // the largest key with at least ke keys at or above it
-#pragma unroll 1
-        for (int b = 31; b >= 0; --b) {
-          const uint32_t cand = thr | (1u << b);
+        auto count_keys = [&](uint32_t x) {
           int c = 0;
 #pragma unroll
-          for (int i = 0; i < NV; ++i) c += __popcll(__builtin_amdgcn_ballot_w64(u[i] >= cand));
-          if (c >= p.ke) thr = cand;
+          for (int i = 0; i < NV; ++i) c += __popcll(__builtin_amdgcn_ballot_w64(u[i] >= x));
+          return c;
+        };
+        // The ke-th largest key: at least ke keys are >= thr, fewer above last. First the search's bounds (the counts
+        // took both zeros as equal), then the best key up to `last`, which is it where few scores differ
+        // (16 x 1036 tokens, top-64, all scores equal 1335 -> 715 us, five values 1600 -> 1000: it was 32 counts
+        // from the top bit down), with three halvings between its tries.
+        const uint32_t from = fkey(lo == 0.f ? -0.f : lo), to = fkey(hi == 0.f ? 0.f : hi);
+        uint32_t thr = 0, last = 0xFFFFFFFFu;
+#pragma unroll 1
+        for (int step = -2; thr < last; ++step) {
+          uint32_t x = step == -2 ? from : step == -1 ? to : thr + ((last - thr) >> 1) + 1;
+          const bool best = step >= 0 && (step & 3) == 0;
+          if (best) {
+            x = 0;
+#pragma unroll
+            for (int i = 0; i < NV; ++i) x = max(x, u[i] <= last ? u[i] : 0u);
+            x = wave_reduce32(x, [](uint32_t a, uint32_t b) { return max(a, b); });
+          }
+          if (count_keys(x) >= p.ke) {
+            thr = x;
+            if (best) break;
+          } else {
+            last = x - 1;
+          }
         }
         int need = p.ke;  // keys equal to thr to take
 #pragma unroll
