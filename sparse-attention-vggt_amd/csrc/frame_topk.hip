@@ -32,6 +32,7 @@ struct FrameTopkParams {
   int64_t ors;        // its row stride
   int ocol;           // first column written
   int lanes;          // lane maxima the first threshold guess aims at
+  int window;         // whether a threshold with k .. kCands keys is searched for (see frame_window)
   uint16_t* okey;     // candidate order keys (cap stage input), row stride ors, or null
 };
 
@@ -113,6 +114,103 @@ __device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t x, Op op) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)op((uint32_t)b[0], (uint32_t)b[1]));
 }
 
+// ---- frame stage, k <= 4 in short frames: four waves, one (row, frame) each ----
+// Every lane keeps the four best of its keys as composites (order key << 16 | 0xFFFF - position: larger is
+// better, equal scores by the lower position; 0 for none), descending; six exchanges merge the lists of
+// the wave, and the k winners are written in increasing key order. Bound by VALU issue.
+// Frames of up to 1407 keys: there the lists beat the threshold search below (16384 rows x 8 frames, top-4, us,
+// search / lists: 256 keys 79 / 40, 512 75 / 50, 1036 83 / 67, 1369 90 / 78; five different scores
+// 63 / 40, 67 / 49, 104 / 67, 114 / 78), beyond they would hold more words than they save.
+constexpr int kListMax = 4;
+constexpr int kListWords = 11;  // per lane
+__device__ __forceinline__ void list_sort(uint32_t (&c)[kListMax]) {  // a bitonic list, descending
+  const uint32_t a = max(c[0], c[2]), b = max(c[1], c[3]), d = min(c[0], c[2]), e = min(c[1], c[3]);
+  c[0] = max(a, b);
+  c[1] = min(a, b);
+  c[2] = max(d, e);
+  c[3] = min(d, e);
+}
+
+template <int NR, int NF>
+__global__ __launch_bounds__(256) void frame_list_kernel(FrameTopkParams p) {
+  const int lane = tid_x() & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid_x() >> 6);
+  const int row = bid_y();
+  const int fs = bid_x() * 4 + w;  // selected-frame index
+  if (fs >= p.F - p.f0) return;
+  const int64_t s0 = (int64_t)(p.f0 + fs) * p.P;  // first key of the frame in the row
+  const int off = (int)(s0 & 1);                  // the span starts at the word of key s0
+  const uint32_t* words = reinterpret_cast<const uint32_t*>(p.scores + (int64_t)row * p.srs + (s0 - off));
+  const int last = (off + p.P - 1) >> 1;          // last word with a key of the frame
+  const int k = p.k;
+  uint32_t key[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) key[r] = words[r < NF ? lane + 64 * r : min(lane + 64 * r, last)];
+  uint32_t c[kListMax] = {0, 0, 0, 0};
+  const int j0 = 2 * lane - off;
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const s16x2 b = __builtin_bit_cast(s16x2, key[r]);
+    key[r] ^= __builtin_bit_cast(uint32_t, b >> (short)15) | 0x80008000u;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t j = (uint32_t)(j0 + 128 * r + h);
+      uint32_t y = (h ? key[r] & 0xFFFF0000u : key[r] << 16) | (0xFFFFu - j);
+      if ((r == 0 && h == 0) || r >= NF - 1)  // other positions are inside the frame
+        y = j < (uint32_t)p.P ? y : 0u;
+#pragma unroll
+      for (int i = kListMax - 1; i > 0; --i) c[i] = max(c[i], min(c[i - 1], y));
+      c[0] = max(c[0], y);
+    }
+  }
+  auto merge = [&](const uint32_t (&x)[kListMax], const uint32_t (&y)[kListMax]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kListMax; ++i) c[i] = max(x[i], y[kListMax - 1 - i]);
+    list_sort(c);
+  };
+  auto step = [&](auto ctl) __attribute__((always_inline)) {
+    uint32_t x[kListMax], y[kListMax];
+#pragma unroll
+    for (int i = 0; i < kListMax; ++i) {
+      x[i] = c[i];
+      y[i] = (uint32_t)__builtin_amdgcn_mov_dpp((int)c[i], decltype(ctl)::value, 0xF, 0xF, true);
+    }
+    merge(x, y);
+  };
+  step(std::integral_constant<int, 0xB1>{});   // quad_perm [1, 0, 3, 2]
+  step(std::integral_constant<int, 0x4E>{});   // quad_perm [2, 3, 0, 1]
+  step(std::integral_constant<int, 0x141>{});  // mirror of 8
+  step(std::integral_constant<int, 0x128>{});  // rotation by 8 of 16
+  uint32_t x[kListMax], y[kListMax];
+#pragma unroll
+  for (int i = 0; i < kListMax; ++i) {
+    const auto s = __builtin_amdgcn_permlane16_swap(c[i], c[i], false, false);
+    x[i] = s[0];
+    y[i] = s[1];
+  }
+  merge(x, y);
+#pragma unroll
+  for (int i = 0; i < kListMax; ++i) {
+    const auto s = __builtin_amdgcn_permlane32_swap(c[i], c[i], false, false);
+    x[i] = s[0];
+    y[i] = s[1];
+  }
+  merge(x, y);
+  // lane i < k: winner i, written behind the winners of lower positions
+  uint32_t mine = 0;
+#pragma unroll
+  for (int i = 0; i < kListMax; ++i)
+    if (i == lane) mine = c[i];
+  int rank = 0;
+#pragma unroll
+  for (int i = 0; i < kListMax; ++i) rank += i < k && (c[i] & 0xFFFFu) > (mine & 0xFFFFu) ? 1 : 0;
+  if (lane < k) {
+    const int64_t at = (int64_t)row * p.ors + (int64_t)fs * k + rank;
+    p.out[at + p.ocol] = (int32_t)(s0 + (0xFFFFu - (mine & 0xFFFFu)));
+    if (p.okey) p.okey[at] = (uint16_t)(mine >> 16);
+  }
+}
+
 // ---- frame stage: four waves, one (row, frame) each ----
 // A lane holds NR words of two scores: word lane + 64 r of the frame's span, so element order (r,
 // lane, half) is increasing key order. Words up to NF are whole (the caller picks NR by the frame's
@@ -126,12 +224,11 @@ __device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t x, Op op) {
 //   3. The exact k-th key by bisection over the candidates, and the k kept ones written out in key
 //      order, equal keys lowest first.
 // A row whose counts jump over the window (many equal scores) takes every key above the one they jump at
-// and the first of those equal to it; k > kCands bisects over all keys instead.
+// and the first of those equal to it. Without a window (frame_window): the exact threshold over all keys.
 // Bound by VALU issue (the loads alone would take half the time): about 260 instructions per row and
 // frame of 1036 keys at k = 64. It replaced one bisection over unpacked keys (24 registers for 1036
-// keys, 9 rounds of two instructions per key) for k > 8, and per-lane sorted lists with a butterfly
-// merge for k <= 8: 4096 rows x 32 frames x 1036 keys, top-64 279 -> 97 us, top-4 111 -> 90 us; 128 x
-// 1369 keys 1070 -> 392 and 475 -> 364 us (3.9 TB/s).
+// keys, 9 rounds of two instructions per key): 4096 rows x 32 frames x 1036 keys, top-64 279 -> 97 us,
+// 128 x 1369 keys 1070 -> 392 us.
 constexpr int kCands = 128;
 template <int NR, int NF>
 __global__ __launch_bounds__(256) void frame_select_kernel(FrameTopkParams p) {
@@ -179,7 +276,7 @@ __global__ __launch_bounds__(256) void frame_select_kernel(FrameTopkParams p) {
   uint32_t t = 1;
   uint32_t thr = 0;  // the k-th largest key, where the counts jump over the window at it (0: the lowest key)
   int n = -1;
-  if (k <= kCands) {
+  if (p.window) {
     if (p.P > kCands) {
       uint32_t a = 1, b = top;
       t = wave_reduce_u32(lmax, [](uint32_t x, uint32_t y) { return min(x, y); });
@@ -271,8 +368,8 @@ __global__ __launch_bounds__(256) void frame_select_kernel(FrameTopkParams p) {
     }
     return;
   }
-  // k > kCands: the exact threshold over all keys, the largest t with at least k keys at or above it
-  if (k > kCands) {
+  // no window: the exact threshold over all keys, the largest t with at least k keys at or above it
+  if (!p.window) {
 #pragma unroll 1
     for (int bit = 15; bit >= 0; --bit) {
       const uint32_t c = thr | (1u << bit);
@@ -394,6 +491,15 @@ __global__ __launch_bounds__(256) void first_samples_kernel(int32_t* idx, int64_
 
 using namespace saf3r;
 
+// Whether the frame stage searches for a window of k .. kCands keys. The closer k comes to kCands, the more counts
+// it takes to hit the window, and frames with few different scores jump over it; the exact threshold takes
+// 16 counts whatever the scores. The line is fitted to (us, 16384 rows x 8 frames of normal scores in bf16, window /
+// exact): 160 keys k = 64 77 / 82, 96 129 / 82; 256 keys k = 80 107 / 100; 512 keys k = 80 120 / 142, 96 152 / 142; 768 keys
+// k = 96 165 / 182; 1036 keys k = 112 213 / 225, 128 284 / 225; 1369 keys k = 112 229 / 263, 128 317 / 263.
+static bool frame_window(int per_frame, int k) {
+  return per_frame <= kCands || k <= std::min(112, std::max(64, 48 + per_frame / 16));
+}
+
 extern "C" int saf3r_frame_topk_scores(const void* scores, int64_t score_stride, int rows, int frames, int per_frame,
                                        int exclude_first, int first_stride, int per_frame_mode, int topk, int cap,
                                        int32_t* idx, int64_t idx_stride, int32_t* cand_idx, uint16_t* cand_key,
@@ -443,22 +549,30 @@ extern "C" int saf3r_frame_topk_scores(const void* scores, int64_t score_stride,
     p.ors = capped ? rest : idx_stride;
     p.ocol = capped ? 0 : fsel;
     p.okey = capped ? cand_key : nullptr;
+    p.window = frame_window(per_frame, k);
     const dim3 grid((nfr + 3) / 4, rows);
     // m keys at or above a threshold, spread at random, reach 64 (1 - e^(-m / 64)) of the lane
     // maxima: aim at the middle of the window
     p.lanes = (int)(64.0 * (1.0 - std::exp(-std::sqrt((double)std::min(k, kCands) * kCands) / 64.0)));
     const int words = per_frame / 2 + 1;  // of a frame's span, at most
-#define SAF3R_FRAME(NR, NF) hipLaunchKernelGGL((frame_select_kernel<NR, NF>), grid, dim3(256), 0, st, p)
-    if (words <= 64 * 2) SAF3R_FRAME(2, 0);
-    else if (words <= 64 * 3) SAF3R_FRAME(3, 1);
-    else if (words <= 64 * 5) SAF3R_FRAME(5, 2);
-    else if (words <= 64 * 7) SAF3R_FRAME(7, 4);
-    else if (words <= 64 * 9) SAF3R_FRAME(9, 6);
-    else if (words <= 64 * 11) SAF3R_FRAME(11, 8);
-    else if (words <= 64 * 13) SAF3R_FRAME(13, 10);
-    else if (words <= 64 * 17) SAF3R_FRAME(17, 12);
-    else if (words <= 64 * 25) SAF3R_FRAME(25, 16);
-    else SAF3R_FRAME(33, 24);
+#define SAF3R_FRAME(KERNEL, NR, NF) hipLaunchKernelGGL((KERNEL<NR, NF>), grid, dim3(256), 0, st, p)
+    if (k <= kListMax && words <= 64 * kListWords) {
+      if (words <= 64 * 2) SAF3R_FRAME(frame_list_kernel, 2, 0);
+      else if (words <= 64 * 3) SAF3R_FRAME(frame_list_kernel, 3, 1);
+      else if (words <= 64 * 5) SAF3R_FRAME(frame_list_kernel, 5, 2);
+      else if (words <= 64 * 7) SAF3R_FRAME(frame_list_kernel, 7, 4);
+      else if (words <= 64 * 9) SAF3R_FRAME(frame_list_kernel, 9, 6);
+      else SAF3R_FRAME(frame_list_kernel, 11, 8);
+    } else if (words <= 64 * 2) SAF3R_FRAME(frame_select_kernel, 2, 0);
+    else if (words <= 64 * 3) SAF3R_FRAME(frame_select_kernel, 3, 1);
+    else if (words <= 64 * 5) SAF3R_FRAME(frame_select_kernel, 5, 2);
+    else if (words <= 64 * 7) SAF3R_FRAME(frame_select_kernel, 7, 4);
+    else if (words <= 64 * 9) SAF3R_FRAME(frame_select_kernel, 9, 6);
+    else if (words <= 64 * 11) SAF3R_FRAME(frame_select_kernel, 11, 8);
+    else if (words <= 64 * 13) SAF3R_FRAME(frame_select_kernel, 13, 10);
+    else if (words <= 64 * 17) SAF3R_FRAME(frame_select_kernel, 17, 12);
+    else if (words <= 64 * 25) SAF3R_FRAME(frame_select_kernel, 25, 16);
+    else SAF3R_FRAME(frame_select_kernel, 33, 24);
 #undef SAF3R_FRAME
     if (int e = check_launch("saf3r_frame_topk_scores")) return e;
     if (!capped) return SAF3R_OK;
