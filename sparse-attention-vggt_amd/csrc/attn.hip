@@ -104,9 +104,6 @@ __device__ inline float partner_sum(float x) {
   return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
 }
 
-// high word of a 32 x 32-bit product as one multiply instruction (the __umulhi library routine is
-// an out-of-line call here, with the call's register saves, once per use)
-
 struct Acc {
   f32x16 o[2][2];  // [dh][gq]: O^T rows 32*dh + (16*half + a), query 32*gq + col
   float m[2];      // reference maximum (raw score units) per query group
@@ -558,8 +555,6 @@ struct Item {
   bool tokord, framed;
 };
 
-// SPLIT: a launch in which some heads' single-range walks are split (AttnParams.split)
-template <bool SPLIT>
 __device__ inline Item decode_item(const AttnParams& p, int item) {
   const Geom& g = p.g;
   Item d;
@@ -574,7 +569,7 @@ __device__ inline Item decode_item(const AttnParams& p, int item) {
   const int groups_pf = (g.NBf + 3) >> 2;
   d.tokord = pat == SAF3R_DENSE && ((p.tok_order >> d.h) & 1);
   d.framed = d.h < 64 && ((p.framed >> d.h) & 1);
-  if (SPLIT && d.h < 64 && ((p.split >> d.h) & 1)) {  // one query tile per item, in tile order
+  if (d.h < 64 && ((p.split >> d.h) & 1)) {  // one query tile per item, in tile order
     d.qt0 = it;
     d.nw = 4;
     d.kind = kSplit;
@@ -630,7 +625,7 @@ __device__ inline uint16_t* item_marker(const AttnParams& p, const Item& d) {
 
 // The kernel body for work item `item` (uniform). FIXUP: walked again, exactly, because the main
 // launch marked it.
-template <bool FIXUP, bool SPLIT>
+template <bool FIXUP>
 __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
   __shared__ __align__(16) char ring[kRing];
   __shared__ int list[kMaxList];
@@ -651,7 +646,7 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
   }
 
   // ---- decode the work item (uniform) ----
-  const Item d = decode_item<SPLIT>(p, item);
+  const Item d = decode_item(p, item);
   const int h = d.h, pat = d.pat, qt0 = d.qt0, nw = d.nw, kind = d.kind;
   const int bfr = d.bfr;  // BROADCAST: the frame whose rows the item writes
   const bool tokord = d.tokord, framed = d.framed;
@@ -1080,8 +1075,8 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
     // The tile list in LDS; an entry holds the key tile and its number of valid keys: tile << 7 | valid
     // (1..64).
     int total = 0;
-    const bool kset = SPLIT && (pat == SAF3R_KEYSET || pat == SAF3R_TOKEN_DYNAMIC_KEYSET);
-    if (!SPLIT || (pat == SAF3R_BLOCK_DYNAMIC && qt >= g.nst)) {
+    const bool kset = pat == SAF3R_KEYSET || pat == SAF3R_TOKEN_DYNAMIC_KEYSET;
+    if (pat == SAF3R_BLOCK_DYNAMIC && qt >= g.nst) {
       // a block-dynamic patch tile: its selection row (invalid entries dropped, order kept)
       const int32_t* srow = p.sel + ((int64_t)p.slot[h] * ((int64_t)g.F * g.NBf) + (qt - g.nst)) * p.sel_width;
       for (int c0 = 0; c0 < p.sel_width; c0 += 256) {
@@ -1326,15 +1321,15 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
     __syncthreads();
     const int row = tid >> 2, d0 = (tid & 3) * 16;
     int64_t tok;  // of the thread's row, as row_info (whose own rows the compiler needs in its form)
-    if (SPLIT && tokord) {
+    if (tokord) {
       const int i = qt * 64 + row;
       tok = i < p.ntok ? (int64_t)i : -1;
-    } else if (SPLIT && framed) {
+    } else if (framed) {
       const int i = qb * 64 + row;
       tok = i < g.T ? (int64_t)qf * g.T + i : -1;
     } else if (qspecial) {
       const int sl = qt * 64 + row;
-      tok = SPLIT && sl < g.S ? (int64_t)(sl / g.ns) * g.T + sl % g.ns : -1;
+      tok = sl < g.S ? (int64_t)(sl / g.ns) * g.T + sl % g.ns : -1;
     } else {
       const int pp = qb * 64 + row;
       tok = pp < g.P ? (int64_t)qf * g.T + g.ns + pp : -1;
@@ -1381,17 +1376,12 @@ __device__ __forceinline__ void attn_body(const AttnParams& p, const int item) {
   }
 }
 
-// Launches without split walks keep a kernel of their own: with the split walks' code in it the compiler
-// spilled 28 bytes a lane instead of 20, which a layer of 48 x 1301 tokens and 24 heads took 3 % longer with
-// (9.76 -> 10.10 ms), one of 32 x 1374 tokens 1.4 % (1.85 -> 1.88 ms).
-template <bool SPLIT>
 __global__ __launch_bounds__(256, 2) void sparse_attn_kernel(AttnParams p) {
-  attn_body<false, SPLIT>(p, __builtin_amdgcn_workgroup_id_x());
+  attn_body<false>(p, __builtin_amdgcn_workgroup_id_x());
 }
 
 // Work-group g reads the markers of items g, g + G, g + 2G, ... (G = fix_groups), 64 at a time on
 // wave 0's lanes, and walks the marked ones exactly, one after the other.
-template <bool SPLIT>
 __global__ __launch_bounds__(256, 2) void sparse_attn_fixup_kernel(AttnParams p) {
   __shared__ uint64_t marked;
   const int tid = __builtin_amdgcn_workitem_id_x();
@@ -1401,7 +1391,7 @@ __global__ __launch_bounds__(256, 2) void sparse_attn_fixup_kernel(AttnParams p)
       const int item = base + G * tid;
       bool m = false;
       if (item < p.n_items) {
-        const Item d = decode_item<SPLIT>(p, item);
+        const Item d = decode_item(p, item);
         m = d.kind != kSkip && *reinterpret_cast<const volatile uint16_t*>(item_marker(p, d)) == 0xFFFFu;
       }
       const uint64_t b = __ballot(m);
@@ -1415,7 +1405,7 @@ __global__ __launch_bounds__(256, 2) void sparse_attn_fixup_kernel(AttnParams p)
     while (b) {
       const int l = __builtin_ctzll(b);
       b &= b - 1;
-      attn_body<true, SPLIT>(p, base + G * l);
+      attn_body<true>(p, base + G * l);
       __syncthreads();  // the next item reuses the LDS
     }
   }
@@ -1697,9 +1687,9 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   p.out = (__bf16*)out;
   p.out_stride = out_row_stride;
   p.c = scale * 1.4426950408889634f;
+  // (the limit of an earlier frame lookup of special keys; frames of thousands of them were never run)
   if (p.g.ns > 0 && (uint64_t)p.g.Sp * (uint64_t)p.g.ns >= 0x100000000ull)
     return fail(SAF3R_ERR_UNSUPPORTED, "saf3r_sparse_attn_fwd: too many special tokens");
-  // ceil(2^32 / ns) fits 32 bits for ns >= 2 only: ns = 1 is magic 0, which the kernel tests for
   if (flags & ~SAF3R_ATTN_FIXED_ORDER) return fail(SAF3R_ERR_INVALID, "saf3r_sparse_attn_fwd: unknown flags 0x%x", flags);
   if ((uintptr_t)pace % 8) return fail(SAF3R_ERR_INVALID, "saf3r_sparse_attn_fwd: pace must be 8-byte aligned");
   const bool fixed = (flags & SAF3R_ATTN_FIXED_ORDER) != 0;
@@ -1749,8 +1739,7 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   }
   p.item_start[p.n_order] = (int)total;
   if (total == 0) return SAF3R_OK;
-  auto kernel = p.split ? sparse_attn_kernel<true> : sparse_attn_kernel<false>;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(256), 0, (hipStream_t)stream, p);
+  hipLaunchKernelGGL(sparse_attn_kernel, dim3((unsigned)total), dim3(256), 0, (hipStream_t)stream, p);
   if (int e = check_launch("saf3r_sparse_attn_fwd")) return e;
   // the exact walk of the items that left the FAST range: the same items of the prescaled heads,
   // in the fixed order; every other item returns after reading its marker
@@ -1771,8 +1760,7 @@ extern "C" int saf3r_sparse_attn_fwd(const void* q_packed, const void* k_packed,
   if (ftotal == 0) return SAF3R_OK;
   f.n_items = (int)ftotal;
   f.fix_groups = (int)std::min<int64_t>(ftotal, 2 * (int64_t)cus);  // one resident round
-  auto fixup = p.split ? sparse_attn_fixup_kernel<true> : sparse_attn_fixup_kernel<false>;
-  hipLaunchKernelGGL(fixup, dim3((unsigned)f.fix_groups), dim3(256), 0, (hipStream_t)stream, f);
+  hipLaunchKernelGGL(sparse_attn_fixup_kernel, dim3((unsigned)f.fix_groups), dim3(256), 0, (hipStream_t)stream, f);
   return check_launch("saf3r_sparse_attn_fwd");
 }
 
