@@ -783,7 +783,8 @@ def keyset_gather(kp: torch.Tensor, geom: Geometry, specs: Sequence[KeySetSpec],
     _need_cuda(kp, v, idx, count)
     lib = _lib.load()
     n = len(specs)
-    cap = max(64, -(-max(s.bound(geom) for s in specs) // 64) * 64)
+    sizes = {(s.mode, s.param, s.start, s.include): s for s in specs}  # a layer's heads share a few
+    cap = max(64, -(-max(s.bound(geom) for s in sizes.values()) // 64) * 64)
     dev = kp.device
     kc = torch.empty(n, cap, HEAD_DIM, dtype=torch.bfloat16, device=dev)
     vc = torch.empty(n, cap // 64, 64, 64, dtype=torch.bfloat16, device=dev)
