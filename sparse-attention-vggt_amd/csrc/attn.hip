@@ -1484,6 +1484,10 @@ static int head_segments(int h, int pat, bool tokord, bool framed, bool split, i
       add(ns4, g.F * g.NBf, max(1, sel_width / 2), split_steps(sel_width));
       break;
     default: {  // frame-relative patterns: one special tile per item, four patch tiles per item
+      // (a special tile's estimate is not what it walks, which is at most F frames and frame 0 once: about half for
+      // 20 frames of 24 x 32 patches. With the tiles it walks, at the masked walk's 2.4 us, choose_split split the
+      // dense heads of more launches and won nothing: 30 frames of 16 x 16 patches, block mix 208 -> 220 us,
+      // 8 dense heads of 16 170 -> 199; 2 to 24 frames of either grid the same heads.)
       const int64_t mult = pat == SAF3R_ANCHOR_LOCAL ? 2 : 1;
       const int64_t span = pat == SAF3R_ANCHOR ? 1 : (g.ns > 0 ? (64 + g.ns - 1) / g.ns + 1 : 1);
       add(0, g.nst, span * (g.NBf + 1) * mult);
