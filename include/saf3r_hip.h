@@ -173,15 +173,16 @@ int saf3r_pack_qkv(const void* q, const void* k, const void* v, int64_t tok_stri
  * 16-byte aligned; fp32 otherwise), SAF3R_PACK_POS_INT64 (int64 positions, of which the low 32 bits
  * are read; int32 otherwise). */
 enum saf3r_pack_param_flags { SAF3R_PACK_LN_BF16 = 1, SAF3R_PACK_POS_INT64 = 2 };
-int saf3r_pack_qkv_typed(const void* q, const void* k, const void* v, int64_t tok_stride, int64_t head_stride,
-                   int frames, int tokens_per_frame, int num_special, int num_heads,
-                   const void* q_ln_weight, const void* q_ln_bias, const void* k_ln_weight,
-                   const void* k_ln_bias, float ln_eps, int apply_ln,
-                   const void* pos, const float* rope_cos, const float* rope_sin, int rope_positions,
-                   void* q_packed, void* k_packed, void* v_packed, const uint8_t* token_order,
-                   const uint8_t* fp32_heads, float* qk32, const uint8_t* q_scaled, float q_scale,
-                   const uint8_t* pool_heads, float* pool_mean, uint16_t* pool_split, float* pool_meta,
-                   int param_flags, void* stream);
+int saf3r_pack_qkv_typed(const void* q, const void* k, const void* v, int64_t tok_stride,
+                         int64_t head_stride, int frames, int tokens_per_frame, int num_special,
+                         int num_heads, const void* q_ln_weight, const void* q_ln_bias,
+                         const void* k_ln_weight, const void* k_ln_bias, float ln_eps, int apply_ln,
+                         const void* pos, const float* rope_cos, const float* rope_sin,
+                         int rope_positions, void* q_packed, void* k_packed, void* v_packed,
+                         const uint8_t* token_order, const uint8_t* fp32_heads, float* qk32,
+                         const uint8_t* q_scaled, float q_scale, const uint8_t* pool_heads,
+                         float* pool_mean, uint16_t* pool_split, float* pool_meta, int param_flags,
+                         void* stream);
 
 /*
  * Pooled patch-block means (fp32) of the packed Q and K of the listed heads.
@@ -281,9 +282,10 @@ int saf3r_probe_scores(const float* q32, const float* k32, int64_t slot_stride, 
 /* saf3r_probe_scores with `slots` in host memory (at most 64, passed in the kernels' arguments: no copy
  * to the device, which would wait for the stream) and the score rows they are written to: selected
  * head i goes to scores + rows[i] * scores_stride (host int32 [n_sel]). */
-int saf3r_probe_scores_host(const float* q32, const float* k32, int64_t slot_stride, int n_tokens, const int32_t* slots, const int32_t* rows,
-                       int n_sel, const int32_t* sample_idx, int n_samples, float scale, float* partial,
-                       float* qbar, float* scores, int64_t scores_stride, void* stream);
+int saf3r_probe_scores_host(const float* q32, const float* k32, int64_t slot_stride, int n_tokens,
+                            const int32_t* slots, const int32_t* rows, int n_sel,
+                            const int32_t* sample_idx, int n_samples, float scale, float* partial,
+                            float* qbar, float* scores, int64_t scores_stride, void* stream);
 
 /*
  * saf3r_probe_scores without the workspace argument: it allocates nothing (no hipMalloc / hipFree,
@@ -315,9 +317,9 @@ int saf3r_keyset_build(const float* scores, int64_t scores_stride, int n_heads, 
 
 /* saf3r_keyset_build with mode, param, start and include in host memory (at most 64 heads). */
 int saf3r_keyset_build_host(const float* scores, int64_t scores_stride, int n_heads, const int32_t* mode,
-                       const int32_t* param, const int32_t* start, const int32_t* include, int frames,
-                       int tokens_per_frame, int num_special, int32_t* idx, int64_t idx_stride, int32_t* count,
-                       void* stream);
+                            const int32_t* param, const int32_t* start, const int32_t* include,
+                            int frames, int tokens_per_frame, int num_special, int32_t* idx,
+                            int64_t idx_stride, int32_t* count, void* stream);
 
 /*
  * Compact K/V of the key sets, in the layout SAF3R_KEYSET heads read: for set s (head head_ids[s]),
@@ -335,9 +337,10 @@ int saf3r_keyset_gather(const void* k_packed, int frames, int tokens_per_frame, 
 
 /* saf3r_keyset_gather with head_ids in host memory (at most 64). */
 int saf3r_keyset_gather_host(const void* k_packed, int frames, int tokens_per_frame, int num_special,
-                        const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
-                        int64_t v_head_stride, const int32_t* idx, int64_t idx_stride, const int32_t* count,
-                        int max_tiles, void* keyset_k, void* keyset_v, int64_t capacity, void* stream);
+                             const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
+                             int64_t v_head_stride, const int32_t* idx, int64_t idx_stride,
+                             const int32_t* count, int max_tiles, void* keyset_k, void* keyset_v,
+                             int64_t capacity, void* stream);
 
 /*
  * Block-sparse attention forward over the packed layout, every head in one launch.
@@ -401,7 +404,6 @@ int saf3r_sparse_attn_split_heads(int frames, int tokens_per_frame, int num_spec
                                   const int32_t* head_pattern, int sel_width, int64_t keyset_capacity,
                                   const uint8_t* token_order, int compute_units, uint64_t* split_heads);
 
-
 /*
  * Gather attention: out[r] = sum_j softmax_j(q[r] . k[idx[r][j]] * scale) v[idx[r][j]], fp32
  * scores and accumulation, head_dim 64 (q, k, v and out rows of 64 elements); idx entries < 0 or
@@ -446,7 +448,9 @@ int64_t saf3r_gather_attn_workspace_bytes(int n, int topk);
  * (the reference's batch dimension B is a loop of calls over q[b], k[b], idx[b]).
  *   q: n_q rows; k: frames*per_frame rows (frame f = rows [f*per_frame, (f+1)*per_frame));
  *   idx: int32 [n_q][frames*min(topk, per_frame)] global key rows, frame-major, score descending,
- *   ties to the lower index. topk >= 1 and min(topk, per_frame) <= 128 (the reference's limit);
+ *   ties to the lower index (the order in which a score's 64 products are summed depends on the sizes of
+ *   the call, and with it which of two keys is first whose scores differ by no more than that
+ *   rounding). topk >= 1 and min(topk, per_frame) <= 128 (the reference's limit);
  *   above 16 per_frame <= 4096.
  *   workspace / workspace_bytes: caller-owned device memory, required when
  *   min(topk, per_frame) > 16 (NULL / 0 otherwise): at least a share for 128 queries
@@ -458,8 +462,8 @@ int saf3r_token_topk(const saf3r_rows* q, const saf3r_rows* k, int n_q, int fram
                      int32_t* idx, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Workspace bytes for every query of a call (at most about 1 GiB; see above for the least that
- * saf3r_token_topk accepts): 0 when min(topk, per_frame) <= 16, -1 for sizes saf3r_token_topk rejects. No counterpart in the
- * reference (its Triton kernel keeps each query's list in registers). */
+ * saf3r_token_topk accepts): 0 when min(topk, per_frame) <= 16, -1 for sizes saf3r_token_topk rejects.
+ * No counterpart in the reference (its Triton kernel keeps each query's list in registers). */
 int64_t saf3r_token_topk_workspace_bytes(int n_q, int frames, int per_frame, int topk);
 
 /*

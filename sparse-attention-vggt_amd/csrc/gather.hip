@@ -4,16 +4,19 @@
 //      fp32 scores, exact max-subtracted softmax, fp32 P.V, output in v.dtype), :115-166 (API:
 //      q [N, D], k/v [Nk, D], kv_indices [N, TopK], scale default 1/sqrt(D); a stride-0 index view
 //      shares one list across rows), :173-258 (online-softmax variant for TopK > 2048).
-// The work is one gathered K row and one V row per (query, listed key): bound by the cache
-// bandwidth of those row reads, not by arithmetic (a list is one query's own, so there is no
-// matrix product to share between queries). A wave owns two query rows (32 lanes each) and walks
+// The work is one gathered K row and one V row per (query, listed key), without a matrix product to share
+// between queries (a list is one query's own). Bound by the issue of the row loads and of the per-key
+// arithmetic more than by the caches: 64 x 1036 fp32 rows, lists of 256, take 396 us (22 TB/s of rows) on lists of
+// near matches, 321 us (27 TB/s; the L1s deliver 39) when every list names the same 32 rows, and 1094 us on random
+// lists, whose 33 MB of rows no L2 holds; 4 x 1036 bf16 rows take 24 us with either, as 2072 waves of 16
+// dependent steps do not fill the chip (16 times the rows 282 us). A wave owns two query rows (32 lanes each) and walks
 // their lists in steps of ENT entries with an fp32 online softmax, so any list length is handled by
 // the same kernel. Lane l of a row's 32 serves key slot ks = l / 8 of every group of 4 keys and 8 dims
 // (dg = l % 8: dims 8 dg .. of a bf16 row; 4 dg .. 4 dg + 3 and 32 + 4 dg .. of an fp32 row): 8 lanes
 // read a K or V row together, 16 bytes each per load, so that one load instruction covers 8 whole
 // 128-byte lines, one per row (32 adjacent bytes of an fp32 row per lane, as two loads, touched 16
-// lines in each: 404 against 398 us at 64 x 1036 fp32 rows, lists of 256), and the 8 partial dot products of a row are summed by three DPP steps inside
-// the 8 lanes. Entries < 0 or >= num_keys are skipped. q and k
+// lines in each: 404 against 398 us at 64 x 1036 fp32 rows, lists of 256), and the 8 partial dot
+// products of a row are summed by three DPP steps inside the 8 lanes. Entries < 0 or >= num_keys are skipped. q and k
 // are bf16 or fp32 rows (the reference's kernel upcasts either); v and out are bf16 or fp32 rows
 // (the reference writes out in v.dtype from its fp32 accumulator).
 //
@@ -423,7 +426,7 @@ static void launch_gather(const GatherParams& p, bool o32, bool narrow, bool sli
 // 24 bits and every byte offset 32, so a lane forms both addresses with a few 24- and 32-bit
 // instructions on uniform bases. The general form's 64-bit multiplies were about 20 of 55 VALU
 // instructions per gathered key (sliced, 64 x 1036 rows, lists of 256: bf16 313 -> 278 us, fp32
-// 422 -> 404; the rest is the rate at which the L1 delivers the rows, 64 bytes a clock and CU).
+// 422 -> 404).
 static bool narrow_rows(GatherParams* p, bool qk32, bool v32) {
   const RowsDev &k = p->k, &v = p->v;
   const bool mapped = k.shift >= 0;

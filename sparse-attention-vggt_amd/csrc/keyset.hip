@@ -578,11 +578,10 @@ extern "C" int saf3r_keyset_build_host(const float* scores, int64_t scores_strid
                       frames, tokens_per_frame, num_special, idx, idx_stride, count, stream);
 }
 
-static int gather_launch(const char* who, bool host, const void* k_packed, int frames, int tokens_per_frame, int num_special,
-                                   const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
-                                   int64_t v_head_stride, const int32_t* idx, int64_t idx_stride,
-                                   const int32_t* count, int max_tiles, void* keyset_k, void* keyset_v,
-                                   int64_t capacity, void* stream) {
+static int gather_launch(const char* who, bool host, const void* k_packed, int frames, int tokens_per_frame,
+                         int num_special, const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
+                         int64_t v_head_stride, const int32_t* idx, int64_t idx_stride, const int32_t* count,
+                         int max_tiles, void* keyset_k, void* keyset_v, int64_t capacity, void* stream) {
   if (int e = injected(who)) return e;
   GatherKParams p;
   if (!make_geom(frames, tokens_per_frame, num_special, &p.g))
@@ -623,13 +622,17 @@ extern "C" int saf3r_keyset_gather(const void* k_packed, int frames, int tokens_
                                    int64_t v_head_stride, const int32_t* idx, int64_t idx_stride,
                                    const int32_t* count, int max_tiles, void* keyset_k, void* keyset_v,
                                    int64_t capacity, void* stream) {
-  return gather_launch("saf3r_keyset_gather", false, k_packed, frames, tokens_per_frame, num_special, head_ids, n_sel, v, v_tok_stride, v_head_stride, idx, idx_stride, count, max_tiles, keyset_k, keyset_v, capacity, stream);
+  return gather_launch("saf3r_keyset_gather", false, k_packed, frames, tokens_per_frame, num_special, head_ids, n_sel,
+                       v, v_tok_stride, v_head_stride, idx, idx_stride, count, max_tiles, keyset_k, keyset_v,
+                       capacity, stream);
 }
 
 extern "C" int saf3r_keyset_gather_host(const void* k_packed, int frames, int tokens_per_frame, int num_special,
-                                   const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
-                                   int64_t v_head_stride, const int32_t* idx, int64_t idx_stride,
-                                   const int32_t* count, int max_tiles, void* keyset_k, void* keyset_v,
-                                   int64_t capacity, void* stream) {
-  return gather_launch("saf3r_keyset_gather_host", true, k_packed, frames, tokens_per_frame, num_special, head_ids, n_sel, v, v_tok_stride, v_head_stride, idx, idx_stride, count, max_tiles, keyset_k, keyset_v, capacity, stream);
+                                        const int32_t* head_ids, int n_sel, const void* v, int64_t v_tok_stride,
+                                        int64_t v_head_stride, const int32_t* idx, int64_t idx_stride,
+                                        const int32_t* count, int max_tiles, void* keyset_k, void* keyset_v,
+                                        int64_t capacity, void* stream) {
+  return gather_launch("saf3r_keyset_gather_host", true, k_packed, frames, tokens_per_frame, num_special, head_ids,
+                       n_sel, v, v_tok_stride, v_head_stride, idx, idx_stride, count, max_tiles, keyset_k, keyset_v,
+                       capacity, stream);
 }

@@ -244,15 +244,14 @@ __global__ __launch_bounds__(512) void pack_qkv_kernel(PackParams p) {
 
 using namespace saf3r;
 
-static int pack_launch(const char* who, const void* q, const void* k, const void* v, int64_t tok_stride, int64_t head_stride,
-                              int frames, int tokens_per_frame, int num_special, int num_heads,
-                              const void* q_ln_weight, const void* q_ln_bias, const void* k_ln_weight,
-                              const void* k_ln_bias, float ln_eps, int apply_ln, const void* pos,
-                              const float* rope_cos, const float* rope_sin, int rope_positions, void* q_packed,
-                              void* k_packed, void* v_packed, const uint8_t* token_order, const uint8_t* fp32_heads,
-                              float* qk32, const uint8_t* q_scaled, float q_scale, const uint8_t* pool_heads,
-                              float* pool_mean, uint16_t* pool_split, float* pool_meta, int param_flags,
-                       void* stream) {
+static int pack_launch(const char* who, const void* q, const void* k, const void* v, int64_t tok_stride,
+                       int64_t head_stride, int frames, int tokens_per_frame, int num_special, int num_heads,
+                       const void* q_ln_weight, const void* q_ln_bias, const void* k_ln_weight, const void* k_ln_bias,
+                       float ln_eps, int apply_ln, const void* pos, const float* rope_cos, const float* rope_sin,
+                       int rope_positions, void* q_packed, void* k_packed, void* v_packed, const uint8_t* token_order,
+                       const uint8_t* fp32_heads, float* qk32, const uint8_t* q_scaled, float q_scale,
+                       const uint8_t* pool_heads, float* pool_mean, uint16_t* pool_split, float* pool_meta,
+                       int param_flags, void* stream) {
   if (int e = injected(who)) return e;
   PackParams p;
   if (param_flags & ~(SAF3R_PACK_LN_BF16 | SAF3R_PACK_POS_INT64))
@@ -367,16 +366,23 @@ extern "C" int saf3r_pack_qkv(const void* q, const void* k, const void* v, int64
                               void* k_packed, void* v_packed, const uint8_t* token_order, const uint8_t* fp32_heads,
                               float* qk32, const uint8_t* q_scaled, float q_scale, const uint8_t* pool_heads,
                               float* pool_mean, uint16_t* pool_split, float* pool_meta, void* stream) {
-  return pack_launch("saf3r_pack_qkv", q, k, v, tok_stride, head_stride, frames, tokens_per_frame, num_special, num_heads, q_ln_weight, q_ln_bias, k_ln_weight, k_ln_bias, ln_eps, apply_ln, pos, rope_cos, rope_sin, rope_positions, q_packed, k_packed, v_packed, token_order, fp32_heads, qk32, q_scaled, q_scale, pool_heads, pool_mean, pool_split, pool_meta, 0, stream);
+  return pack_launch("saf3r_pack_qkv", q, k, v, tok_stride, head_stride, frames, tokens_per_frame, num_special,
+                     num_heads, q_ln_weight, q_ln_bias, k_ln_weight, k_ln_bias, ln_eps, apply_ln, pos, rope_cos,
+                     rope_sin, rope_positions, q_packed, k_packed, v_packed, token_order, fp32_heads, qk32, q_scaled,
+                     q_scale, pool_heads, pool_mean, pool_split, pool_meta, 0, stream);
 }
 
-extern "C" int saf3r_pack_qkv_typed(const void* q, const void* k, const void* v, int64_t tok_stride, int64_t head_stride,
-                              int frames, int tokens_per_frame, int num_special, int num_heads,
-                              const void* q_ln_weight, const void* q_ln_bias, const void* k_ln_weight,
-                              const void* k_ln_bias, float ln_eps, int apply_ln, const void* pos,
-                              const float* rope_cos, const float* rope_sin, int rope_positions, void* q_packed,
-                              void* k_packed, void* v_packed, const uint8_t* token_order, const uint8_t* fp32_heads,
-                              float* qk32, const uint8_t* q_scaled, float q_scale, const uint8_t* pool_heads,
-                              float* pool_mean, uint16_t* pool_split, float* pool_meta, int param_flags, void* stream) {
-  return pack_launch("saf3r_pack_qkv_typed", q, k, v, tok_stride, head_stride, frames, tokens_per_frame, num_special, num_heads, q_ln_weight, q_ln_bias, k_ln_weight, k_ln_bias, ln_eps, apply_ln, pos, rope_cos, rope_sin, rope_positions, q_packed, k_packed, v_packed, token_order, fp32_heads, qk32, q_scaled, q_scale, pool_heads, pool_mean, pool_split, pool_meta, param_flags, stream);
+extern "C" int saf3r_pack_qkv_typed(const void* q, const void* k, const void* v, int64_t tok_stride,
+                                    int64_t head_stride, int frames, int tokens_per_frame, int num_special,
+                                    int num_heads, const void* q_ln_weight, const void* q_ln_bias,
+                                    const void* k_ln_weight, const void* k_ln_bias, float ln_eps, int apply_ln,
+                                    const void* pos, const float* rope_cos, const float* rope_sin, int rope_positions,
+                                    void* q_packed, void* k_packed, void* v_packed, const uint8_t* token_order,
+                                    const uint8_t* fp32_heads, float* qk32, const uint8_t* q_scaled, float q_scale,
+                                    const uint8_t* pool_heads, float* pool_mean, uint16_t* pool_split,
+                                    float* pool_meta, int param_flags, void* stream) {
+  return pack_launch("saf3r_pack_qkv_typed", q, k, v, tok_stride, head_stride, frames, tokens_per_frame, num_special,
+                     num_heads, q_ln_weight, q_ln_bias, k_ln_weight, k_ln_bias, ln_eps, apply_ln, pos, rope_cos,
+                     rope_sin, rope_positions, q_packed, k_packed, v_packed, token_order, fp32_heads, qk32, q_scaled,
+                     q_scale, pool_heads, pool_mean, pool_split, pool_meta, param_flags, stream);
 }

@@ -523,10 +523,11 @@ __device__ __forceinline__ int lanes_before(uint64_t m, int base) {
 // The next frame's fragments load while the rows of this one are selected (NV <= 24; longer frames
 // have no registers for it).
 // Bound by the VALU of the selection and the loads' latency: a work-group of 16 waves fills a CU
-// (its LDS rows take 74 KB at 1036 keys and 90 KB at 1369), scoring takes 220 us of 497 at
-// 16 x 1036 tokens, top-64, and the 128-entry sort 80 us. It replaced a dump of every score to a
-// workspace in HBM and a radix select of eight digit passes over LDS bins per row: 1630 -> 497 us
-// there, 21.9 -> 6.8 ms at 48 x 1369 tokens. A 64-bit sort of (score, index)
+// (its LDS rows take 74 KB at 1036 keys and 90 KB at 1369), scoring takes 220 us of 500 at
+// 16 x 1036 tokens, top-64, and the 128-entry sort 80 us. The prefetch takes the registers to their limit of 128:
+// none spilled at 1036 keys, 42 at 1369, 157 at 4096 (most of them of the exact path). It replaced a
+// dump of every score to a workspace in HBM and a radix select of eight digit passes over LDS bins per row:
+// 1630 -> 500 us there, 21.9 -> 6.2 ms at 48 x 1369 tokens. A 64-bit sort of (score, index)
 // took 220 VALU instructions against 82, fragments loaded without the LDS stage 50 us more.
 template <int NV, bool FLAT>
 __global__ __launch_bounds__(64 * kRowWaves) void topk_rows_kernel(TopkParams p) {
@@ -820,6 +821,8 @@ static int launch_topk_rows(TopkParams p, hipStream_t st) {
 // 40 / 29, 3 x 1369 (3) 47 / 36; top-8 3 x 1036 21 / 35, 4 x 1036 41 / 35; top-16 5 x 1036 (6.3)
 // 54 / 57, 5 x 1369 (8.4) 81 / 73, 16 x 1036 418 / 274. Short frames leave the two-pass bound of a
 // top-16 weak (64 groups of P / 64 keys): 16 x 256 42 / 79, 64 x 256 553 / 1050.
+// The two sum a score's products in different orders (16x16x32 and 32x32x16 MFMAs), so keys whose scores are
+// within that rounding can change places between a small call and a large one.
 static bool topk_takes_rows(const TopkParams& p) {
   if (p.kmode == 2 || p.P > 1536) return false;
   if (p.ke > 8 && p.P <= 512) return true;

@@ -568,7 +568,8 @@ def gather_attn_rows(qr, kr, vr, idx, idx_row_stride, n, topk, num_keys, scale, 
 
 
 def token_topk_workspace_bytes(n_q: int, frames: int, per_frame: int, topk: int) -> int:
-    """Bytes of the score workspace ``saf3r_token_topk`` takes for these sizes (0 for top-k <= 16)."""
+    """Workspace bytes ``saf3r_token_topk`` states for these sizes (0 for top-k <= 16; it accepts a share for 128
+    queries and does not use it)."""
     nbytes = _lib.load().saf3r_token_topk_workspace_bytes(n_q, frames, per_frame, topk)
     if nbytes < 0:
         _lib.check(_lib.SAF3R_ERR_INVALID)  # raises with the library's message
