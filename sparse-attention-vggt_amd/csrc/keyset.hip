@@ -77,6 +77,7 @@ __device__ __forceinline__ float ordered_sum(int n, At&& at) {
 // grid (nchunks, n_sel), 64 threads: feature d of chunk c, summed over the chunk's rows in order
 __global__ __launch_bounds__(64) void probe_partial_kernel(ProbeParams p) {
   const int c = bid_x(), hs = bid_y(), d = tid_x();
+  if (probe_slot(p, hs) < 0) return;  // a row of zeros (probe_scores_kernel)
   const float* base = p.q + (int64_t)probe_slot(p, hs) * p.slot_stride + d;
   const int i0 = c * p.chunk, i1 = min(p.n_samp, i0 + p.chunk);
   const float acc = ordered_sum(i1 - i0, [&](int i) {
@@ -89,6 +90,7 @@ __global__ __launch_bounds__(64) void probe_partial_kernel(ProbeParams p) {
 // grid (n_sel), 64 threads: chunk sums in chunk order, then one correctly rounded division
 __global__ __launch_bounds__(64) void probe_finish_kernel(ProbeParams p) {
   const int hs = bid_x(), d = tid_x();
+  if (probe_slot(p, hs) < 0) return;
   const float* part = p.partial + (int64_t)hs * kProbeChunks * 64 + d;
   const float total = ordered_sum(p.nchunks, [&](int c) { return part[(int64_t)c * 64]; });
   p.qbar[hs * 64 + d] = __fdiv_rn(total, (float)p.n_samp);
@@ -98,6 +100,11 @@ __global__ __launch_bounds__(64) void probe_finish_kernel(ProbeParams p) {
 __global__ __launch_bounds__(256) void probe_scores_kernel(ProbeParams p) {
   __shared__ float qb[64];
   const int hs = bid_y();
+  if (probe_slot(p, hs) < 0) {  // (uniform; a fill of its own for such rows is a launch more, 5 us of host time)
+    const int z = bid_x() * 256 + tid_x();
+    if (z < p.n) p.scores[(p.slots ? hs : p.row_val[hs]) * p.scores_stride + z] = 0.f;
+    return;
+  }
   if (tid_x() < 64) qb[tid_x()] = p.qbar[hs * 64 + tid_x()];
   __syncthreads();
   const int t = bid_x() * 256 + tid_x();
@@ -514,7 +521,7 @@ extern "C" int saf3r_probe_scores_host(const float* q32, const float* k32, int64
   if (int e = host_lists(who, n_sel)) return e;
   p.slots = nullptr;
   for (int i = 0; i < n_sel; ++i) {
-    if (slots[i] < 0 || rows[i] < 0) return fail(SAF3R_ERR_INVALID, "%s: negative slot or row", who);
+    if (slots[i] < -1 || rows[i] < 0) return fail(SAF3R_ERR_INVALID, "%s: negative slot or row", who);
     p.slot_val[i] = slots[i];
     p.row_val[i] = rows[i];
   }

@@ -129,6 +129,13 @@ def _i32_values(key: bytes):
 
 
 @lru_cache(maxsize=1024)
+def _i32_quarters(key: bytes) -> tuple:
+    """Four arrays of the same length from their values in a row."""
+    n = len(key) // 4
+    return tuple(_i32_values(key[i * n:(i + 1) * n]) for i in range(4))
+
+
+@lru_cache(maxsize=1024)
 def _flag_values(key: bytes, n: int):
     if len(key) != n:
         raise ValueError(f"one flag per head: got {len(key)} for {n} heads")
@@ -676,13 +683,14 @@ class KeySets:
 
 def probe_scores(qk32: torch.Tensor, slots: Sequence[int], scale: float | None = None,
                  sample: torch.Tensor | None = None, noalloc: bool = False, out: torch.Tensor | None = None,
-                 rows: Sequence[int] | None = None):
+                 rows: Sequence[int] | None = None, zero_rows: Sequence[int] = ()):
     """Mean query and probe scores (``saf3r/patch/sparse_attention.py:150-168``) of the heads stored at
     ``slots`` of ``qk32`` (fp32 [n, 2, N, 64], q and k rows in token order, as ``pack_qkv`` writes them
     for ``fp32_heads``): returns (qbar fp32 [n_sel][64], scores fp32 [n_sel][N]). ``sample`` (int tokens)
     restricts the mean to those query rows, in list order (the reference's ``q_sample_ratio < 1``).
     ``noalloc`` uses the allocation-free entry (its partial sums in the library's static workspace).
-    ``out`` (fp32 [.., >= N], contiguous) with ``rows`` receives head i's scores in row ``rows[i]``."""
+    ``out`` (fp32 [.., >= N], contiguous) with ``rows`` receives head i's scores in row ``rows[i]``, and zeros in
+    ``zero_rows``."""
     _need_cuda(qk32)
     lib = _lib.load()
     if qk32.dtype != torch.float32 or qk32.dim() != 4 or qk32.shape[1] != 2 or qk32.shape[3] != HEAD_DIM \
@@ -693,10 +701,13 @@ def probe_scores(qk32: torch.Tensor, slots: Sequence[int], scale: float | None =
     dev = qk32.device
     slots = [int(s) for s in slots]
     rows = list(range(n)) if rows is None else [int(r) for r in rows]
+    zeros = [int(r) for r in zero_rows]
     if slots and not 0 <= min(slots) <= max(slots) < qk32.shape[0]:
         raise ValueError(f"slots {slots} of {qk32.shape[0]}")
     if len(rows) != n or (rows and (min(rows) < 0 or (out is not None and max(rows) >= out.shape[0]))):
         raise ValueError(f"rows {rows}: one per slot, inside out")
+    if zeros and (out is None or min(zeros) < 0 or max(zeros) >= out.shape[0]):
+        raise ValueError(f"zero rows {zeros}: inside out")
     qbar = torch.empty(n, HEAD_DIM, dtype=torch.float32, device=dev)
     if out is None:
         scores = torch.empty(max(rows) + 1 if rows else 0, N, dtype=torch.float32, device=dev)
@@ -713,9 +724,9 @@ def probe_scores(qk32: torch.Tensor, slots: Sequence[int], scale: float | None =
     stride = qk32.stride(0)
     kptr = qk32.data_ptr() + 4 * qk32.stride(1)
     n_samp = 0 if sample is None else sample.numel()
-    by_value = n <= MAX_HEADS and not noalloc  # the lists go with the launch
+    by_value = n + len(zeros) <= MAX_HEADS and not noalloc  # the lists go with the launch
     hs = None if by_value else torch.tensor(slots, dtype=torch.int32, device=dev)
-    if not by_value and rows != list(range(n)):
+    if not by_value and (zeros or rows != list(range(n))):
         raise ValueError("rows need at most 64 heads and the allocating entry")
     _mark("probe", "start")
     if noalloc:
@@ -725,9 +736,10 @@ def probe_scores(qk32: torch.Tensor, slots: Sequence[int], scale: float | None =
     else:
         partial = torch.empty(n, 256, HEAD_DIM, dtype=torch.float32, device=dev)
         if by_value:
-            _lib.check(lib.saf3r_probe_scores_host(_ptr(qk32), kptr, stride, N, _i32_array(slots), _i32_array(rows), n,
-                                                   _ptr(sample), n_samp, float(scale), _ptr(partial), _ptr(qbar),
-                                                   _ptr(scores), scores.stride(0), _lib.stream_ptr()))
+            _lib.check(lib.saf3r_probe_scores_host(_ptr(qk32), kptr, stride, N, _i32_array(slots + [-1] * len(zeros)),
+                                                   _i32_array(rows + zeros), n + len(zeros), _ptr(sample), n_samp,
+                                                   float(scale), _ptr(partial), _ptr(qbar), _ptr(scores),
+                                                   scores.stride(0), _lib.stream_ptr()))
         else:
             _lib.check(lib.saf3r_probe_scores(_ptr(qk32), kptr, stride, N, _ptr(hs), n, _ptr(sample), n_samp,
                                               float(scale), _ptr(partial), _ptr(qbar), _ptr(scores), scores.stride(0),
@@ -755,8 +767,8 @@ def keyset_build(specs: Sequence[KeySetSpec], geom: Geometry, scores: torch.Tens
         raise ValueError("key-set stride / k must be positive")
     if scores is None and any(s.mode == KEYSET_TOPK for s in specs):
         raise ValueError("top-k key sets need scores")
-    lists = [[s.mode for s in specs], [s.param for s in specs], [s.start for s in specs],
-             [int(bool(s.include)) for s in specs]]
+    lists = [s.mode for s in specs] + [s.param for s in specs] + [s.start for s in specs]
+    lists += [bool(s.include) for s in specs]
     idx = torch.empty(n, geom.tokens, dtype=torch.int32, device=device)
     count = torch.empty(n, dtype=torch.int32, device=device)
     if scores is not None:
@@ -766,9 +778,9 @@ def keyset_build(specs: Sequence[KeySetSpec], geom: Geometry, scores: torch.Tens
         scores = scores.contiguous()
     _mark("keyset_build", "start")
     if n <= MAX_HEADS:
-        entry, args = lib.saf3r_keyset_build_host, [_i32_array(x) for x in lists]
+        entry, args = lib.saf3r_keyset_build_host, _i32_quarters(_i32_key(lists))
     else:
-        arr = torch.tensor(lists, dtype=torch.int32, device=device)
+        arr = torch.tensor(lists, dtype=torch.int32, device=device).view(4, n)
         entry, args = lib.saf3r_keyset_build, [_ptr(arr[i]) for i in range(4)]
     _lib.check(entry(_ptr(scores), 0 if scores is None else scores.stride(0), n, *args, geom.frames,
                      geom.tokens_per_frame, geom.num_special, _ptr(idx), idx.stride(0), _ptr(count),

@@ -51,6 +51,12 @@ def _head_layouts(patterns: tuple, geom: Geometry) -> tuple:
     return tuple(ops.token_order_heads(patterns, geom))
 
 
+@lru_cache(maxsize=1024)
+def _flags_but(n: int, on, skip) -> tuple:
+    """``on`` for every head but ``skip``."""
+    return tuple(on and h != skip for h in range(n))
+
+
 class BaseHeadwiseSparseAttentionWrapper(nn.Module):
     def __init__(self, orig_module, num_special_tokens, num_heads, **kwargs):
         super().__init__()
@@ -111,7 +117,7 @@ class BaseHeadwiseSparseAttentionWrapper(nn.Module):
         correspondence head of a lazy dino_topk layer, whose packed Q the token top-k reads as the
         reference's q (``fused_qk_topk.py:120-217``)."""
         skip = self.first_dino_head if self.lazy_dino_topk else None
-        return [self.prescale_q and h != skip for h in range(self.num_heads)]
+        return list(_flags_but(self.num_heads, self.prescale_q, skip))
 
     # ------------------------------------------------------------------------------------
     def geometry(self, num_tokens: int) -> Geometry:
@@ -209,12 +215,14 @@ class BaseHeadwiseSparseAttentionWrapper(nn.Module):
                 _, scores = ops.probe_scores(qk32, [self.fp32_slot[specs[i].head] for i in probe_rows],
                                              sample=ops.probe_sample(geom.tokens, ratios[0]))
             else:  # one call per sample ratio; rows of stride heads are not read, and stay zeros in ks.scores
-                new = torch.empty if len(probe_rows) == len(specs) else torch.zeros
-                scores = new(len(specs), geom.tokens, dtype=torch.float32, device=kp.device)
+                scores = torch.empty(len(specs), geom.tokens, dtype=torch.float32, device=kp.device)
+                stride_rows = [i for i, s in enumerate(specs) if s.mode != ops.KEYSET_TOPK]
                 for r in ratios:
                     rows_r = [i for i in probe_rows if specs[i].sample_ratio == r]
                     ops.probe_scores(qk32, [self.fp32_slot[specs[i].head] for i in rows_r],
-                                     sample=ops.probe_sample(geom.tokens, r), out=scores, rows=rows_r)
+                                     sample=ops.probe_sample(geom.tokens, r), out=scores, rows=rows_r,
+                                     zero_rows=stride_rows)
+                    stride_rows = []
         idx, count = ops.keyset_build(specs, geom, scores, kp.device)
         ks = ops.keyset_gather(kp, geom, specs, qkv[:, 2 * C:], qkv.stride(0), HEAD_DIM, idx, count)
         ks.scores = scores

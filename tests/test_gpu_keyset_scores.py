@@ -39,3 +39,17 @@ def test_scores_of_stride_heads_are_zero(pkg, ratios, monkeypatch):
     scores = w.last_keysets.scores.cpu()
     print(f"stride rows: max |score| {scores[[0, 3]].abs().max().item()}", flush=True)
     assert (scores[[0, 3]] == 0).all() and (scores[[1, 2]] != 0).any(dim=1).all()
+
+
+def test_cleared_rows_of_a_wider_output(pkg):
+    """``zero_rows`` beside scored rows: each written over its N scores, every other value left alone, the scored rows
+    those of a call without them."""
+    ops = importlib.import_module(pkg.__name__ + ".ops")
+    N = 1300
+    g = torch.Generator().manual_seed(9)
+    qk32 = torch.randn(3, 2, N, 64, generator=g).to(DEV)
+    out = torch.full((7, N + 4), 7.0, device=DEV)
+    qbar, _ = ops.probe_scores(qk32, [2, 0], out=out, rows=[5, 1], zero_rows=[0, 6, 3])
+    ref_bar, ref = ops.probe_scores(qk32, [2, 0])
+    assert torch.equal(qbar, ref_bar) and torch.equal(out[[5, 1], :N], ref)
+    assert (out[[0, 6, 3], :N] == 0).all() and (out[[2, 4]] == 7).all() and (out[:, N:] == 7).all()

@@ -106,6 +106,16 @@ def test_probe_scores_checks_its_rows_and_output(ops, monkeypatch):
             ops.probe_scores(qk32, slots)
 
 
+def test_probe_scores_checks_its_zero_rows(ops, monkeypatch):
+    """Rows to clear are rows of ``out``."""
+    import torch
+    monkeypatch.setattr(ops, "_need_cuda", lambda *a: None)
+    qk32, out = torch.zeros(3, 2, 10, 64), torch.zeros(4, 10)
+    for kw in ({}, {"out": out, "zero_rows": [4]}, {"out": out, "zero_rows": [-1]}):
+        with pytest.raises(ValueError, match="zero rows"):
+            ops.probe_scores(qk32, [2, 0], **{"zero_rows": [1], **kw})
+
+
 def test_topk_key_sets_need_scores(ops, pkg):
     """Refused on the host: the kernel reads a score row for every top-k head."""
     geom = pkg.Geometry(2, 20, 5)
