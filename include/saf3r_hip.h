@@ -281,8 +281,8 @@ int saf3r_probe_scores(const float* q32, const float* k32, int64_t slot_stride, 
 
 /* saf3r_probe_scores with `slots` in host memory (at most 64, passed in the kernels' arguments: no copy
  * to the device, which would wait for the stream) and the score rows they are written to: selected
- * head i goes to scores + rows[i] * scores_stride (host int32 [n_sel]). Slot -1: no head, that row's n_tokens
- * scores are zeros (its partial and qbar rows are not written and need not exist at the arrays' ends). */
+ * head i goes to scores + rows[i] * scores_stride (host int32 [n_sel]). Slot -1, behind all
+ * heads: no head, that row's n_tokens scores are zeros (without a row in partial and qbar). */
 int saf3r_probe_scores_host(const float* q32, const float* k32, int64_t slot_stride, int n_tokens,
                             const int32_t* slots, const int32_t* rows, int n_sel,
                             const int32_t* sample_idx, int n_samples, float scale, float* partial,

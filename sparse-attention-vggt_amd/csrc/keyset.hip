@@ -52,6 +52,7 @@ struct ProbeParams {
   float* scores;         // [n_sel][scores_stride]
   int64_t scores_stride;
   float scale;
+  int n_heads;           // selected heads (by value: rows from there on are zeros)
 };
 
 __device__ inline int probe_slot(const ProbeParams& p, int hs) { return p.slots ? p.slots[hs] : p.slot_val[hs]; }
@@ -77,7 +78,6 @@ __device__ __forceinline__ float ordered_sum(int n, At&& at) {
 // grid (nchunks, n_sel), 64 threads: feature d of chunk c, summed over the chunk's rows in order
 __global__ __launch_bounds__(64) void probe_partial_kernel(ProbeParams p) {
   const int c = bid_x(), hs = bid_y(), d = tid_x();
-  if (probe_slot(p, hs) < 0) return;  // a row of zeros (probe_scores_kernel)
   const float* base = p.q + (int64_t)probe_slot(p, hs) * p.slot_stride + d;
   const int i0 = c * p.chunk, i1 = min(p.n_samp, i0 + p.chunk);
   const float acc = ordered_sum(i1 - i0, [&](int i) {
@@ -90,7 +90,6 @@ __global__ __launch_bounds__(64) void probe_partial_kernel(ProbeParams p) {
 // grid (n_sel), 64 threads: chunk sums in chunk order, then one correctly rounded division
 __global__ __launch_bounds__(64) void probe_finish_kernel(ProbeParams p) {
   const int hs = bid_x(), d = tid_x();
-  if (probe_slot(p, hs) < 0) return;
   const float* part = p.partial + (int64_t)hs * kProbeChunks * 64 + d;
   const float total = ordered_sum(p.nchunks, [&](int c) { return part[(int64_t)c * 64]; });
   p.qbar[hs * 64 + d] = __fdiv_rn(total, (float)p.n_samp);
@@ -100,9 +99,9 @@ __global__ __launch_bounds__(64) void probe_finish_kernel(ProbeParams p) {
 __global__ __launch_bounds__(256) void probe_scores_kernel(ProbeParams p) {
   __shared__ float qb[64];
   const int hs = bid_y();
-  if (probe_slot(p, hs) < 0) {  // (uniform; a fill of its own for such rows is a launch more, 5 us of host time)
+  if (hs >= p.n_heads) {  // a row of zeros (a fill of its own is a launch more, 5 us of host time)
     const int z = bid_x() * 256 + tid_x();
-    if (z < p.n) p.scores[(p.slots ? hs : p.row_val[hs]) * p.scores_stride + z] = 0.f;
+    if (z < p.n) p.scores[p.row_val[hs] * p.scores_stride + z] = 0.f;
     return;
   }
   if (tid_x() < 64) qb[tid_x()] = p.qbar[hs * 64 + tid_x()];
@@ -412,13 +411,16 @@ static int probe_setup(const char* who, const float* q32, const float* k32, int6
   p.scores = scores;
   p.scores_stride = scores_stride;
   p.scale = scale;
+  p.n_heads = n_sel;
   return SAF3R_OK;
 }
 
 static int probe_launch(const ProbeParams& p, int n_sel, void* stream) {
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(probe_partial_kernel, dim3(p.nchunks, n_sel), dim3(64), 0, s, p);
-  hipLaunchKernelGGL(probe_finish_kernel, dim3(n_sel), dim3(64), 0, s, p);
+  if (p.n_heads > 0) {
+    hipLaunchKernelGGL(probe_partial_kernel, dim3(p.nchunks, p.n_heads), dim3(64), 0, s, p);
+    hipLaunchKernelGGL(probe_finish_kernel, dim3(p.n_heads), dim3(64), 0, s, p);
+  }
   hipLaunchKernelGGL(probe_scores_kernel, dim3((unsigned)((p.n + 255) / 256), n_sel), dim3(256), 0, s, p);
   return check_launch("saf3r_probe_scores");
 }
@@ -520,8 +522,11 @@ extern "C" int saf3r_probe_scores_host(const float* q32, const float* k32, int64
   if (!partial || !rows) return fail(SAF3R_ERR_INVALID, "%s: null workspace or rows", who);
   if (int e = host_lists(who, n_sel)) return e;
   p.slots = nullptr;
+  p.n_heads = 0;
   for (int i = 0; i < n_sel; ++i) {
     if (slots[i] < -1 || rows[i] < 0) return fail(SAF3R_ERR_INVALID, "%s: negative slot or row", who);
+    if (slots[i] >= 0 && p.n_heads < i) return fail(SAF3R_ERR_INVALID, "%s: a head behind a row of zeros", who);
+    if (slots[i] >= 0) p.n_heads = i + 1;
     p.slot_val[i] = slots[i];
     p.row_val[i] = rows[i];
   }
