@@ -116,6 +116,17 @@ def test_probe_scores_checks_its_zero_rows(ops, monkeypatch):
             ops.probe_scores(qk32, [2, 0], **{"zero_rows": [1], **kw})
 
 
+def test_probe_entry_takes_zero_rows_behind_the_heads(pkg):
+    """Refused before any launch: negative slots other than -1, and a head behind a row of zeros."""
+    import ctypes
+    lib = import_module(pkg.__name__ + "._lib").load()
+    for slots, message in (([-2], b"negative"), ([0, -1, 1], b"behind"), ([-1, 0], b"behind")):
+        n = len(slots)
+        rc = lib.saf3r_probe_scores_host(16, 16, 640, 10, (ctypes.c_int32 * n)(*slots), (ctypes.c_int32 * n)(), n, None, 0,
+                                         1.0, 16, 16, 16, 10, None)
+        assert rc == 1 and message in lib.saf3r_last_error(), slots
+
+
 def test_topk_key_sets_need_scores(ops, pkg):
     """Refused on the host: the kernel reads a score row for every top-k head."""
     geom = pkg.Geometry(2, 20, 5)
